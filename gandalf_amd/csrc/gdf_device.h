@@ -15,17 +15,19 @@ namespace gdf {
 __device__ __forceinline__ float rcp_f(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float rsq_f(float x) { return __builtin_amdgcn_rsqf(x); }
 __device__ __forceinline__ float sqrt_f(float x) { return __builtin_amdgcn_sqrtf(x); }
-// FP64 1/sqrt(x) for x > 0: hardware estimate (about 2^-23 relative) refined by two Newton
-// steps y <- y + y (1 - x y^2)/2, which leaves about an ulp
+// FP64 1/sqrt(x) for x > 0: hardware estimate (about 2^-23 relative) refined by one third-order
+// step y <- y (1 + e/2 + 3 e^2/8), e = 1 - x y^2, whose error is 5 e^3/16: rounding only
 __device__ __forceinline__ double rsq_d(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  #pragma unroll
-  for (int it = 0; it < 2; it++) {
-    const double e = fma(-(x*y), y, 1.0);
-    y = fma(0.5*y, e, y);
-  }
-  return y;
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x*y), y, 1.0);
+  return fma(y*e, fma(0.375, e, 0.5), y);
 }
+// sqrt(x) for x >= 0 from it
+__device__ __forceinline__ double sqrt_d(double x) { return x*rsq_d(fmax(x, 1.0e-280)); }
+__device__ __forceinline__ float rsq_t(float x) { return rsq_f(x); }
+__device__ __forceinline__ double rsq_t(double x) { return rsq_d(x); }
+__device__ __forceinline__ float sqrt_t(float x) { return sqrt_f(x); }
+__device__ __forceinline__ double sqrt_t(double x) { return sqrt_d(x); }
 
 enum { KW0 = 0, KW1, KWOMEGA, KWZETA, KWGRAV, KWPOT, KW0S2, KWOMEGAS2, KWZETAS2 };
 
@@ -42,12 +44,6 @@ template <typename T> __device__ __forceinline__ T m4_w0(T norm, T s) {
 template <typename T> __device__ __forceinline__ T m4_w1(T norm, T s) {
   if (s < T(1)) return norm*(T(-3)*s + T(2.25)*s*s);
   if (s < T(2)) return T(-0.75)*norm*(T(2) - s)*(T(2) - s);
-  return T(0);
-}
-template <typename T> __device__ __forceinline__ T m4_womega(T norm, T s) {
-  const T s3 = s*s*s;
-  if (s < T(1)) return norm*(T(-3) + T(1.5)*T(5)*s*s - T(0.75)*T(6)*s3);
-  if (s < T(2)) return norm*(T(-6) + T(3)*T(4)*s - T(1.5)*T(5)*s*s + T(0.25)*T(6)*s3);
   return T(0);
 }
 template <typename T> __device__ __forceinline__ T m4_wzeta(T s) {
@@ -86,17 +82,6 @@ template <typename T> __device__ __forceinline__ T q_w1(T norm, T s) {
   if (s < T(1)) return norm*(T(-120)*s + T(120)*s3 - T(50)*s4);
   if (s < T(2)) return norm*(T(75) - T(420)*s + T(450)*s2 - T(180)*s3 + T(25)*s4);
   if (s < T(3)) return norm*(T(-405) + T(540)*s - T(270)*s2 + T(60)*s3 - T(5)*s4);
-  return T(0);
-}
-template <typename T> __device__ __forceinline__ T q_womega(T norm, T s) {
-  const T s2 = s*s, s3 = s2*s, s4 = s2*s2, s5 = s4*s;
-  if (s < T(1)) return norm*(T(-198) + T(60)*T(5)*s2 - T(30)*T(7)*s4 + T(10)*T(8)*s5);
-  if (s < T(2))
-    return norm*(T(-153) - T(75)*T(4)*s + T(210)*T(5)*s2 - T(150)*T(6)*s3 + T(45)*T(7)*s4 -
-                 T(5)*T(8)*s5);
-  if (s < T(3))
-    return norm*(T(-729) + T(405)*T(4)*s - T(270)*T(5)*s2 + T(90)*T(6)*s3 - T(15)*T(7)*s4 +
-                 T(8)*s5);
   return T(0);
 }
 template <typename T> __device__ __forceinline__ T q_wzeta(T s) {
@@ -141,11 +126,6 @@ template <typename T> __device__ __forceinline__ T tab_lin(const KernelDesc& k, 
   if (s >= T(k.range)) return T(0);
   return ktab<T>(k)[w*k.res + (int) (s*T(k.resinv))];
 }
-template <typename T> __device__ __forceinline__ T tab_sq(const KernelDesc& k, int w, T s2) {
-  if (s2 >= T(k.rangesqd)) return T(0);
-  return ktab<T>(k)[w*k.res + (int) (s2*T(k.resinvsqd))];
-}
-
 template <typename T> __device__ __forceinline__ T kw0(const KernelDesc& k, T s) {
   if (k.tabulated) return tab_lin<T>(k, KW0, s);
   return k.type == 0 ? m4_w0<T>(T(k.norm), s) : q_w0<T>(T(k.norm), s);
@@ -154,23 +134,17 @@ template <typename T> __device__ __forceinline__ T kw0(const KernelDesc& k, T s)
 // W and dW/ds as truncated powers, i.e. the reference's piecewise polynomials summed without the
 // cancellation of their expanded form: M4 W = (norm/4)[(2-s)^3_+ - 4(1-s)^3_+], quintic
 // W = norm[(3-s)^5_+ - 6(2-s)^5_+ + 15(1-s)^5_+]; womega = -3 w0 - s w1 exactly for both.
+// With W = norm sum_k c_k (a_k - s)^n_+ (M4: n = 3, a = 2, 1, c = 1, -4; quintic: n = 5,
+// a = 3, 2, 1, c = 1, -6, 15), the enclosed mass M(s) and the outer potential integral
+// P(s) = 4 pi int_s^inf u W du are polynomials in x_k = (a_k - s)_+:
+//   M = 1 - sum_k c_k x_k^(n+1) (a_k^2/(n+1) - 2 a_k x_k/(n+2) + x_k^2/(n+3)) * C,
+//   P = sum_k c_k x_k^(n+1) (a_k/(n+1) - x_k/(n+2)) * C      (C = 1 for M4, 1/30 quintic),
+// and wgrav = M/s^2, wpot = M/s + P, wzeta = wpot - s wgrav = P.  These are the reference's
+// piecewise polynomials (SmoothingKernel.h:132-408) summed without branches; the reference's
+// quintic wgrav and wpot carry 360/359 inside the kernel (its 12/359 in place of 1/30) and its
+// quintic wzeta is -30 P, both kept.  Below s = 1 the mass comes from the inner polynomial,
+// which avoids the cancellation of 1 - (...) at small s.
 template <typename T> __device__ __forceinline__ T tpos(T x) { return x > T(0) ? x : T(0); }
-
-template <typename T>
-__device__ __forceinline__ void kw01_an(int type, T norm, T s, T& w0, T& w1) {
-  if (type == 0) {
-    const T A = tpos(T(2) - s), B = tpos(T(1) - s);
-    const T A2 = A*A, B2 = B*B;
-    w0 = T(0.25)*norm*(A2*A - T(4)*(B2*B));
-    w1 = T(-0.75)*norm*(A2 - T(4)*B2);
-  } else {
-    const T A = tpos(T(3) - s), B = tpos(T(2) - s), C = tpos(T(1) - s);
-    const T A2 = A*A, B2 = B*B, C2 = C*C;
-    const T A4 = A2*A2, B4 = B2*B2, C4 = C2*C2;
-    w0 = norm*(A4*A - T(6)*(B4*B) + T(15)*(C4*C));
-    w1 = T(-5)*norm*(A4 - T(6)*B4 + T(15)*C4);
-  }
-}
 
 template <typename T> __device__ __forceinline__ T kw1(const KernelDesc& k, T s) {
   if (k.tabulated) return tab_lin<T>(k, KW1, s);
@@ -198,78 +172,115 @@ template <typename T> __device__ __forceinline__ T kwpot(const KernelDesc& k, T 
   }
   return k.type == 0 ? m4_wpot<T>(s) : q_wpot<T>(s);
 }
-// ---- branch-free gravity kernels for the FP32 pair sums ----
-// With W written as truncated powers, W = norm sum_k c_k (a_k - s)^n_+ (M4: n = 3, a = 2, 1,
-// c = 1, -4; quintic: n = 5, a = 3, 2, 1, c = 1, -6, 15), the enclosed mass M(s) and the
-// outer potential integral P(s) = 4 pi int_s^inf u W du are polynomials in x_k = (a_k - s)_+:
-//   M = 1 - sum_k c_k x_k^(n+1) (a_k^2/(n+1) - 2 a_k x_k/(n+2) + x_k^2/(n+3)) * C,
-//   P = sum_k c_k x_k^(n+1) (a_k/(n+1) - x_k/(n+2)) * C      (C = 1 for M4, 1/30 quintic),
-// and wgrav = M/s^2, wpot = M/s + P, wzeta = wpot - s wgrav = P.  These are the reference's
-// piecewise polynomials (SmoothingKernel.h:132-408) summed without branches; the reference's
-// quintic wgrav and wpot carry 360/359 inside the kernel (its 12/359 in place of 1/30) and its
-// quintic wzeta is -30 P, both kept.  Below s = 1 the mass comes from the inner polynomial,
-// which avoids the cancellation of 1 - (...) at small s.  Agreement with the reference's
-// polynomials: ~1e-8 relative (wgrav), ~1e-12 (wpot), within the reference's own constants
-// (wzeta) -- far below FP32 rounding; the FP64 path keeps the piecewise forms.
-__device__ __forceinline__ void kgravpot_f(const KernelDesc& k, float s, float inv, float& wg,
-                                           float& wp) {
-  if (k.tabulated) { wg = kwgrav<float>(k, s); wp = kwpot<float>(k, s); return; }
-  const float x1 = fmaxf(1.f - s, 0.f), x2 = fmaxf(2.f - s, 0.f);
-  const float x1s = x1*x1, x2s = x2*x2, s2 = s*s;
-  if (k.type == 0) {
-    const float x1q = x1s*x1s, x2q = x2s*x2s;
-    const float D = fmaf(-4.f*x1q, fmaf(x1, fmaf(x1, 1.f/6.f, -0.4f), 0.25f),
-                         x2q*fmaf(x2, fmaf(x2, 1.f/6.f, -0.8f), 1.f));
-    const float P = fmaf(-4.f*x1q, fmaf(x1, -0.2f, 0.25f), x2q*fmaf(x2, -0.2f, 0.5f));
-    const float Min = s2*s*fmaf(s2, fmaf(s, 0.5f, -1.2f), 4.f/3.f);
-    const float M = s < 1.f ? Min : 1.f - D;
-    wg = M*inv*inv;
-    wp = fmaf(M, inv, P);
-    return;
+// ---- sums of the h-rho pass ----
+// KT: 0 M4, 1 quintic, 2 tabulated; the sums of the density triple at s^2 (GradhSph.cpp:197-204).
+// The analytic kernels in truncated powers, their constant factors taken out of the sums: with w0, w1
+// and P without the norm, womega = -3 w0 - s w1 makes sum(m womega) two sums, and wzeta is P (M4)
+// or -30 P (quintic).  The reference's quintic wzeta polynomials are rounded to ten digits: their
+// differences from -30 P, a constant and an s^7 term per segment, are added in FP64.
+template <typename T, int KT> struct DensSums {
+  T r = T(0), o = T(0), z = T(0);
+  __device__ __forceinline__ void add(const KernelDesc& k, T ssqd, T m) {
+    if (KT == 2) {
+      if (ssqd >= T(k.rangesqd)) return;
+      const int i = (int) (ssqd*T(k.resinvsqd));
+      const T* t = ktab<T>(k);
+      r += m*t[KW0S2*k.res + i]; o += m*t[KWOMEGAS2*k.res + i]; z += m*t[KWZETAS2*k.res + i];
+      return;
+    }
+    const T s = sqrt_t(ssqd);
+    const T c = tpos(T(1) - s), b = tpos(T(2) - s);
+    const T c2 = c*c, b2 = b*b;
+    if (KT == 0) {
+      const T w1 = b2 - T(4)*c2;                        // -4/3 w1
+      const T c4 = c2*c2, b4 = b2*b2;
+      r += m*(b*b2 - T(4)*(c*c2));                      // 4 w0
+      o += (m*s)*w1;
+      z += m*(b4*(T(0.5) - T(0.2)*b) - T(4)*c4*(T(0.25) - T(0.2)*c));
+    } else {
+      const T a = tpos(T(3) - s);
+      const T a2 = a*a;
+      const T a4 = a2*a2, b4 = T(-6)*(b2*b2), c4 = T(15)*(c2*c2);
+      r += m*(a4*a + b4*b + c4*c);                      // w0
+      o += (m*s)*(a4 + b4 + c4);                        // -w1/5
+      T p = (a4*a2)*(T(0.5) - T(1.0/7.0)*a) + (b4*b2)*(T(1.0/3.0) - T(1.0/7.0)*b) +
+            (c4*c2)*(T(1.0/6.0) - T(1.0/7.0)*c);        // 30 P
+      if (sizeof(T) == 8) {
+        const double d0 = s < T(1) ? 34.14285714 - 239.0/7.0
+                                   : s < T(2) ? 33.785714286 - 236.5/7.0
+                                              : 52.07142857 - 364.5/7.0;
+        const double d7 = s < T(1) ? 1.42857142857 - 10.0/7.0
+                                   : s < T(2) ? 5.0/7.0 - 0.7142857143 : 0.142857143 - 1.0/7.0;
+        const T s2 = s*s;
+        const T d = T(d0) + T(d7)*((s2*s2)*(s2*s));
+        p += s < T(3) ? d : T(0);
+      }
+      z += m*p;
+    }
   }
-  const float x3 = fmaxf(3.f - s, 0.f), x3s = x3*x3;
-  const float x1h = x1s*x1s*x1s, x2h = x2s*x2s*x2s, x3h = x3s*x3s*x3s;
-  const float D = fmaf(15.f*x1h, fmaf(x1, fmaf(x1, 0.125f, -2.f/7.f), 1.f/6.f),
-                  fmaf(-6.f*x2h, fmaf(x2, fmaf(x2, 0.125f, -4.f/7.f), 2.f/3.f),
-                       x3h*fmaf(x3, fmaf(x3, 0.125f, -6.f/7.f), 1.5f)));
-  const float P30 = fmaf(15.f*x1h, fmaf(x1, -1.f/7.f, 1.f/6.f),
-                    fmaf(-6.f*x2h, fmaf(x2, -1.f/7.f, 1.f/3.f), x3h*fmaf(x3, -1.f/7.f, 0.5f)));
-  const float Min = s2*s*fmaf(s2, fmaf(s2, fmaf(s, -1.25f, 30.f/7.f), -12.f), 22.f)*(1.f/30.f);
-  const float M = s < 1.f ? Min : fmaf(D, -1.f/30.f, 1.f);
-  const float f = s < 3.f ? 360.f/359.f : 1.f;
-  wg = f*M*inv*inv;
-  wp = f*fmaf(M, inv, P30*(1.f/30.f));
-}
-
-// wzeta of the analytic kernels in FP32 without branches: P(s) for M4, -30 P(s) for quintic
-__device__ __forceinline__ float kwzeta_f(int type, float s) {
-  const float x1 = fmaxf(1.f - s, 0.f), x2 = fmaxf(2.f - s, 0.f);
-  const float x1s = x1*x1, x2s = x2*x2;
-  if (type == 0)
-    return fmaf(-4.f*x1s*x1s, fmaf(x1, -0.2f, 0.25f), x2s*x2s*fmaf(x2, -0.2f, 0.5f));
-  const float x3 = fmaxf(3.f - s, 0.f), x3s = x3*x3;
-  return -fmaf(15.f*x1s*x1s*x1s, fmaf(x1, -1.f/7.f, 1.f/6.f),
-               fmaf(-6.f*x2s*x2s*x2s, fmaf(x2, -1.f/7.f, 1.f/3.f),
-                    x3s*x3s*x3s*fmaf(x3, -1.f/7.f, 0.5f)));
-}
-
-// density triple w0, womega, wzeta at s^2 (GradhSph.cpp:197-204)
-template <typename T>
-__device__ __forceinline__ void kdens(const KernelDesc& k, T s2, T& w0, T& wom, T& wz) {
-  if (k.tabulated) {
-    if (s2 >= T(k.rangesqd)) { w0 = wom = wz = T(0); return; }
-    const int idx = (int) (s2*T(k.resinvsqd));
-    const T* t = ktab<T>(k);
-    w0 = t[KW0S2*k.res + idx]; wom = t[KWOMEGAS2*k.res + idx]; wz = t[KWZETAS2*k.res + idx];
-    return;
+  // sum(m w0), sum(m womega), sum(m wzeta) of these sums
+  __device__ __forceinline__ static void finish(const KernelDesc& k, double& r_, double& o_,
+                                                double& z_) {
+    if (KT == 2) return;
+    if (KT == 0) {
+      r_ *= 0.25*k.norm;
+      o_ = -3.0*r_ + 0.75*k.norm*o_;
+    } else {
+      r_ *= k.norm;
+      o_ = -3.0*r_ + 5.0*k.norm*o_;
+      z_ = -z_;
+    }
   }
-  const T s = sizeof(T) == 4 ? (T) sqrt_f((float) s2) : (T) sqrt((double) s2);
-  T w1;
-  kw01_an<T>(k.type, T(k.norm), s, w0, w1);
-  wom = T(-3)*w0 - s*w1;
-  if (sizeof(T) == 4) wz = (T) kwzeta_f(k.type, (float) s);
-  else wz = k.type == 0 ? m4_wzeta<T>(s) : q_wzeta<T>(s);
-}
+};
+
+// ---- kernels of the hydro pairs ----
+// KT as DensSums.  set(s): w1 without its constant factor (w1_factor).  grav: the enclosed mass M
+// and outer potential integral P above, with the reference's 360/359 (quintic, inside the
+// kernel): wgrav = M/s^2, wpot = M/s + P.  The truncated-power forms are the reference's
+// piecewise polynomials exactly, so the FP64 path takes them too: no branches, and the terms of
+// the force and the potential share their powers.  (Tabulated kernels: M = s^2 wgrav, and P is
+// what then remains of wpot.)
+template <typename T, int KT> struct HydroKern {
+  T w1, s, a, b, c, a2, b2, c2, a4, b4, c4;
+  __device__ __forceinline__ static double w1_factor(const KernelDesc& k) {
+    return KT == 0 ? -0.75*k.norm : KT == 1 ? -5.0*k.norm : 1.0;
+  }
+  __device__ __forceinline__ void set(const KernelDesc& k, T s_) {
+    s = s_;
+    if (KT == 2) { w1 = tab_lin<T>(k, KW1, s); return; }
+    b = tpos(T(2) - s); c = tpos(T(1) - s);
+    b2 = b*b; c2 = c*c;
+    if (KT == 0) { w1 = b2 - T(4)*c2; return; }
+    a = tpos(T(3) - s);
+    a2 = a*a;
+    a4 = a2*a2; b4 = T(-6)*(b2*b2); c4 = T(15)*(c2*c2);
+    w1 = a4 + b4 + c4;
+  }
+  __device__ __forceinline__ void grav(const KernelDesc& k, T& M, T& P) const {
+    if (KT == 2) {
+      M = kwgrav<T>(k, s)*(s*s);
+      P = s > T(0) ? kwpot<T>(k, s) - M/s : kwpot<T>(k, s);
+    } else if (KT == 0) {
+      const T x = b2*b2, y = T(-4)*(c2*c2);
+      const T D = x*(T(1) + b*(b*T(1.0/6.0) - T(0.8))) + y*(T(0.25) + c*(c*T(1.0/6.0) - T(0.4)));
+      P = x*(T(0.5) - T(0.2)*b) + y*(T(0.25) - T(0.2)*c);
+      const T s2 = s*s;
+      const T in = (s2*s)*(T(4.0/3.0) + s2*(T(0.5)*s - T(1.2)));
+      M = s < T(1) ? in : T(1) - D;
+    } else {
+      const T x = a4*a2, y = b4*b2, z = c4*c2;
+      const T D = x*(T(1.5) + a*(T(0.125)*a - T(6.0/7.0))) +
+                  y*(T(2.0/3.0) + b*(T(0.125)*b - T(4.0/7.0))) +
+                  z*(T(1.0/6.0) + c*(T(0.125)*c - T(2.0/7.0)));
+      const T f = T(12.0/359.0);
+      P = f*(x*(T(0.5) - T(1.0/7.0)*a) + y*(T(1.0/3.0) - T(1.0/7.0)*b) +
+             z*(T(1.0/6.0) - T(1.0/7.0)*c));
+      const T s2 = s*s;
+      const T in = (f*(s2*s))*(T(22) + s2*(T(-12) + s2*(T(30.0/7.0) - T(1.25)*s)));
+      M = s < T(1) ? in : (s < T(3) ? T(360.0/359.0) : T(1)) - f*D;
+    }
+  }
+};
 
 // wzeta at s^2 alone (the stars' zeta terms, GradhSph.cpp:289-303)
 __device__ __forceinline__ double kwzeta_s2(const KernelDesc& k, double s2) {
@@ -366,6 +377,9 @@ __device__ __forceinline__ double range2_rn(double krsqd, double h) {
 __device__ __forceinline__ float dot3_f(float a, float b, float c) {
   return fmaf(c, c, fmaf(b, b, a*a));
 }
+
+__device__ __forceinline__ float dot3_t(float a, float b, float c) { return dot3_f(a, b, c); }
+__device__ __forceinline__ double dot3_t(double a, double b, double c) { return dot3_rn(a, b, c); }
 
 // Kernel-range box test of the gravity walk with a relative slack: a node whose box comes within
 // (1 + slack) k max(h) of the group is resolved to particles, so no pair of the scatter-gather

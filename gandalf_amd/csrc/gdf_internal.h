@@ -104,9 +104,9 @@ struct TreeView {
   const double* mp;       // 10 doubles per node: comx comy comz m q0..q4 pad
 };
 
-// Candidate set of the SPH passes, per walk group g: idx[g][b*64 + c] is candidate c of batch b,
-// mask[g][b*64 + l] the 64-bit set of batch-b candidates inside target l's range, ncand[g] the
-// number of candidates.  capb batches are reserved per group.
+// Candidate set of the SPH passes, per walk group g: idx[g][k] is candidate k in walk order,
+// ncand[g] their number; capb*64 are reserved per group.  The parity tap's set also holds
+// mask[g][b*64 + l], the candidates b, b + nbat, ... inside target l's range.
 struct CandSet {
   int* idx = nullptr;
   unsigned long long* mask = nullptr;

@@ -5,23 +5,29 @@
 // per-particle physics of GradhSph::ComputeH (src/GradhSph/GradhSph.cpp:142-326) and
 // ComputeSphHydroForces / ComputeSphHydroGravForces (:361-460, :474-585).
 //
-// Work mapping: one wavefront per walk group (a tree node of <= 64 Morton-consecutive
-// particles, one target per lane).  A walk pass resolves the group's candidate particles from
-// the tree once (all particles of buckets that come within the group's search range, in walk
-// order) and, for every batch of up to 64 candidates, records one 64-bit mask per target
-// holding the candidates that are inside that target's own range (the exact neighbour test).
-// Batch b of nbat takes the candidates at walk positions b, b + nbat, b + 2 nbat, ...: every
-// batch then samples the whole candidate region, each target's neighbours spread evenly over
-// the batches, and the per-target mask loops below leave fewer lanes idle than with batches of
-// consecutive (spatially clustered) candidates.  The pair passes stage each batch's candidate
-// records in LDS with one load per lane, shared by all 64 targets, and every lane walks the set
-// bits of its own mask.  The h-rho pass re-sweeps the same batches until every target of the
-// group has converged.  A target sums its neighbours batch by batch, in bit order within a
-// batch.
+// Work mapping: a walk pass (one wavefront per walk group, a tree node of up to 64
+// Morton-consecutive particles) resolves the group's candidate particles from the tree: the
+// members of every bucket that come within the group's search range, in walk order.  The h-rho
+// pass walks with bounds that also hold the scatter-gather sets of the converged smoothing
+// lengths, so the force pass reads the same lists.  A pair pass takes one walk group per
+// workgroup, one target a lane, and its wavefronts share the group's candidates: each stages its
+// own in LDS batch by batch, filters them against the 64 targets on the matrix cores
+// (gdf_filter.h) and lets every lane take its own target's hits, deciding each pair by the path's
+// own range test.  The h-rho pass re-sweeps the same candidates until every target of the group
+// has converged.
+//
+// The lists hold no masks: exact 64-bit masks per batch and target, made by the walk with 64
+// distance tests a candidate and read back by the pair passes, cost 12 to 19 VALU instructions a
+// test and 640 bytes a batch, and the FP64 force pass a walk of its own.  One FP64 force
+// evaluation of a million particles (quintic, 64-particle groups) takes 13.2 ms against 17.2 ms
+// with them: walks 0.88 against 1.51 + 1.52 ms, h-rho pass 1.51 (1.59), hydro pass 3.45 (5.06).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "gdf_internal.h"
 #include "gdf_device.h"
+#include "gdf_filter.h"
 
 namespace gdf {
 namespace {
@@ -39,7 +45,7 @@ struct CandWalk {
   const int4* lnk;
   const double4* geo_c; const double4* geo_h;
   const double* x; const double* y; const double* z; const double* hcand; const double* htarget;
-  const int* status;                 // gather walks: only targets with status 1 take part
+  const int* status;                 // only targets with status 1 take part (NULL = every member)
   const int* grp_root;               // serving batches: the group's segment subtree (NULL = root)
   const int* glist;                  // groups to walk (count at glist[Ncap]); NULL = all groups
   int ncap;
@@ -48,33 +54,21 @@ struct CandWalk {
   PhysParams p;
 };
 
-// The mixed gather pass's candidate radius^2 in FP32: k hs_i widened by 1e-6 of the group's
-// half-extent plus k hs_i, squared and widened by 1e-5 (r2i = (k hs_i)^2)
-__device__ __forceinline__ float gather_r2f(double r2i, const double4& gh) {
-#pragma clang fp contract(off)
-  const double rg = sqrt(r2i) + 1.0e-6*(gh.x + gh.y + gh.z + sqrt(r2i));
-  return (float) (rg*rg*(1.0 + 1.0e-5));
-}
-
-// MODE 0: search set |r_ij|^2 <= (k hs_i)^2 (FP64); 1: scatter-gather set
-// |r_ij|^2 < (k h_i)^2 or < (k h_j)^2 (FP64, the oracle's operation order); 2: the same set
-// decided in FP32 in the group-centred frame, exactly as the mixed-precision gravity walk
-// decides it; 3: a superset of the MODE 0 set decided in FP32 in the group-centred frame, the
-// radius widened by 1e-6 of the group's half-extent plus k hs_i (sixteen times the FP32
-// rounding of the frame's coordinates) and the square by 1e-5 (mixed h-rho pass: the extra
-// candidates lie beyond k h_i and carry zero weight).  PER: periodic nearest images.
-// MASKS = false (FP32 modes): the walk records the candidates only, and the pair pass that
-// reads them makes the same tests on its own staged records.  UNION (MODE 3, no masks): the
-// gather walk's candidates also include every particle whose own search radius reaches the
-// group box (hcand = the search radii hs_j = 1.05 h_j; a node's hs bound is 1.05 times its h
-// maximum), so that while no smoothing length outgrows its search radius the list holds the
-// scatter-gather set of the converged smoothing lengths as well.
-template <int MODE, bool PER, bool MASKS = true, bool UNION = false>
+// Candidate lists.  MODE 0: the gather search, every particle within k hs_i of a target (hs the
+// search radii); MODE 1, 2: scatter-gather, within k h_i of a target i or k h_j of its own.
+// UNION (MODE 0): the gather search's candidates also include every particle whose own search
+// radius reaches the targets' box (hcand = the search radii hs_j = 1.05 h_j; a node's hs bound is
+// 1.05 times its h maximum), so that while no smoothing length outgrows its search radius the
+// list holds the scatter-gather set of the converged smoothing lengths as well.  The lists err on
+// the inclusive side; the pair passes test every pair.  MASKS (the parity tap): also each target's exact scatter-gather set as masks over the list, MODE 1 in FP64 with
+// the oracle's operation order, MODE 2 in FP32 in the frame of the mixed path's pair kernels with
+// their expression.  PER: periodic nearest images.
+template <int MODE, bool PER, bool MASKS = false, bool UNION = false>
 __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
-  constexpr bool F32 = MODE >= 2;      // group-frame FP32 tests
-  constexpr bool GATHER = MODE == 0 || MODE == 3;
-  __shared__ double4 sc[F32 ? 1 : kWave];   // MODE 0/1: (x, y, z, (k h_j)^2)
-  __shared__ float4 fc[F32 ? kWave : 1];    // MODE 2/3: group-frame (x, y, z, (k h_j)^2)
+  constexpr bool F32 = MODE == 2;      // group-frame FP32 tests
+  constexpr bool GATHER = MODE == 0;
+  __shared__ double4 sc[MASKS && !F32 ? kWave : 1];   // MODE 1: (x, y, z, (k h_j)^2)
+  __shared__ float4 fc[MASKS && F32 ? kWave : 1];     // MODE 2: the same in the FP32 frame
   __shared__ int lstk[kLdsStack];    // node stack; deeper entries go to the global region
   const int lane = threadIdx.x;
   int* stk = a.stacks + (size_t) blockIdx.x*kStackCap;
@@ -88,39 +82,34 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
     if (k >= q.nq) break;
     const int g = a.glist ? a.glist[k] : k;
     const int G = a.grp_node[g], gfirst = a.grp_first[g], gcnt = a.grp_count[g];
+    // tc, th: the box the walk tests nodes and members against, that of the group's targets
+    // alone; a block step's sparse groups hold a few targets each and reach far fewer buckets
+    // with it.  hG: their largest search radius
+    double lox = HUGE_VAL, loy = HUGE_VAL, loz = HUGE_VAL, hG = 0.0;
+    double hix = -HUGE_VAL, hiy = -HUGE_VAL, hiz = -HUGE_VAL;
     const int i = gfirst + lane;
-    bool has = lane < gcnt;
-    if (has && a.status) has = a.status[i] == 1;
+    const bool has = lane < gcnt && (!a.status || a.status[i] == 1);
+    double xi = 0.0, yi = 0.0, zi = 0.0, r2i = 0.0;
+    if (has) {
+      lox = hix = xi = a.x[i]; loy = hiy = yi = a.y[i]; loz = hiz = zi = a.z[i];
+      hG = a.htarget[i];
+      r2i = range2_rn(krsqd, hG);
+    }
     if (__ballot(has) == 0) {        // nothing left to do in this group
       if (lane == 0) a.ncand[g] = 0;
       continue;
     }
-    double xi = 0.0, yi = 0.0, zi = 0.0, hi = 0.0, r2i = 0.0;
-    if (has) {
-      xi = a.x[i]; yi = a.y[i]; zi = a.z[i]; hi = a.htarget[i];
-      r2i = range2_rn(krsqd, hi);
-    }
-    const double hG = wave_max_d(has ? hi : 0.0);
-    // gc, gh: the group node's box, the frame of the FP32 tests.  tc, th: the box the walk
-    // tests nodes and members against, that of the group's targets alone (the refit's
-    // expressions, so it is the node's box when every member is a target); a block step's
-    // sparse groups hold a few targets each and reach far fewer buckets with it
-    const double4 gc = a.geo_c[G], gh = a.geo_h[G];
+    hG = wave_max_d(hG);
     double4 tc, th;
     {
 #pragma clang fp contract(off)
-      const double lox = -wave_max_d(has ? -xi : -HUGE_VAL), hix = wave_max_d(has ? xi : -HUGE_VAL);
-      const double loy = -wave_max_d(has ? -yi : -HUGE_VAL), hiy = wave_max_d(has ? yi : -HUGE_VAL);
-      const double loz = -wave_max_d(has ? -zi : -HUGE_VAL), hiz = wave_max_d(has ? zi : -HUGE_VAL);
+      lox = -wave_max_d(-lox); hix = wave_max_d(hix);
+      loy = -wave_max_d(-loy); hiy = wave_max_d(hiy);
+      loz = -wave_max_d(-loz); hiz = wave_max_d(hiz);
       tc = make_double4(0.5*(lox + hix), 0.5*(loy + hiy), 0.5*(loz + hiz), 0.0);
       th = make_double4(0.5*(hix - lox), 0.5*(hiy - loy), 0.5*(hiz - loz), 0.0);
     }
-    const float rxi = (float) (xi - gc.x), ryi = (float) (yi - gc.y), rzi = (float) (zi - gc.z);
-    const float r2if = (float) r2i;
-    float r2gf = 0.f;
-    if (MODE == 3 && has) r2gf = gather_r2f(r2i, gh);
     int* idx = a.idx + (size_t) g*a.capb*kWave;
-    unsigned long long* msk = a.mask + (size_t) g*a.capb*kWave;
     const int cap = a.capb*kWave;
     int sp = 1, tail = 0;
     bool overflow = false;
@@ -211,6 +200,10 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
       continue;
     }
     __threadfence_block();
+    unsigned long long* msk = a.mask + (size_t) g*a.capb*kWave;
+    const double4 gc = a.geo_c[G];
+    const float rxi = (float) (xi - gc.x), ryi = (float) (yi - gc.y), rzi = (float) (zi - gc.z);
+    const float r2if = (float) r2i;
     // 2. masks: batch b holds the candidates at walk positions b, b + nbat, b + 2 nbat, ...,
     // so every batch samples the whole candidate region and each target's neighbours spread
     // evenly over the batches (fewer idle lanes in the per-target mask loops of the pair passes)
@@ -218,7 +211,7 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
     // candidate indices of batch b + 2 with them.
     auto nbat_of = [&](int bb) { return (tail - bb + nbat - 1)/nbat; };
     auto record = [&](int j) {
-      return make_double4(a.x[j], a.y[j], a.z[j], GATHER ? 0.0 : a.hcand[j]);
+      return make_double4(a.x[j], a.y[j], a.z[j], a.hcand[j]);
     };
     double4 cur = make_double4(0.0, 0.0, 0.0, 0.0), nxt = cur;
     int jn = 0;
@@ -227,7 +220,7 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
     for (int b = 0; b < nbat; b++) {
       const int nb = nbat_of(b);
       if (lane < nb) {
-        const double r2j = GATHER ? 0.0 : range2_rn(krsqd, cur.w);
+        const double r2j = range2_rn(krsqd, cur.w);
         if (F32) {
           double dx = cur.x - gc.x, dy = cur.y - gc.y, dz = cur.z - gc.z;
           nearest_image<double>(pp, dx, dy, dz);
@@ -248,10 +241,7 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
         #pragma unroll 16
         for (int q = 0; q < kWave; q++) {
           bool in;
-          if (MODE == 3) {
-            const float4 c = fc[q];
-            in = dot3_f(c.x - rxi, c.y - ryi, c.z - rzi) <= r2gf;
-          } else if (MODE == 2) {
+          if (F32) {
             const float4 c = fc[q];
             const float d2 = dot3_f(c.x - rxi, c.y - ryi, c.z - rzi);
             in = (d2 < r2if) | (d2 < c.w);
@@ -260,8 +250,7 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
             double dx = c.x - xi, dy = c.y - yi, dz = c.z - zi;
             nearest_image<double>(pp, dx, dy, dz);
             const double d2 = dot3_rn(dx, dy, dz);
-            if (MODE == 0) in = d2 <= r2i;
-            else in = (d2 < r2i) | (d2 < c.w);
+            in = (d2 < r2i) | (d2 < c.w);
           }
           m |= (unsigned long long) in << q;
         }
@@ -280,7 +269,7 @@ struct DensArgs {
   int N, ngroups, capb, nopbc;
   const int* grp_node; const int* grp_first; const int* grp_count; const double4* geo_c;
   const double4* geo_h;
-  const int* idx; unsigned long long* mask; const int* ncand;
+  const int* idx; const int* ncand;
   const double4* posm;
   double* h; double* hsearch; double* rho; double* invomega; double* zeta; double* hfactor;
   double* u; double* sound; double* pressure;
@@ -299,7 +288,7 @@ __device__ __forceinline__ int hrho_step(const PhysParams& p, double m, double h
                                          double rho, double& h, double& h_lower,
                                          double& h_upper) {
   const double invh = 1.0/h;
-  const double hrho = rho > 0.0 ? p.h_fac*pow(m/rho, 1.0/3) : 0.0;
+  const double hrho = rho > 0.0 ? p.h_fac*cbrt(m/rho) : 0.0;
   if (rho > 0.0 && h > h_lower && fabs(h - hrho)*invh < p.h_converge) return 1;
   if (iteration < p.hrho_itmax) h = hrho;
   else if (iteration == p.hrho_itmax) h = 0.5*(h_lower + h_upper);
@@ -342,144 +331,171 @@ __device__ void hrho_finish(const DensArgs& a, const PhysParams& p, int i, doubl
   a.u[i] = u; a.sound[i] = snd; a.pressure[i] = press;
 }
 
-// h-rho pass over one walk group per workgroup.  T = double: FP64 sums in candidate order;
-// T = float: FP32 pair terms in the group-centred frame, per-batch register sums and
-// Kahan-compensated totals (the convergence test and the final h stay FP64).  FUSED (FP32): the
-// candidate walk recorded no masks; the first sweep tests each staged batch against the
-// target's widened radius exactly as the walk's MODE 3 would, keeps the masks for the later
-// sweeps and sums the same pairs.
-template <typename T, bool FUSED = false>
-__global__ __launch_bounds__(64) void k_density(DensArgs a) {
-  __shared__ double4 sd[kWave];
-  __shared__ float4 sf[kWave];
+// h-rho pass, one walk group per workgroup, its W wavefronts sharing the candidates.  A sweep
+// stages the candidates' positions batch by batch, filters them against the targets' current
+// ranges and sums the hits; every wavefront adds the W partial sums in the same order and takes
+// the same step of the iteration.  T = double: FP64 sums; T = float: FP32 pair terms in the group-centred frame summed
+// batch by batch, FP64 totals (the convergence test and the final h are always FP64).  KT:
+// DensSums' kernel.
+// Bound by vector issue where the device is full (1M particles, quintic: 0.25 VALU instructions
+// a cycle and SIMD), by the latency of the dependent loads and of each sweep's reduction below;
+// 3 wavefronts a SIMD, as 4 spill.  1M, quintic: 0.95 ms against 1.20 with masks (FP32), 1.51
+// against 1.59 (FP64).
+template <typename T, int KT, int W>
+__global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
+  constexpr bool F64 = sizeof(T) == 8;
+  typedef typename std::conditional<F64, double4, float4>::type Rec;
+  __shared__ Rec stage[W][kPairSlots];
+  __shared__ double red[W > 1 ? W : 1][3][W > 1 ? kWave : 1];
   const int g = xcd_block(blockIdx.x, gridDim.x);
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & (kWave - 1), wv = W == 1 ? 0 : (int) threadIdx.x/kWave;
   const int nc = a.ncand[g];
   if (nc <= 0 || nc > a.capb*kWave) return;   // no active target, or the walk overflowed
   const int gfirst = a.grp_first[g], gcnt = a.grp_count[g];
+  Rec* const st = stage[wv];
   const int i = gfirst + lane;
-  const bool has = lane < gcnt;
-  int state = (has && a.status[i] == 1) ? 2 : 3;     // 2 iterating, 3 not a target here
+  const bool has = lane < gcnt && a.status[i] == 1;
+  int state = has ? 2 : 3;                    // 2 iterating, 3 not a target
   PhysParams p = a.p;
   if (a.nopbc) p.periodic = 0;
-  const double4 gc = a.geo_c[a.grp_node[g]];
-  const double4 me = has ? a.posm[i] : make_double4(0.0, 0.0, 0.0, 1.0);
+  const double4 gc = a.geo_c[a.grp_node[g]], gh = a.geo_h[a.grp_node[g]];
+  double4 me = make_double4(gc.x, gc.y, gc.z, 1.0);
+  double h = 1.0, hmax = 1.0;
+  if (has) { me = a.posm[i]; h = a.h[i]; hmax = a.hsearch[i]; }
   const double m = me.w;
-  double h = has ? a.h[i] : 1.0;
-  const double hmax = has ? a.hsearch[i] : 1.0;
   double h_lower = 0.0, h_upper = hmax;
-  int iteration = 0;
-  long long ngather = 0, evals = 0;
+  int iteration = 0, ngather = 0, evals = 0;
   const float rxi = (float) (me.x - gc.x), ryi = (float) (me.y - gc.y), rzi = (float) (me.z - gc.z);
   const double rsq = p.kern.rangesqd;
-  const int nbat = (nc + kWave - 1)/kWave;
-  const int* idx = a.idx + (size_t) g*a.capb*kWave;
-  unsigned long long* msk = a.mask + (size_t) g*a.capb*kWave;
-  float r2gf = 0.f;
-  if (FUSED && state == 2) r2gf = gather_r2f(range2_rn(rsq, hmax), a.geo_h[a.grp_node[g]]);
-  bool first = true;
+  // the filter's frame: the group's half-diagonal plus the targets' largest search range below one
+  const double rG = p.kern.range*wave_max_d(has ? hmax : 0.0);
+  const float fs = filter_scale(sqrt(gh.x*gh.x + gh.y*gh.y + gh.z*gh.z) + rG);
+  // FP64 separations take the nearest image target by target: where a candidate's image about
+  // the group's centre need not be its image about every target, all candidates are taken
+  const bool all = F64 && p.periodic && (gh.x + rG >= p.boxhalf[0] || gh.y + rG >= p.boxhalf[1] ||
+                                         gh.z + rG >= p.boxhalf[2]);
+  FiltTargets ft;
+  ft.position(rxi*fs, ryi*fs, rzi*fs);
+  const PairBatches pb((nc - wv + W - 1)/W);
+  const int* idx = a.idx + (size_t) g*a.capb*kWave + wv;
   while (__ballot(state == 2)) {
     const bool run = state == 2;
     if (run) iteration++;
     const double invh = 1.0/h;
-    const double hfac3 = invh*invh*invh;
     const double invhsqd = invh*invh;
-    const float invhf = (float) invh, invhsqdf = (float) invhsqd;
+    const float invhsqdf = (float) invhsqd, hs = (float) h*fs;
+    ft.range(rxi*fs, ryi*fs, rzi*fs, run ? (float) rsq*hs*hs : -1.f);
     int inside = 0;
-    double r_ = 0.0, om_ = 0.0, z_ = 0.0;
-    KahanF kr, kom, kz;
-    for (int b = 0; b < nbat; b++) {
-      const int nb = (nc - b + nbat - 1)/nbat;   // candidates b, b + nbat, ...
-      if (lane < nb) {
-        const double4 pj = a.posm[idx[b + lane*nbat]];
-        if (sizeof(T) == 8) {
-          sd[lane] = pj;
-        } else {
-          double dx = pj.x - gc.x, dy = pj.y - gc.y, dz = pj.z - gc.z;
-          nearest_image<double>(p, dx, dy, dz);
-          sf[lane] = make_float4((float) dx, (float) dy, (float) dz, (float) pj.w);
-        }
+    DensSums<double, KT> sum;
+    HitQueue hq;
+    Rec rec{};
+    // the next batch's record and the indices of the one after it are in flight
+    double4 nx = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (pb.filled(0, lane)) nx = a.posm[idx[pb.index(0, lane)*W]];
+    int jn = pb.filled(1, lane) ? idx[pb.index(1, lane)*W] : -1;
+    for (int b = 0; b < pb.nb; b++) {
+      const int s0 = kWave*(b & 1);
+      if constexpr (F64) {
+        st[s0 + lane] = nx;
+      } else {
+        double dx = nx.x - gc.x, dy = nx.y - gc.y, dz = nx.z - gc.z;
+        nearest_image<double>(p, dx, dy, dz);
+        st[s0 + lane] = make_float4((float) dx, (float) dy, (float) dz, (float) nx.w);
       }
+      wave_lds_order();
+      if (jn >= 0) nx = a.posm[jn];
+      jn = pb.filled(b + 2, lane) ? idx[pb.index(b + 2, lane)*W] : -1;
+      const uint2 hit = filter64<false>(ft, [&](int l) {
+        FiltCand f;
+        const Rec r = st[s0 + l];
+        if (F64) {
+          double dx = r.x - gc.x, dy = r.y - gc.y, dz = r.z - gc.z;
+          nearest_image<double>(p, dx, dy, dz);
+          f.x = (float) dx; f.y = (float) dy; f.z = (float) dz;
+        } else {
+          f.x = (float) r.x; f.y = (float) r.y; f.z = (float) r.z;
+        }
+        f.x *= fs; f.y *= fs; f.z *= fs; f.thr = 0.f;
+        f.state = !pb.filled(b, l) ? 1 : all ? -1 : 0;
+        return f;
+      });
+      hq.stage(b == 0, run ? hit : make_uint2(0u, 0u));
+      const int need = b + 1 < pb.nb ? hq.older : hq.staged;
+      if constexpr (F64) {
+        hq.run(need, rec, [&](int q) { return st[q]; }, [&](const Rec& pj, bool take) {
+          double dx = pj.x - me.x, dy = pj.y - me.y, dz = pj.z - me.z;
+          nearest_image<double>(p, dx, dy, dz);
+          const double ssqd = invhsqd*(dx*dx + dy*dy + dz*dz);
+          inside += take & (ssqd < rsq);
+          sum.add(p.kern, ssqd, take ? pj.w : 0.0);
+        });
+      } else {
+        DensSums<float, KT> part;
+        hq.run(need, rec, [&](int q) { return st[q]; }, [&](const Rec& pj, bool take) {
+          const float dx = pj.x - rxi, dy = pj.y - ryi, dz = pj.z - rzi;
+          const float ssqd = invhsqdf*(dx*dx + dy*dy + dz*dz);
+          inside += take & (ssqd < (float) rsq);
+          part.add(p.kern, ssqd, take ? pj.w : 0.f);
+        });
+        sum.r += (double) part.r; sum.o += (double) part.o; sum.z += (double) part.z;
+      }
+      wave_lds_order();
+    }
+    evals += hq.staged;
+    double r_ = sum.r, om_ = sum.o, z_ = sum.z;
+    if (W > 1) {
+      red[wv][0][lane] = r_; red[wv][1][lane] = om_; red[wv][2][lane] = z_;
       __syncthreads();
-      if (run) {
-        unsigned long long mk;
-        if (FUSED && first) {
-          mk = 0;
-          #pragma unroll 16
-          for (int q = 0; q < kWave; q++) {
-            const float4 c = sf[q];
-            mk |= (unsigned long long) (dot3_f(c.x - rxi, c.y - ryi, c.z - rzi) <= r2gf) << q;
-          }
-          if (nb < kWave) mk &= (1ULL << nb) - 1ULL;
-          msk[b*kWave + lane] = mk;
-        } else {
-          mk = msk[b*kWave + lane];
-        }
-        evals += __popcll(mk);
-        if (sizeof(T) == 8) {
-          while (mk) {
-            const int q = __builtin_ctzll(mk);
-            mk &= mk - 1;
-            const double4 pj = sd[q];
-            double dx = pj.x - me.x, dy = pj.y - me.y, dz = pj.z - me.z;
-            nearest_image<double>(p, dx, dy, dz);
-            const double ssqd = invhsqd*(dx*dx + dy*dy + dz*dz);
-            inside += ssqd < rsq;
-            double w0, wom, wz;
-            kdens<double>(p.kern, ssqd, w0, wom, wz);
-            r_ += pj.w*w0;
-            om_ += pj.w*invh*wom;
-            z_ += pj.w*wz;
-          }
-        } else {
-          float br = 0.f, bom = 0.f, bz = 0.f;
-          while (mk) {
-            const int q = __builtin_ctzll(mk);
-            mk &= mk - 1;
-            const float4 c = sf[q];
-            const float dx = c.x - rxi, dy = c.y - ryi, dz = c.z - rzi;
-            const float ssqd = invhsqdf*(dx*dx + dy*dy + dz*dz);
-            inside += ssqd < (float) rsq;
-            float w0, wom, wz;
-            kdens<float>(p.kern, ssqd, w0, wom, wz);
-            br += c.w*w0;
-            bom += c.w*invhf*wom;
-            bz += c.w*wz;
-          }
-          kr.add(br); kom.add(bom); kz.add(bz);
-        }
+      r_ = om_ = z_ = 0.0;
+      for (int w = 0; w < W; w++) {
+        r_ += red[w][0][lane]; om_ += red[w][1][lane]; z_ += red[w][2][lane];
       }
       __syncthreads();
     }
-    first = false;
     if (run) {
-      double rho, invomega, zeta;
-      if (sizeof(T) == 8) { rho = r_; invomega = om_; zeta = z_; }
-      else { rho = (double) kr.s; invomega = (double) kom.s; zeta = (double) kz.s; }
-      rho *= hfac3;
-      invomega *= hfac3;
-      zeta *= invhsqd;
+      const double hfac3 = invh*invhsqd;
+      DensSums<T, KT>::finish(p.kern, r_, om_, z_);
+      const double rho = r_*hfac3, invomega = om_*invh*hfac3, zeta = z_*invhsqd;
       const int rc = hrho_step(p, m, hmax, iteration, rho, h, h_lower, h_upper);
       if (rc == 1) {
         // converged: the sums and the bracket go to k_hrho_finish (status 2), which keeps
         // the final h, grad-h terms and EOS out of this kernel's register budget
-        a.rho[i] = rho; a.invomega[i] = invomega; a.zeta[i] = zeta; a.hfactor[i] = h_lower;
-        a.status[i] = 2;
+        if (wv == 0) {
+          a.rho[i] = rho; a.invomega[i] = invomega; a.zeta[i] = zeta; a.hfactor[i] = h_lower;
+          a.status[i] = 2;
+        }
         ngather = inside;
         state = 1;
       } else if (rc == 0) {
-        a.hsearch[i] = hmax*1.05;       // GradhSphTree.cpp:154: hmax = 1.05 hmax per retry
-        atomicAdd(&a.flags[0], 1);
+        if (wv == 0) {
+          a.hsearch[i] = hmax*1.05;     // GradhSphTree.cpp:154: hmax = 1.05 hmax per retry
+          atomicAdd(&a.flags[0], 1);
+        }
         state = 0;
       } else if (rc < 0) {
-        a.status[i] = 0;
-        atomicOr(&a.flags[3], 1);
+        if (wv == 0) {
+          a.status[i] = 0;
+          atomicOr(&a.flags[3], 1);
+        }
         state = -1;
       }
     }
   }
   wave_add_ll(&a.icount[0], ngather);
   wave_add_ll(&a.icount[4], evals);
+}
+
+template <typename T, int KT>
+void launch_density_k(const DensArgs& d, int waves, hipStream_t s) {
+  if (waves == 4) k_density<T, KT, 4><<<d.ngroups, 4*kWave, 0, s>>>(d);
+  else k_density<T, KT, 1><<<d.ngroups, kWave, 0, s>>>(d);
+}
+
+template <typename T>
+void launch_density(const DensArgs& d, int waves, hipStream_t s) {
+  if (d.p.kern.tabulated) launch_density_k<T, 2>(d, waves, s);
+  else if (d.p.kern.type == 0) launch_density_k<T, 0>(d, waves, s);
+  else launch_density_k<T, 1>(d, waves, s);
 }
 
 // Final h, grad-h terms and EOS of the particles the h-rho pass has just converged (status 2:
@@ -524,10 +540,11 @@ __global__ void k_pack_hydro(int N, const double* __restrict__ vx, const double*
 
 struct HydroArgs {
   int N, ngroups, capb;
-  const int* grp_node; const int* grp_first; const int* grp_count; const double4* geo_c;
-  const int* idx; const unsigned long long* mask; const int* ncand;
+  const int* grp_node; const int* grp_first; const int* grp_count;
+  const double4* geo_c; const double4* geo_h;
+  const int* idx; const int* ncand;
   const double4* posm; const double4* A; const double4* B;
-  const double* h;                  // smoothing lengths, for the fused scatter-gather tests
+  const double* h;
   const double* invomega; const double* pressure; const double* zeta;
   double* ax; double* ay; double* az; double* dudt; double* div_v;
   double* gx; double* gy; double* gz; double* gpot;    // softened neighbour gravity (VAR 1)
@@ -546,255 +563,269 @@ __device__ __forceinline__ int blk_record(const HydroArgs& a, int j) {
   return a.level[j] | ((a.act[j] ? 255 : a.levelneib[j]) << 8);
 }
 
+// The nine sums of a hydro pass
+template <typename T> struct HydroSums {
+  T ax = T(0), ay = T(0), az = T(0), du = T(0), dv = T(0);
+  T gx = T(0), gy = T(0), gz = T(0), gp = T(0);
+  template <typename U> __device__ __forceinline__ void add(const HydroSums<U>& o) {
+    ax += (T) o.ax; ay += (T) o.ay; az += (T) o.az; du += (T) o.du; dv += (T) o.dv;
+    gx += (T) o.gx; gy += (T) o.gy; gz += (T) o.gz; gp += (T) o.gp;
+  }
+  template <typename U> __device__ __forceinline__ void to(HydroSums<U>& o) const {
+    o.ax = (U) ax; o.ay = (U) ay; o.az = (U) az; o.du = (U) du; o.dv = (U) dv;
+    o.gx = (U) gx; o.gy = (U) gy; o.gz = (U) gz; o.gp = (U) gp;
+  }
+};
+
+template <typename T> struct Vec4 { T x, y, z, w; };
+// A wavefront's staged candidates of the hydro passes: position and mass, velocity and 1/h,
+// (1/rho, P Omega^-1/rho^2, c_s, hfactor), zeta, the squared range, and a block step's particle
+// and level record
+template <typename T, int VAR, bool BLK> struct HydroStage {
+  Vec4<T> P[kPairSlots], V[kPairSlots], B[kPairSlots];
+  T Z[VAR == 1 ? kPairSlots : 1], R[kPairSlots];
+  int J[BLK ? kPairSlots : 1], L[BLK ? kPairSlots : 1];
+};
+
 // VAR 0: ComputeSphHydroForces (GradhSph.cpp:361-460); VAR 1: ComputeSphHydroGravForces
 // (:474-585), the hydro terms plus the kernel-softened gravity of the pair (into gx, gy, gz,
-// gpot; the tree walk adds the direct and multipole terms afterwards).  FP64, one walk group
-// per workgroup, neighbour records staged in LDS per batch of 64 candidates.
-template <int VAR, bool BLK>
-__global__ __launch_bounds__(64) void k_hydro(HydroArgs a) {
-  __shared__ double4 sP[kWave], sA[kWave], sB[kWave];
-  __shared__ double sZ[kWave];
+// gpot; the tree walk adds the direct and multipole terms afterwards).  One walk group per
+// workgroup, its W wavefronts sharing the candidates.  T = double: FP64
+// throughout, separations target by target.  T = float: records in FP32 in the group's frame
+// (positions relative to its centre, velocities to its first particle), pair terms in FP32 summed
+// batch by batch, FP64 totals.  A hit of the filter is a pair if the path's own test says so, the
+// one its gravity walk masks with.
+// Bound by vector issue (1M particles, quintic: 0.27 VALU instructions a cycle and SIMD in FP32,
+// 0.18 in FP64); the launch bounds are the most wavefronts a SIMD without spills (one more cost
+// 24 % in FP32).  1M, quintic, with gravity, alone on the device: 2.02 ms against 2.25 (FP32) and
+// 3.45 against 5.06 (FP64) with masks.
+template <typename T, int KT, int VAR, bool BLK, int W>
+__global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArgs a) {
+  constexpr bool F64 = sizeof(T) == 8;
+  constexpr int NS = VAR == 1 ? 9 : 5;
+  __shared__ HydroStage<T, VAR, BLK> stage[W];
   const int g = xcd_block(blockIdx.x, gridDim.x);
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & (kWave - 1), wv = W == 1 ? 0 : (int) threadIdx.x/kWave;
   const int nc = a.ncand[g];
+  if (nc <= 0) return;                        // no target in this group
   const int gfirst = a.grp_first[g], gcnt = a.grp_count[g];
+  HydroStage<T, VAR, BLK>& st = stage[wv];
   const int i = gfirst + lane;
-  const bool has = lane < gcnt && (!BLK || a.act[gfirst + lane]);
-  __shared__ int sJ[kWave], sL[kWave];
-  int lmax = 0;
-  const int level_i = (BLK && has) ? a.level[i] : 0;
+  const bool has = lane < gcnt && (!BLK || a.act[i] != 0);
   const PhysParams& p = a.p;
-  double4 me = make_double4(0.0, 0.0, 0.0, 1.0), mA = make_double4(0.0, 0.0, 0.0, 1.0);
-  double4 mB = make_double4(1.0, 0.0, 0.0, 0.0);
-  double zeta_i = 0.0;
-  if (has) {
-    me = a.posm[i]; mA = a.A[i]; mB = a.B[i];
-    if (VAR == 1) zeta_i = a.zeta[i];
-  }
-  const double invh_i = mA.w, invrho_i = mB.x;
-  const double pterm_i = mB.y, snd_i = mB.z, hf_i = mB.w;
-  const double alpha = p.alpha_visc, beta = p.beta_visc;
-  const double invhsqd_i = invh_i*invh_i;
-  double ax = 0, ay = 0, az = 0, du = 0, dv = 0;
-  double gx = 0, gy = 0, gz = 0, gp = 0;
-  long long npairs = 0;
-  const int nbat = (nc + kWave - 1)/kWave;
-  const int* idx = a.idx + (size_t) g*a.capb*kWave;
-  const unsigned long long* msk = a.mask + (size_t) g*a.capb*kWave;
-  for (int b = 0; b < nbat; b++) {
-    const int nb = (nc - b + nbat - 1)/nbat;   // candidates b, b + nbat, ...
-    if (lane < nb) {
-      const int j = idx[b + lane*nbat];
-      sP[lane] = a.posm[j]; sA[lane] = a.A[j]; sB[lane] = a.B[j];
-      if (VAR == 1) sZ[lane] = a.zeta[j];
-      if (BLK) { sJ[lane] = j; sL[lane] = blk_record(a, j); }
-    }
-    __syncthreads();
-    if (has) {
-      unsigned long long mk = msk[b*kWave + lane];
-      npairs += __popcll(mk);
-      while (mk) {
-        const int q = __builtin_ctzll(mk);
-        mk &= mk - 1;
-        if (BLK) {
-          const int lj = sL[q];
-          lmax = max(lmax, lj & 255);
-          if (level_i > (lj >> 8)) atomicMax(&a.levelneib[sJ[q]], level_i);
-        }
-        const double4 pj = sP[q], Aj = sA[q], Bj = sB[q];
-        double dx = pj.x - me.x, dy = pj.y - me.y, dz = pj.z - me.z;
-        nearest_image<double>(p, dx, dy, dz);
-        const double mj = pj.w;
-        const double invh_j = Aj.w, invrho_j = Bj.x;
-        double drmag, dvdr;
-        if (VAR == 0) {
-          drmag = sqrt(dx*dx + dy*dy + dz*dz);
-          if (drmag > 0.0) { dx /= drmag; dy /= drmag; dz /= drmag; }
-        } else {
-          drmag = sqrt(dx*dx + dy*dy + dz*dz + 1.0e-20);
-          const double inv = 1.0/drmag;
-          dx *= inv; dy *= inv; dz *= inv;
-        }
-        const double si = drmag*invh_i, sj = drmag*invh_j;
-        const double wkerni = hf_i*kw1<double>(p.kern, si);
-        const double wkernj = Bj.w*kw1<double>(p.kern, sj);
-        if (VAR == 0) {
-          dvdr = Aj.x*dx + Aj.y*dy + Aj.z*dz;
-          dvdr -= mA.x*dx + mA.y*dy + mA.z*dz;
-          dv -= mj*dvdr*wkerni;
-        } else {
-          const double dvx = Aj.x - mA.x, dvy = Aj.y - mA.y, dvz = Aj.z - mA.z;
-          dvdr = dvx*dx + dvy*dy + dvz*dz;
-        }
-        double paux = pterm_i*wkerni + Bj.y*wkernj;
-        if (dvdr < 0.0) {
-          const double winvrho = 0.25*(wkerni + wkernj)*(invrho_i + invrho_j);
-          const double vsignal = snd_i + Bj.z - beta*alpha*dvdr;
-          paux -= alpha*vsignal*dvdr*winvrho;
-          du -= 0.5*mj*alpha*vsignal*dvdr*dvdr*winvrho;
-        }
-        ax += mj*dx*paux; ay += mj*dy*paux; az += mj*dz*paux;
-        if (VAR == 1) {
-          const double pg = 0.5*(invhsqd_i*kwgrav<double>(p.kern, si) + zeta_i*wkerni +
-                                 invh_j*invh_j*kwgrav<double>(p.kern, sj) + sZ[q]*wkernj);
-          gx += mj*dx*pg; gy += mj*dy*pg; gz += mj*dz*pg;
-          gp += 0.5*mj*(invh_i*kwpot<double>(p.kern, si) + invh_j*kwpot<double>(p.kern, sj));
-          dv -= mj*dvdr*wkerni;
-        }
-      }
-    }
-    __syncthreads();
-  }
-  wave_add_ll(&a.icount[1], npairs);
-  if (!has) return;
-  if (BLK) a.levelneib[i] = lmax;
-  const double dvd = dv*mB.x;
-  const double dud = du - a.pressure[i]*dvd*mB.x*a.invomega[i];
-  a.ax[i] = ax; a.ay[i] = ay; a.az[i] = az;
-  a.dudt[i] = dud; a.div_v[i] = dvd;
-  if (VAR == 1) { a.gx[i] = gx; a.gy[i] = gy; a.gz[i] = gz; a.gpot[i] = gp; }
-}
-
-// FP32 variant: records staged in LDS in the group frame (positions relative to the group
-// centre, velocities relative to the group's first particle), pair terms in FP32 with the
-// hardware reciprocal and square root, per-batch register sums, Kahan-compensated totals.
-// (at most 96 VGPRs: five wavefronts per SIMD instead of four, a few registers spilled)
-// FUSED: the candidate walk recorded no masks; each staged batch is tested against both
-// smoothing ranges exactly as the walk's MODE 2 would, giving the same scatter-gather set.
-template <int VAR, bool BLK, bool FUSED = false>
-__global__ __launch_bounds__(64, 5) void k_hydro_mixed(HydroArgs a) {
-  __shared__ float4 fP[kWave], fV[kWave], fB[kWave];
-  __shared__ float fZ[kWave], fR[kWave];
-  const int g = xcd_block(blockIdx.x, gridDim.x);
-  const int lane = threadIdx.x;
-  const int nc = a.ncand[g];
-  const int gfirst = a.grp_first[g], gcnt = a.grp_count[g];
-  const int i = gfirst + lane;
-  const bool has = lane < gcnt && (!BLK || a.act[gfirst + lane]);
-  __shared__ int sJ[kWave], sL[kWave];
-  int lmax = 0;
-  const int level_i = (BLK && has) ? a.level[i] : 0;
-  const PhysParams& p = a.p;
-  const double4 gc = a.geo_c[a.grp_node[g]];
-  const double4 vref = a.A[gfirst];
-  double4 me = make_double4(0.0, 0.0, 0.0, 1.0), mA = make_double4(0.0, 0.0, 0.0, 1.0);
-  double4 mB = make_double4(1.0, 0.0, 0.0, 0.0);
-  float zeta_i = 0.f;
-  if (has) {
-    me = a.posm[i]; mA = a.A[i]; mB = a.B[i];
-    if (VAR == 1) zeta_i = (float) a.zeta[i];
-  }
-  const float rxi = (float) (me.x - gc.x), ryi = (float) (me.y - gc.y), rzi = (float) (me.z - gc.z);
-  const float vxi = (float) (mA.x - vref.x), vyi = (float) (mA.y - vref.y), vzi = (float) (mA.z - vref.z);
-  const float invh_i = (float) mA.w;
-  const float invrho_i = (float) mB.x;
-  const float pterm_i = (float) mB.y, snd_i = (float) mB.z, hf_i = (float) mB.w;
-  const float alpha = (float) p.alpha_visc, beta = (float) p.beta_visc;
-  const float invhsqd_i = invh_i*invh_i;
   const double krsqd = p.kern.rangesqd;
-  const float r2if = (FUSED && has) ? (float) range2_rn(krsqd, a.h[i]) : 0.f;
-  KahanF ax, ay, az, du, dv, gx, gy, gz, gp;
-  long long npairs = 0, ntests = 0;
-  const int nbat = (nc + kWave - 1)/kWave;
-  const int* idx = a.idx + (size_t) g*a.capb*kWave;
-  const unsigned long long* msk = a.mask + (size_t) g*a.capb*kWave;
-  for (int b = 0; b < nbat; b++) {
-    const int nb = (nc - b + nbat - 1)/nbat;   // candidates b, b + nbat, ...
-    if (FUSED && has) ntests += nb;
-    if (lane < nb) {
-      const int j = idx[b + lane*nbat];
+  const double4 gc = a.geo_c[a.grp_node[g]], gh = a.geo_h[a.grp_node[g]];
+  const double4 vref = a.A[gfirst];
+  int lmax = 0, npairs = 0;
+  const int level_i = BLK && has ? a.level[i] : 0;
+  double4 me = make_double4(gc.x, gc.y, gc.z, 1.0), mA = make_double4(vref.x, vref.y, vref.z, 1.0);
+  double4 mB = make_double4(1.0, 0.0, 0.0, 0.0);
+  T zeta_i = T(0), r2i = T(-1);
+  double h_i = 0.0;
+  if (has) {
+    me = a.posm[i]; mA = a.A[i]; mB = a.B[i];
+    if (VAR == 1) zeta_i = (T) a.zeta[i];
+    h_i = a.h[i];
+    r2i = (T) range2_rn(krsqd, h_i);
+  }
+  const float rxf = (float) (me.x - gc.x), ryf = (float) (me.y - gc.y), rzf = (float) (me.z - gc.z);
+  const T rxi = F64 ? (T) me.x : (T) rxf, ryi = F64 ? (T) me.y : (T) ryf, rzi = F64 ? (T) me.z : (T) rzf;
+  const T vxi = F64 ? (T) mA.x : (T) (mA.x - vref.x), vyi = F64 ? (T) mA.y : (T) (mA.y - vref.y),
+          vzi = F64 ? (T) mA.z : (T) (mA.z - vref.z);
+  const T invh_i = (T) mA.w, invrho_i = (T) mB.x, pterm_i = (T) mB.y, snd_i = (T) mB.z;
+  const T hf_i = (T) (mB.w*HydroKern<T, KT>::w1_factor(p.kern));
+  const T alpha = (T) p.alpha_visc, beta = (T) p.beta_visc;
+  // the filter's frame: the group's half-diagonal plus the targets' largest range below one
+  const double rG = p.kern.range*wave_max_d(h_i);
+  const double diag = sqrt(gh.x*gh.x + gh.y*gh.y + gh.z*gh.z);
+  const float fs = filter_scale(diag + rG);
+  FiltTargets ft;
+  ft.position(rxf*fs, ryf*fs, rzf*fs);
+  ft.range(rxf*fs, ryf*fs, rzf*fs, has ? (float) ((double) r2i*fs*fs) : -1.f);
+  HydroSums<double> sum;
+  const PairBatches pb((nc - wv + W - 1)/W);
+  const int* idx = a.idx + (size_t) g*a.capb*kWave + wv;
+  const double w1f = HydroKern<T, KT>::w1_factor(p.kern);
+  HitQueue hq;
+  int rec = 0;
+  int jn = pb.filled(0, lane) ? idx[pb.index(0, lane)*W] : -1;
+  for (int b = 0; b < pb.nb; b++) {
+    const int s0 = kWave*(b & 1);
+    if (jn >= 0) {
+      const int j = jn, s = s0 + lane;
       const double4 pj = a.posm[j], Aj = a.A[j], Bj = a.B[j];
-      double dx = pj.x - gc.x, dy = pj.y - gc.y, dz = pj.z - gc.z;
-      nearest_image<double>(p, dx, dy, dz);
-      fP[lane] = make_float4((float) dx, (float) dy, (float) dz, (float) pj.w);
-      fV[lane] = make_float4((float) (Aj.x - vref.x), (float) (Aj.y - vref.y),
-                             (float) (Aj.z - vref.z), (float) Aj.w);
-      fB[lane] = make_float4((float) Bj.x, (float) Bj.y, (float) Bj.z, (float) Bj.w);
-      if (VAR == 1) fZ[lane] = (float) a.zeta[j];
-      if (FUSED) fR[lane] = (float) range2_rn(krsqd, a.h[j]);
-      if (BLK) { sJ[lane] = j; sL[lane] = blk_record(a, j); }
-    }
-    __syncthreads();
-    if (has) {
-      unsigned long long mk;
-      if (FUSED) {
-        mk = 0;
-        #pragma unroll 8
-        for (int q = 0; q < kWave; q++) {
-          const float4 c = fP[q];
-          const float d2 = dot3_f(c.x - rxi, c.y - ryi, c.z - rzi);
-          mk |= (unsigned long long) ((d2 < r2if) | (d2 < fR[q])) << q;
-        }
-        if (nb < kWave) mk &= (1ULL << nb) - 1ULL;
+      if (F64) {
+        st.P[s] = {(T) pj.x, (T) pj.y, (T) pj.z, (T) pj.w};
+        st.V[s] = {(T) Aj.x, (T) Aj.y, (T) Aj.z, (T) Aj.w};
       } else {
-        mk = msk[b*kWave + lane];
+        double dx = pj.x - gc.x, dy = pj.y - gc.y, dz = pj.z - gc.z;
+        nearest_image<double>(p, dx, dy, dz);
+        st.P[s] = {(T) dx, (T) dy, (T) dz, (T) pj.w};
+        st.V[s] = {(T) (Aj.x - vref.x), (T) (Aj.y - vref.y), (T) (Aj.z - vref.z), (T) Aj.w};
       }
-      npairs += __popcll(mk);
-      float bax = 0.f, bay = 0.f, baz = 0.f, bdu = 0.f, bdv = 0.f;
-      float bgx = 0.f, bgy = 0.f, bgz = 0.f, bgp = 0.f;
-      while (mk) {
-        const int q = __builtin_ctzll(mk);
-        mk &= mk - 1;
-        if (BLK) {
-          const int lj = sL[q];
-          lmax = max(lmax, lj & 255);
-          if (level_i > (lj >> 8)) atomicMax(&a.levelneib[sJ[q]], level_i);
-        }
-        const float4 P = fP[q], V = fV[q], B = fB[q];
-        float dx = P.x - rxi, dy = P.y - ryi, dz = P.z - rzi;
-        const float mj = P.w;
-        const float invh_j = V.w;
-        const float invrho_j = B.x;
-        float drmag;
-        if (VAR == 0) {
-          drmag = sqrt_f(dx*dx + dy*dy + dz*dz);
-          if (drmag > 0.f) { const float inv = rcp_f(drmag); dx *= inv; dy *= inv; dz *= inv; }
-        } else {
-          drmag = sqrt_f(dx*dx + dy*dy + dz*dz + 1.0e-20f);
-          const float inv = rcp_f(drmag);
-          dx *= inv; dy *= inv; dz *= inv;
-        }
-        const float si = drmag*invh_i, sj = drmag*invh_j;
-        const float wkerni = hf_i*kw1<float>(p.kern, si);
-        const float wkernj = B.w*kw1<float>(p.kern, sj);
-        const float dvx = V.x - vxi, dvy = V.y - vyi, dvz = V.z - vzi;
-        const float dvdr = dvx*dx + dvy*dy + dvz*dz;
-        bdv -= mj*dvdr*wkerni;
-        float paux = pterm_i*wkerni + B.y*wkernj;
-        if (dvdr < 0.f) {
-          const float winvrho = 0.25f*(wkerni + wkernj)*(invrho_i + invrho_j);
-          const float vsignal = snd_i + B.z - beta*alpha*dvdr;
-          paux -= alpha*vsignal*dvdr*winvrho;
-          bdu -= 0.5f*mj*alpha*vsignal*dvdr*dvdr*winvrho;
-        }
-        bax += mj*dx*paux; bay += mj*dy*paux; baz += mj*dz*paux;
-        if (VAR == 1) {
-          float wgi, wpi, wgj, wpj;
-          kgravpot_f(p.kern, si, rcp_f(si), wgi, wpi);
-          kgravpot_f(p.kern, sj, rcp_f(sj), wgj, wpj);
-          const float pg = 0.5f*(invhsqd_i*wgi + zeta_i*wkerni + invh_j*invh_j*wgj +
-                                 fZ[q]*wkernj);
-          bgx += mj*dx*pg; bgy += mj*dy*pg; bgz += mj*dz*pg;
-          bgp += 0.5f*mj*(invh_i*wpi + invh_j*wpj);
-        }
-      }
-      ax.add(bax); ay.add(bay); az.add(baz); du.add(bdu); dv.add(bdv);
-      if (VAR == 1) { gx.add(bgx); gy.add(bgy); gz.add(bgz); gp.add(bgp); }
+      st.B[s] = {(T) Bj.x, (T) Bj.y, (T) Bj.z, (T) (Bj.w*w1f)};
+      if (VAR == 1) st.Z[s] = (T) a.zeta[j];
+      st.R[s] = (T) range2_rn(krsqd, a.h[j]);
+      if (BLK) { st.J[s] = j; st.L[s] = blk_record(a, j); }
     }
-    __syncthreads();
+    jn = pb.filled(b + 1, lane) ? idx[pb.index(b + 1, lane)*W] : -1;
+    wave_lds_order();
+    const uint2 hit = filter64<true>(ft, [&](int l) {
+      FiltCand f = {0.f, 0.f, 0.f, 0.f, 1};
+      if (!pb.filled(b, l)) return f;
+      const Vec4<T> r = st.P[s0 + l];
+      const T r2 = st.R[s0 + l];
+      f.state = 0;
+      if (F64) {
+        double dx = r.x - gc.x, dy = r.y - gc.y, dz = r.z - gc.z;
+        nearest_image<double>(p, dx, dy, dz);
+        f.x = (float) dx; f.y = (float) dy; f.z = (float) dz;
+        if (p.periodic) {
+          // taken unless its image about the centre is its image about every target in range
+          const double R = fmax(rG, sqrt((double) r2));
+          if (gh.x + R >= p.boxhalf[0] || gh.y + R >= p.boxhalf[1] || gh.z + R >= p.boxhalf[2])
+            f.state = -1;
+        }
+      } else {
+        f.x = (float) r.x; f.y = (float) r.y; f.z = (float) r.z;
+      }
+      f.x *= fs; f.y *= fs; f.z *= fs;
+      f.thr = filter_thr((float) ((double) r2*fs*fs));
+      return f;
+    });
+    hq.stage(b == 0, has ? hit : make_uint2(0u, 0u));
+    const int need = b + 1 < pb.nb ? hq.older : hq.staged;
+    HydroSums<T> part;
+    if (F64) sum.to(part);
+    hq.run(need, rec, [&](int q) { return q; }, [&](int q, bool take) {
+      const Vec4<T> P = st.P[q], V = st.V[q], B = st.B[q];
+      T dx = P.x - rxi, dy = P.y - ryi, dz = P.z - rzi;
+      if (F64) nearest_image<T>(p, dx, dy, dz);
+      const T d2 = dot3_t(dx, dy, dz);
+      const bool in = take & ((d2 < r2i) | (d2 < st.R[q]));
+      const T mj = in ? P.w : T(0);
+      npairs += in;
+      if (BLK) {
+        const int lj = st.L[q];
+        if (in) lmax = max(lmax, lj & 255);
+        if (in && level_i > (lj >> 8)) atomicMax(&a.levelneib[st.J[q]], level_i);
+      }
+      // unit separation; the particle itself has none
+      const T tiny = F64 ? T(1.0e-280) : T(1.0e-36);
+      const T d2e = VAR == 1 ? d2 + T(1.0e-20) : (d2 > tiny ? d2 : tiny);
+      const T inv = rsq_t(d2e);
+      const T drmag = d2e*inv;
+      dx *= inv; dy *= inv; dz *= inv;
+      const T invh_j = V.w;
+      HydroKern<T, KT> ki, kj;
+      ki.set(p.kern, drmag*invh_i);
+      kj.set(p.kern, drmag*invh_j);
+      const T wkerni = hf_i*ki.w1, wkernj = B.w*kj.w1;
+      const T dvdr = (V.x - vxi)*dx + (V.y - vyi)*dy + (V.z - vzi)*dz;
+      part.dv -= mj*dvdr*wkerni;
+      T paux = pterm_i*wkerni + B.y*wkernj;
+      if (dvdr < T(0)) {
+        const T winvrho = T(0.25)*(wkerni + wkernj)*(invrho_i + B.x);
+        const T q2 = alpha*(snd_i + B.z - beta*alpha*dvdr)*dvdr*winvrho;
+        paux -= q2;
+        part.du -= T(0.5)*mj*q2*dvdr;
+      }
+      const T ma = mj*paux;
+      part.ax += ma*dx; part.ay += ma*dy; part.az += ma*dz;
+      if (VAR == 1) {
+        T mi, poti, mjj, potj;
+        ki.grav(p.kern, mi, poti);
+        kj.grav(p.kern, mjj, potj);
+        // wgrav/h^2 = M/d^2 and wpot/h = M/d + P/h (enclosed mass M, outer integral P); the
+        // factor 1/2 of the pair mean is applied to the sums
+        const T M = mi + mjj;
+        const T mg = mj*(M*(inv*inv) + zeta_i*wkerni + st.Z[q]*wkernj);
+        part.gx += mg*dx; part.gy += mg*dy; part.gz += mg*dz;
+        part.gp += mj*(M*inv + (invh_i*poti + invh_j*potj));
+      }
+    });
+    if (F64) part.to(sum);
+    else sum.add(part);
+    wave_lds_order();
+  }
+  if (W > 1) {
+    // the wavefronts' sums, added in order by the first
+    double v[NS] = {sum.ax, sum.ay, sum.az, sum.du, sum.dv};
+    if (VAR == 1) { v[NS - 4] = sum.gx; v[NS - 3] = sum.gy; v[NS - 2] = sum.gz; v[NS - 1] = sum.gp; }
+    static_assert(sizeof(stage) >= sizeof(double)*64*W, "a row of sums per wavefront");
+    double* red = reinterpret_cast<double*>(&stage[0]);     // one sum at a time
+    for (int k = 0; k < NS; k++) {
+      __syncthreads();
+      red[threadIdx.x] = v[k];
+      __syncthreads();
+      if (wv == 0)
+        for (int w = 1; w < W; w++) v[k] += red[w*kWave + lane];
+    }
+    sum.ax = v[0]; sum.ay = v[1]; sum.az = v[2]; sum.du = v[3]; sum.dv = v[4];
+    if (VAR == 1) { sum.gx = v[NS - 4]; sum.gy = v[NS - 3]; sum.gz = v[NS - 2]; sum.gp = v[NS - 1]; }
+    if (BLK) {
+      int* ri = reinterpret_cast<int*>(&stage[0]);
+      __syncthreads();
+      ri[threadIdx.x] = lmax;
+      __syncthreads();
+      if (wv == 0)
+        for (int w = 1; w < W; w++) lmax = max(lmax, ri[w*kWave + lane]);
+    }
   }
   wave_add_ll(&a.icount[1], npairs);
-  if (FUSED) wave_add_ll(&a.icount[5], ntests);
-  if (!has) return;
+  // the filter's candidate-target tests (counted for the mixed path)
+  if (!F64) wave_add_ll(&a.icount[5], has && wv == 0 ? nc : 0);
+  if (!has || wv != 0) return;
   if (BLK) a.levelneib[i] = lmax;
-  const double dvd = (double) dv.s*mB.x;
-  const double dud = (double) du.s - a.pressure[i]*dvd*mB.x*a.invomega[i];
-  a.ax[i] = (double) ax.s; a.ay[i] = (double) ay.s; a.az[i] = (double) az.s;
+  const double dvd = sum.dv*mB.x;
+  const double dud = sum.du - a.pressure[i]*dvd*mB.x*a.invomega[i];
+  a.ax[i] = sum.ax; a.ay[i] = sum.ay; a.az[i] = sum.az;
   a.dudt[i] = dud; a.div_v[i] = dvd;
   if (VAR == 1) {
-    a.gx[i] = (double) gx.s; a.gy[i] = (double) gy.s; a.gz[i] = (double) gz.s;
-    a.gpot[i] = (double) gp.s;
+    a.gx[i] = 0.5*sum.gx; a.gy[i] = 0.5*sum.gy; a.gz[i] = 0.5*sum.gz;
+    a.gpot[i] = 0.5*sum.gp;
   }
+}
+
+template <typename T, int KT, int W>
+void launch_hydro_w(const HydroArgs& h, int variant, bool blk, hipStream_t s) {
+  const int grid = h.ngroups;
+  if (variant == 0) {
+    if (blk) k_hydro<T, KT, 0, true, W><<<grid, W*kWave, 0, s>>>(h);
+    else k_hydro<T, KT, 0, false, W><<<grid, W*kWave, 0, s>>>(h);
+  } else {
+    if (blk) k_hydro<T, KT, 1, true, W><<<grid, W*kWave, 0, s>>>(h);
+    else k_hydro<T, KT, 1, false, W><<<grid, W*kWave, 0, s>>>(h);
+  }
+}
+
+template <typename T, int KT>
+void launch_hydro_k(const HydroArgs& h, int variant, bool blk, int waves, hipStream_t s) {
+  if (waves == 4) launch_hydro_w<T, KT, 4>(h, variant, blk, s);
+  else if (waves == 2) launch_hydro_w<T, KT, 2>(h, variant, blk, s);
+  else launch_hydro_w<T, KT, 1>(h, variant, blk, s);
+}
+
+template <typename T>
+void launch_hydro(const HydroArgs& h, int variant, bool blk, int waves, hipStream_t s) {
+  if (h.p.kern.tabulated) launch_hydro_k<T, 2>(h, variant, blk, waves, s);
+  else if (h.p.kern.type == 0) launch_hydro_k<T, 0>(h, variant, blk, waves, s);
+  else launch_hydro_k<T, 1>(h, variant, blk, waves, s);
+}
+
+// Wavefronts that share a walk group's candidates in the pair passes.  A group's pass is a chain
+// of dependent loads, sums and reductions, so while one wavefront a group leaves most of the 1024
+// SIMDs idle more of them finish sooner; once the device is full every further wavefront only
+// adds partly filled batches and, in the h-rho pass, barriers between sweeps.  Times (us) with 1,
+// 2 and 4 wavefronts, by groups (FP64 below 2048, FP32 from there on):
+//   groups      128          512          1024          2048          4096
+//   h-rho    36 24 20     46 43 61     91  89 133    164 183 257   198 319 589
+//   hydro    48 32 22     94 63 70    159 153 177    575 474 456   547 560 668
+// A serving batch keeps to one: a request's sums must not depend on what else is resident.
+int density_waves(const gdf_ctx* c) { return c->ngroups <= 256 && c->nseg == 0 ? 4 : 1; }
+int hydro_waves(const gdf_ctx* c) {
+  if (c->nseg > 0 || c->ngroups > 2048) return 1;
+  return c->ngroups <= 256 ? 4 : 2;
 }
 
 int read_flags(gdf_ctx* c) {
@@ -812,15 +843,16 @@ void free_cand(CandSet& cs) {
   cs.capb = 0; cs.gcap = 0;
 }
 
-// (Re)allocate a candidate set for at least the current number of groups and capb batches.
-int alloc_cand(gdf_ctx* c, CandSet& cs, int capb) {
-  const int gcap = std::max(cs.gcap, c->ngroups + c->ngroups/4 + 64);
-  if (cs.idx && gcap == cs.gcap && capb == cs.capb) return GDF_OK;
+// (Re)allocate a candidate set for at least ng groups and capb batches; masks: with room for
+// the parity tap's masks.
+int alloc_cand(gdf_ctx* c, CandSet& cs, int ng, int capb, bool masks) {
+  const int gcap = ng <= cs.gcap ? cs.gcap : ng + ng/4 + 64;
+  if (cs.idx && gcap == cs.gcap && capb == cs.capb && (cs.mask || !masks)) return GDF_OK;
   GDF_HIP(c, hipStreamSynchronize(c->stream));
   free_cand(cs);
   const size_t n = (size_t) gcap*(size_t) capb*kWave;
   if (hipMalloc(&cs.idx, sizeof(int)*n) != hipSuccess ||
-      hipMalloc(&cs.mask, sizeof(unsigned long long)*n) != hipSuccess ||
+      (masks && hipMalloc(&cs.mask, sizeof(unsigned long long)*n) != hipSuccess) ||
       hipMalloc(&cs.ncand, sizeof(int)*(size_t) gcap) != hipSuccess) {
     free_cand(cs);
     return fail(c, GDF_ERR_NOMEM, "candidate set allocation failed");
@@ -830,31 +862,33 @@ int alloc_cand(gdf_ctx* c, CandSet& cs, int capb) {
   return GDF_OK;
 }
 
-int ensure_cand(gdf_ctx* c, CandSet& cs) {
-  if (cs.idx && c->ngroups <= cs.gcap) return GDF_OK;
-  return alloc_cand(c, cs, cs.capb > 0 ? cs.capb
-                            : (c->cfg.cand_batches_init > 0 ? c->cfg.cand_batches_init
-                                                            : kInitBatches));
+int ensure_cand(gdf_ctx* c, CandSet& cs, int ng, bool masks) {
+  const int capb = cs.capb > 0 ? cs.capb : c->cfg.cand_batches_init > 0 ? c->cfg.cand_batches_init
+                                                                       : kInitBatches;
+  return alloc_cand(c, cs, ng, capb, masks);
 }
 
-int grow_cand(gdf_ctx* c, CandSet& cs, int need) {
-  return alloc_cand(c, cs, std::max(need + need/4 + 1, cs.capb + 1));
+int grow_cand(gdf_ctx* c, CandSet& cs, int ng, int need, bool masks) {
+  return alloc_cand(c, cs, ng, std::max(need + need/4 + 1, cs.capb + 1), masks);
 }
+
+// The candidate walks of the h-rho pass (gather; uni: with the scatter-gather bounds) and of the
+// force pass (scatter-gather); masks: the parity tap's sets.
+enum WalkKind { WALK_GATHER, WALK_UNION, WALK_SG, WALK_MASKS };
 
 // glist: the groups holding targets (from group_list), or NULL to walk every group
 // (the walk's queue counters, counters[4, 12), must be zero: the list builder clears them)
-// masks = false (mixed path): the FP32 walks record candidates only (the pair pass tests them);
-// uni: the mixed gather walk's union lists (gather and scatter-gather candidates)
-int launch_walk(gdf_ctx* c, int mode, int nopbc, CandSet& cs, const int* status,
-                const int* glist, bool masks, bool uni = false) {
+int launch_walk(gdf_ctx* c, WalkKind kind, int nopbc, CandSet& cs, const int* status,
+                const int* glist) {
   CandWalk w;
-  w.N = c->N; w.ngroups = c->ngroups; w.nleaf = c->phys.nleaf; w.capb = cs.capb;
+  const int ng = c->ngroups;
+  w.N = c->N; w.ngroups = ng; w.nleaf = c->phys.nleaf; w.capb = cs.capb;
   w.grp_node = c->grp_node; w.grp_first = c->grp_first; w.grp_count = c->grp_count;
   w.lnk = c->lnk;
   w.geo_c = c->geo_c; w.geo_h = c->geo_h;
   w.x = c->pf[F_X]; w.y = c->pf[F_Y]; w.z = c->pf[F_Z];
-  w.hcand = uni ? c->df[D_HSEARCH] : c->pf[F_H];
-  w.htarget = mode == 0 ? c->df[D_HSEARCH] : c->pf[F_H];
+  w.hcand = kind == WALK_UNION ? c->df[D_HSEARCH] : c->pf[F_H];
+  w.htarget = kind == WALK_GATHER || kind == WALK_UNION ? c->df[D_HSEARCH] : c->pf[F_H];
   w.status = status;
   w.grp_root = c->nseg > 0 ? c->grp_root : nullptr;
   w.glist = glist; w.ncap = c->Ncap;
@@ -863,32 +897,21 @@ int launch_walk(gdf_ctx* c, int mode, int nopbc, CandSet& cs, const int* status,
   w.p = c->phys;
   if (nopbc) w.p.periodic = 0;
   if (!glist) k_zero_ints<<<1, BS, 0, c->stream>>>(8, c->counters + 4);
-  const int grid = std::min(c->ngroups, kWalkSlots);
+  const int grid = std::min(ng, kWalkSlots);
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
-  const int m = mode == 0 ? (mixed ? 3 : 0) : (mixed ? 2 : 1);
   hipStream_t st = c->stream;
   if (w.p.periodic) {
-    if (m == 0) k_walk_cand<0, true><<<grid, kWave, 0, st>>>(w);
-    else if (m == 1) k_walk_cand<1, true><<<grid, kWave, 0, st>>>(w);
-    else if (m == 2) {
-      if (masks) k_walk_cand<2, true><<<grid, kWave, 0, st>>>(w);
-      else k_walk_cand<2, true, false><<<grid, kWave, 0, st>>>(w);
-    } else {
-      if (masks) k_walk_cand<3, true><<<grid, kWave, 0, st>>>(w);
-      else if (uni) k_walk_cand<3, true, false, true><<<grid, kWave, 0, st>>>(w);
-      else k_walk_cand<3, true, false><<<grid, kWave, 0, st>>>(w);
-    }
+    if (kind == WALK_GATHER) k_walk_cand<0, true><<<grid, kWave, 0, st>>>(w);
+    else if (kind == WALK_UNION) k_walk_cand<0, true, false, true><<<grid, kWave, 0, st>>>(w);
+    else if (kind == WALK_SG) k_walk_cand<1, true><<<grid, kWave, 0, st>>>(w);
+    else if (mixed) k_walk_cand<2, true, true><<<grid, kWave, 0, st>>>(w);
+    else k_walk_cand<1, true, true><<<grid, kWave, 0, st>>>(w);
   } else {
-    if (m == 0) k_walk_cand<0, false><<<grid, kWave, 0, st>>>(w);
-    else if (m == 1) k_walk_cand<1, false><<<grid, kWave, 0, st>>>(w);
-    else if (m == 2) {
-      if (masks) k_walk_cand<2, false><<<grid, kWave, 0, st>>>(w);
-      else k_walk_cand<2, false, false><<<grid, kWave, 0, st>>>(w);
-    } else {
-      if (masks) k_walk_cand<3, false><<<grid, kWave, 0, st>>>(w);
-      else if (uni) k_walk_cand<3, false, false, true><<<grid, kWave, 0, st>>>(w);
-      else k_walk_cand<3, false, false><<<grid, kWave, 0, st>>>(w);
-    }
+    if (kind == WALK_GATHER) k_walk_cand<0, false><<<grid, kWave, 0, st>>>(w);
+    else if (kind == WALK_UNION) k_walk_cand<0, false, false, true><<<grid, kWave, 0, st>>>(w);
+    else if (kind == WALK_SG) k_walk_cand<1, false><<<grid, kWave, 0, st>>>(w);
+    else if (mixed) k_walk_cand<2, false, true><<<grid, kWave, 0, st>>>(w);
+    else k_walk_cand<1, false, true><<<grid, kWave, 0, st>>>(w);
   }
   GDF_HIP(c, hipGetLastError());
   return GDF_OK;
@@ -920,9 +943,9 @@ int sph_density(gdf_ctx* c, int nopbc) {
   const int N = c->N;
   hipStream_t s = c->stream;
   if (!c->tree_valid) return fail(c, GDF_ERR_INVALID, "density pass before tree build");
-  GDF_TRY(ensure_cand(c, c->cs_g));
-  k_init_density<<<nblocks(N, BS), BS, 0, s>>>(N, c->pf[F_H], c->df[D_HSEARCH], c->status,
-                                               c->nlevels > 1 ? c->pi[I_ACT] : nullptr);
+  GDF_TRY(ensure_cand(c, c->cs_g, c->ngroups, false));
+  const int* act = c->nlevels > 1 ? c->pi[I_ACT] : nullptr;
+  k_init_density<<<nblocks(N, BS), BS, 0, s>>>(N, c->pf[F_H], c->df[D_HSEARCH], c->status, act);
   DensArgs d;
   d.N = N; d.ngroups = c->ngroups; d.nopbc = nopbc;
   d.grp_node = c->grp_node; d.grp_first = c->grp_first; d.grp_count = c->grp_count;
@@ -938,38 +961,55 @@ int sph_density(gdf_ctx* c, int nopbc) {
   d.p = c->phys;
   c->sg_union = false;
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
-  // mixed path with periodic images: the first round walks the union lists; they stay valid for
-  // the force pass if that round settles every target (a regrowth or retry round would walk
-  // again only the unsettled groups, and a retry grows search radii past the lists' bounds)
-  const bool uni = mixed && !nopbc;
+  const int waves = density_waves(c);
+  // with periodic images the walk makes the union lists, which the force pass reads if they
+  // still bound its set: no search radius may have grown (a retry) or been outgrown
+  const bool uni = !nopbc;
+  const WalkKind kind = uni ? WALK_UNION : WALK_GATHER;
+  bool grown = false, retried = false, outgrown = false;
   for (int round = 0; round < 64; round++) {
     // also clears the round's flags and the walk's queue counters
-    GDF_TRY(group_list(c, c->status, c->glist, c->cs_g.ncand, nullptr, nullptr, c->counters, 12));
-    GDF_TRY(launch_walk(c, 0, nopbc, c->cs_g, c->status, c->glist, !mixed, uni));
-    d.capb = c->cs_g.capb; d.idx = c->cs_g.idx; d.mask = c->cs_g.mask; d.ncand = c->cs_g.ncand;
-    if (mixed) k_density<float, true><<<c->ngroups, kWave, 0, s>>>(d);
-    else k_density<double><<<c->ngroups, kWave, 0, s>>>(d);
+    GDF_TRY(group_list(c, c->status, c->glist, c->cs_g.ncand, nullptr, nullptr, c->counters,
+                       12));
+    GDF_TRY(launch_walk(c, kind, nopbc, c->cs_g, c->status, c->glist));
+    d.capb = c->cs_g.capb; d.idx = c->cs_g.idx; d.ncand = c->cs_g.ncand;
+    if (mixed) launch_density<float>(d, waves, s);
+    else launch_density<double>(d, waves, s);
     k_hrho_finish<<<nblocks(N, BS), BS, 0, s>>>(d);
     GDF_HIP(c, hipGetLastError());
     GDF_TRY(read_flags(c));
     const int* f = c->h_counters;
     if (f[2]) return fail(c, GDF_ERR_CAPACITY, "tree walk stack overflow in gather pass");
     if (f[3] & 1) return fail(c, GDF_ERR_NOCONV, "Problem with convergence of h-rho iteration");
+    outgrown = outgrown || (f[3] & 2);
+    retried = retried || f[0] > 0;
     // groups whose candidates overflowed skipped the density kernel and keep status 1
-    if (f[1] > 0) { GDF_TRY(grow_cand(c, c->cs_g, f[1])); continue; }
-    if (f[0] == 0) {
-      c->sg_valid = false;
-      GDF_TRY(tree_refit_h(c));
-      c->sg_union = uni && round == 0 && !(f[3] & 2);
-      return GDF_OK;
+    if (f[1] > 0) {
+      GDF_TRY(grow_cand(c, c->cs_g, c->ngroups, f[1], false));
+      grown = true;
+      continue;
     }
+    if (f[0] != 0) continue;
+    c->sg_valid = false;
+    c->sg_union = uni && !retried && !outgrown;
+    if (c->sg_union && grown) {
+      // growing dropped the lists of the groups settled before: every group's again, as the
+      // first round would have made them with room enough (the radii and the nodes' bounds are
+      // still those of its start)
+      if (act) GDF_TRY(group_list(c, act, c->glist, c->cs_g.ncand, nullptr, nullptr,
+                                  c->counters, 12));
+      else k_zero_ints<<<1, BS, 0, s>>>(4, c->counters);
+      GDF_TRY(launch_walk(c, kind, nopbc, c->cs_g, act, act ? c->glist : nullptr));
+      GDF_TRY(read_flags(c));
+      if (c->h_counters[2]) return fail(c, GDF_ERR_CAPACITY, "tree walk stack overflow in gather pass");
+      if (c->h_counters[1] > 0) c->sg_union = false;
+    }
+    return tree_refit_h(c);
   }
   return fail(c, GDF_ERR_CAPACITY, "h-rho neighbour search did not settle after 64 rounds");
 }
 
 int sph_build_sg(gdf_ctx* c, bool masks) {
-  // the mixed hydro kernel tests its candidates itself unless the masks are asked for
-  masks = masks || c->cfg.precision != GDF_PREC_MIXED;
   c->sg_from_union = false;
   if (!masks && c->sg_union) {      // the density pass's union lists hold the set
     c->sg_from_union = true;
@@ -977,16 +1017,20 @@ int sph_build_sg(gdf_ctx* c, bool masks) {
     c->sg_masks = false;
     return GDF_OK;
   }
-  GDF_TRY(ensure_cand(c, c->cs_s));
+  const int ng = c->ngroups;
+  GDF_TRY(ensure_cand(c, c->cs_s, ng, masks));
   for (int round = 0; round < 8; round++) {
     const int* act = c->nlevels > 1 ? c->pi[I_ACT] : nullptr;
     int* sl = c->glist + (c->Ncap + 1);
     if (act) GDF_TRY(group_list(c, act, sl, c->cs_s.ncand, nullptr, nullptr, c->counters, 12));
     else k_zero_ints<<<1, BS, 0, c->stream>>>(4, c->counters);
-    GDF_TRY(launch_walk(c, 1, 0, c->cs_s, act, act ? sl : nullptr, masks));
+    GDF_TRY(launch_walk(c, masks ? WALK_MASKS : WALK_SG, 0, c->cs_s, act, act ? sl : nullptr));
     GDF_TRY(read_flags(c));
     if (c->h_counters[2]) return fail(c, GDF_ERR_CAPACITY, "tree walk stack overflow in force pass");
-    if (c->h_counters[1] > 0) { GDF_TRY(grow_cand(c, c->cs_s, c->h_counters[1])); continue; }
+    if (c->h_counters[1] > 0) {
+      GDF_TRY(grow_cand(c, c->cs_s, ng, c->h_counters[1], masks));
+      continue;
+    }
     c->sg_valid = true;
     c->sg_masks = masks;
     return GDF_OK;
@@ -997,7 +1041,7 @@ int sph_build_sg(gdf_ctx* c, bool masks) {
 int sph_hydro(gdf_ctx* c, int variant) {
   const int N = c->N;
   hipStream_t s = c->stream;
-  if (!c->sg_valid) GDF_TRY(sph_build_sg(c));
+  if (!c->sg_valid || c->sg_masks) GDF_TRY(sph_build_sg(c));
   k_pack_hydro<<<nblocks(N, BS), BS, 0, s>>>(N, c->pf[F_VX], c->pf[F_VY], c->pf[F_VZ],
                                              c->pf[F_H], c->df[D_RHO], c->df[D_PRESSURE],
                                              c->df[D_INVOMEGA], c->df[D_SOUND],
@@ -1006,8 +1050,8 @@ int sph_hydro(gdf_ctx* c, int variant) {
   const CandSet& cs = c->sg_from_union ? c->cs_g : c->cs_s;
   h.N = N; h.ngroups = c->ngroups; h.capb = cs.capb;
   h.grp_node = c->grp_node; h.grp_first = c->grp_first; h.grp_count = c->grp_count;
-  h.geo_c = c->geo_c;
-  h.idx = cs.idx; h.mask = cs.mask; h.ncand = cs.ncand;
+  h.geo_c = c->geo_c; h.geo_h = c->geo_h;
+  h.idx = cs.idx; h.ncand = cs.ncand;
   h.posm = c->posm; h.A = c->hrecA; h.B = c->hrecB; h.h = c->pf[F_H];
   h.invomega = c->df[D_INVOMEGA]; h.pressure = c->df[D_PRESSURE]; h.zeta = c->df[D_ZETA];
   h.ax = c->df[D_AX]; h.ay = c->df[D_AY]; h.az = c->df[D_AZ];
@@ -1017,7 +1061,6 @@ int sph_hydro(gdf_ctx* c, int variant) {
   h.act = c->pi[I_ACT]; h.level = c->pi[I_LEVEL]; h.levelneib = c->pi[I_LEVELNEIB];
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
   const bool blk = c->nlevels > 1;
-  const int G = c->ngroups;
   if (mixed) {
     // the pass's targets, for decoding the sets it evaluates (its lists cover those alone)
     c->sg_tgt_all = !blk;
@@ -1034,28 +1077,8 @@ int sph_hydro(gdf_ctx* c, int variant) {
     }
   }
   const int kt = ktime_begin(c, s, 6);
-  const bool fused = mixed && !c->sg_masks;
-  if (variant == 0) {
-    if (blk) {
-      if (fused) k_hydro_mixed<0, true, true><<<G, kWave, 0, s>>>(h);
-      else if (mixed) k_hydro_mixed<0, true><<<G, kWave, 0, s>>>(h);
-      else k_hydro<0, true><<<G, kWave, 0, s>>>(h);
-    } else {
-      if (fused) k_hydro_mixed<0, false, true><<<G, kWave, 0, s>>>(h);
-      else if (mixed) k_hydro_mixed<0, false><<<G, kWave, 0, s>>>(h);
-      else k_hydro<0, false><<<G, kWave, 0, s>>>(h);
-    }
-  } else {
-    if (blk) {
-      if (fused) k_hydro_mixed<1, true, true><<<G, kWave, 0, s>>>(h);
-      else if (mixed) k_hydro_mixed<1, true><<<G, kWave, 0, s>>>(h);
-      else k_hydro<1, true><<<G, kWave, 0, s>>>(h);
-    } else {
-      if (fused) k_hydro_mixed<1, false, true><<<G, kWave, 0, s>>>(h);
-      else if (mixed) k_hydro_mixed<1, false><<<G, kWave, 0, s>>>(h);
-      else k_hydro<1, false><<<G, kWave, 0, s>>>(h);
-    }
-  }
+  if (mixed) launch_hydro<float>(h, variant, blk, hydro_waves(c), s);
+  else launch_hydro<double>(h, variant, blk, hydro_waves(c), s);
   GDF_HIP(c, hipGetLastError());
   ktime_end(c, s, kt);
   return GDF_OK;

@@ -542,82 +542,120 @@ struct NbDirectArgs {
   int add;          // add to a, adot and gpot (after the stars' gas terms) instead of writing
 };
 
-// Star-star direct sums, one thread per star, source stars staged 256 at a time in LDS.
-// SMOOTH = false: Nbody::CalculateDirectGravForces (src/Nbody/Nbody.cpp:233-293), point
-// masses with jerk; SMOOTH = true: NbodyLeapfrogKDK::CalculateDirectSmoothedGravForces
-// (src/Nbody/NbodyLeapfrogKDK.cpp:78-150), kernel softening over the mean smoothing length,
-// whose (2/(h_i+h_j))^3 factor the reference forms in single precision (powf).
-template <bool SMOOTH>
+// Star-star direct sums.  SMOOTH = false: Nbody::CalculateDirectGravForces
+// (src/Nbody/Nbody.cpp:233-293), point masses with jerk; SMOOTH = true:
+// NbodyLeapfrogKDK::CalculateDirectSmoothedGravForces (src/Nbody/NbodyLeapfrogKDK.cpp:78-150),
+// kernel softening over the mean smoothing length, whose (2/(h_i+h_j))^3 factor the reference
+// forms in single precision (powf).
+//
+// A block of 256 threads takes T targets; the 256/T threads of a target take every (256/T)-th
+// source of the tiles staged in LDS (the next tile is in flight meanwhile) and their sums are
+// added in a fixed order.  Bound by FP64 issue, about 45 instructions a pair.  T small enough that
+// the blocks fill the device: one thread a target put 6007 stars on 24 of the 256 CUs, and a
+// division and a square root cost more than the rest of the pair.  6007 stars, softened: 99 us
+// against 3690.
+template <bool SMOOTH, int T>
 __global__ __launch_bounds__(256) void k_nbody_direct(NbDirectArgs a) {
-  constexpr int T = 256;
-  __shared__ double sx[T], sy[T], sz[T], svx[T], svy[T], svz[T], sm[T], sh[T];
-  const int i = blockIdx.x*T + threadIdx.x;
-  const bool has = i < a.N;
-  double xi = 0, yi = 0, zi = 0, vxi = 0, vyi = 0, vzi = 0, hi = 1.0;
-  if (has) {
-    xi = a.x[i]; yi = a.y[i]; zi = a.z[i]; vxi = a.vx[i]; vyi = a.vy[i]; vzi = a.vz[i];
-    if (SMOOTH) hi = a.h[i];
-  }
-  double ax = 0, ay = 0, az = 0, jx = 0, jy = 0, jz = 0, pot = 0;
-  for (int j0 = 0; j0 < a.N; j0 += T) {
-    const int jl = j0 + threadIdx.x;
-    if (jl < a.N) {
-      sx[threadIdx.x] = a.x[jl]; sy[threadIdx.x] = a.y[jl]; sz[threadIdx.x] = a.z[jl];
-      svx[threadIdx.x] = a.vx[jl]; svy[threadIdx.x] = a.vy[jl]; svz[threadIdx.x] = a.vz[jl];
-      sm[threadIdx.x] = a.m[jl]; sh[threadIdx.x] = SMOOTH ? a.h[jl] : 0.0;
-    }
+  constexpr int BT = 256, S = BT/T;
+  __shared__ double2 sxy[BT], szm[BT], suv[BT], swh[BT];
+  __shared__ double red[BT/kWave][7][T];
+  const int tid = threadIdx.x, t = tid % T;
+  const int i = blockIdx.x*T + t;
+  const int ii = min(i, a.N - 1);
+  const double xi = a.x[ii], yi = a.y[ii], zi = a.z[ii];
+  const double vxi = a.vx[ii], vyi = a.vy[ii], vzi = a.vz[ii];
+  const double hi = SMOOTH ? a.h[ii] : 1.0;
+  const double hrange = 0.5*a.kern.range*(1.0 + 1.0e-12);
+  double sum[7] = {0, 0, 0, 0, 0, 0, 0};      // a, adot, gpot
+  double2 nxy, nzm, nuv, nwh;
+  auto fetch = [&](int j0) {
+    const int j = min(j0 + tid, a.N - 1);
+    nxy = make_double2(a.x[j], a.y[j]);
+    nzm = make_double2(a.z[j], a.m[j]);
+    nuv = make_double2(a.vx[j], a.vy[j]);
+    nwh = make_double2(a.vz[j], SMOOTH ? a.h[j] : 0.0);
+  };
+  fetch(0);
+  for (int j0 = 0; j0 < a.N; j0 += BT) {
+    sxy[tid] = nxy; szm[tid] = nzm; suv[tid] = nuv; swh[tid] = nwh;
     __syncthreads();
-    const int nb = min(T, a.N - j0);
-    if (has) {
-      for (int q = 0; q < nb; q++) {
-        if (j0 + q == i) continue;
-        const double dx = sx[q] - xi, dy = sy[q] - yi, dz = sz[q] - zi;
-        const double dvx = svx[q] - vxi, dvy = svy[q] - vyi, dvz = svz[q] - vzi;
-        const double drsqd = dx*dx + dy*dy + dz*dz;
-        const double mj = sm[q];
-        if (!SMOOTH) {
-          const double invdrmag = 1.0/sqrt(drsqd);
-          const double drdt = (dvx*dx + dvy*dy + dvz*dz)*invdrmag;
-          const double inv3 = invdrmag*invdrmag*invdrmag;
-          pot += mj*invdrmag;
-          ax += mj*dx*inv3; ay += mj*dy*inv3; az += mj*dz*inv3;
-          const double c3 = 3.0*drdt*invdrmag;
-          jx += mj*inv3*(dvx - c3*dx); jy += mj*inv3*(dvy - c3*dy); jz += mj*inv3*(dvz - c3*dz);
+    if (j0 + BT < a.N) fetch(j0 + BT);
+    const int nb = min(BT, a.N - j0);
+    for (int q = tid/T; q < nb; q += S) {
+      if (j0 + q == i) continue;
+      const double2 xy = sxy[q], zm = szm[q], uv = suv[q], wh = swh[q];
+      const double dx = xy.x - xi, dy = xy.y - yi, dz = zm.x - zi;
+      const double dvx = uv.x - vxi, dvy = uv.y - vyi, dvz = wh.x - vzi;
+      const double drsqd = dx*dx + dy*dy + dz*dz;
+      const double mj = zm.y;
+      // 1/|dr| from the estimate; coincident stars and separations at the ends of the exponent
+      // range keep the division
+      const bool easy = drsqd > (SMOOTH ? 1.0e-30 : 1.0e-280) && drsqd < 1.0e280;
+      double invdrmag, drmag;
+      if (easy) {
+        const double y = rsq_d(drsqd);
+        if (SMOOTH) {
+          // drmag = sqrt(drsqd) + 1e-20 and its reciprocal: the shift is below 1e-5 of either
+          drmag = fma(drsqd, y, 1.0e-20);
+          const double e = 1.0e-20*y;
+          invdrmag = fma(-e*(1.0 - e), y, y);
         } else {
-          const double drmag = sqrt(drsqd) + 1.0e-20;
-          const double invdrmag = 1.0/drmag;
-          const double invhmean = 2.0/(hi + sh[q]);
-          const double drdt = (dvx*dx + dvy*dy + dvz*dz)*invdrmag;
-          const double s = drmag*invhmean;
-          const double paux = mj*invhmean*invhmean*kwgrav<double>(a.kern, s)*invdrmag;
-          // the reference's single-precision powf(invhmean, 3): the correctly rounded cube
-          // (exact in double before the one rounding to float), which is what glibc's powf
-          // returns for all but ~0.07% of arguments (those differ by one float ulp)
-          const float hmf = (float) invhmean;
-          const double wmean = kw0<double>(a.kern, s)*
-                               (double) (float) ((double) hmf*(double) hmf*(double) hmf);
-          pot += mj*invhmean*kwpot<double>(a.kern, s);
-          ax += paux*dx; ay += paux*dy; az += paux*dz;
-          const double c3 = 3.0*paux*drdt*invdrmag;
-          const double cw = 2.0*6.28318530717959*mj*drdt*wmean*invdrmag;
-          jx += paux*dvx - c3*dx + cw*dx;
-          jy += paux*dvy - c3*dy + cw*dy;
-          jz += paux*dvz - c3*dz + cw*dz;
+          invdrmag = y;
+          drmag = 0.0;
         }
+      } else {
+        drmag = sqrt(drsqd) + (SMOOTH ? 1.0e-20 : 0.0);
+        invdrmag = 1.0/drmag;
       }
+      const double inv2 = invdrmag*invdrmag;
+      const double c = 3.0*(dvx*dx + dvy*dy + dvz*dz)*inv2;      // 3 drdt/|dr|
+      double paux = mj*(inv2*invdrmag), p = mj*invdrmag, cw = 0.0;
+      if (SMOOTH && drmag < hrange*(hi + wh.y)) {     // at or inside the kernel's range
+        const double invhmean = 2.0/(hi + wh.y);
+        const double s = drmag*invhmean;
+        paux = mj*invhmean*invhmean*kwgrav<double>(a.kern, s)*invdrmag;
+        p = mj*invhmean*kwpot<double>(a.kern, s);
+        // the reference's single-precision powf(invhmean, 3): the correctly rounded cube
+        // (exact in double before the one rounding to float), which is what glibc's powf
+        // returns for all but ~0.07% of arguments (those differ by one float ulp)
+        const float hmf = (float) invhmean;
+        const double wmean = kw0<double>(a.kern, s)*
+                             (double) (float) ((double) hmf*(double) hmf*(double) hmf);
+        cw = 2.0*6.28318530717959*(1.0/3.0)*mj*c*wmean;
+      }
+      const double cj = cw - paux*c;
+      sum[0] += paux*dx; sum[1] += paux*dy; sum[2] += paux*dz;
+      sum[3] += paux*dvx + cj*dx; sum[4] += paux*dvy + cj*dy; sum[5] += paux*dvz + cj*dz;
+      sum[6] += p;
     }
     __syncthreads();
   }
-  if (!has) return;
-  if (a.add) {
-    a.ax[i] += ax; a.ay[i] += ay; a.az[i] += az;
-    a.adx[i] += jx; a.ady[i] += jy; a.adz[i] += jz;
-    a.gpot[i] += pot;
-    return;
+  for (int k = 0; k < 7; k++) {
+    #pragma unroll
+    for (int o = T; o < kWave; o *= 2) sum[k] += __shfl_xor(sum[k], o, kWave);
+    if (tid % kWave < T) red[tid/kWave][k][t] = sum[k];
   }
-  a.ax[i] = ax; a.ay[i] = ay; a.az[i] = az;
-  a.adx[i] = jx; a.ady[i] = jy; a.adz[i] = jz;
-  a.gpot[i] = pot;
+  __syncthreads();
+  if (tid >= T || i >= a.N) return;
+  for (int k = 0; k < 7; k++)
+    sum[k] = (red[0][k][t] + red[1][k][t]) + (red[2][k][t] + red[3][k][t]);
+  double* out[7] = {a.ax, a.ay, a.az, a.adx, a.ady, a.adz, a.gpot};
+  for (int k = 0; k < 7; k++) out[k][i] = a.add ? out[k][i] + sum[k] : sum[k];
+}
+
+// Four targets a block while eight leave CUs idle: 500 stars 7.1 against 8.6 us, 2000 19.4 against
+// 22.7, 4000 50 against 53; then eight, which read half the source tiles: 6007 99 against 102 us,
+// 16000 576 against 622.  (Sixteen: 68 us at 4000, 132 at 6007, 589 at 16000.)
+void launch_nbody_direct(const NbDirectArgs& a, int smoothed, hipStream_t s) {
+  if (a.N < 8*512) {
+    const int nb = (a.N + 3)/4;
+    if (smoothed) k_nbody_direct<true, 4><<<nb, 256, 0, s>>>(a);
+    else k_nbody_direct<false, 4><<<nb, 256, 0, s>>>(a);
+  } else {
+    const int nb = (a.N + 7)/8;
+    if (smoothed) k_nbody_direct<true, 8><<<nb, 256, 0, s>>>(a);
+    else k_nbody_direct<false, 8><<<nb, 256, 0, s>>>(a);
+  }
 }
 
 __global__ void k_pack_grav(int N, const double* __restrict__ h, const double* __restrict__ zeta,
@@ -662,9 +700,7 @@ int nbody_direct(gdf_ctx* c, int smoothed) {
   a.gpot = c->df[D_GPOT];
   a.kern = c->phys.kern;
   a.add = 0;
-  const int nb = (N + 255)/256;
-  if (smoothed) k_nbody_direct<true><<<nb, 256, 0, c->stream>>>(a);
-  else k_nbody_direct<false><<<nb, 256, 0, c->stream>>>(a);
+  launch_nbody_direct(a, smoothed, c->stream);
   GDF_HIP(c, hipGetLastError());
   return GDF_OK;
 }
@@ -682,9 +718,7 @@ int nbody_direct_stars(gdf_ctx* c, int smoothed) {
   a.gpot = c->sv[S_GPOT];
   a.kern = c->phys.kern;
   a.add = 1;
-  const int nb = (N + 255)/256;
-  if (smoothed) k_nbody_direct<true><<<nb, 256, 0, c->stream>>>(a);
-  else k_nbody_direct<false><<<nb, 256, 0, c->stream>>>(a);
+  launch_nbody_direct(a, smoothed, c->stream);
   GDF_HIP(c, hipGetLastError());
   return GDF_OK;
 }

@@ -7,7 +7,8 @@
 // GradhSphBase::ComputeDirectGravForces (:657-690) and the quadrupole cell terms of
 // ComputeQuadropole (src/Headers/NeighbourSearch.h:423-449).
 //
-// One wavefront per walk group.  Acceptance per node, with the group's bounding box G:
+// One workgroup of W wavefronts per walk group, which share its node stack: a round tests up to 64
+// nodes a wavefront.  Acceptance per node, with the group's bounding box G:
 //   * kernel-range test (as the reference's neighbour-cell test, Tree.cpp:662-663): if the
 //     minimum box-box distance is below k*max(hmax_G, hmax_cell) (with a 1e-4 relative slack
 //     on the squared distance) the node is resolved to particles (bucket of <= Nleafmax
@@ -21,19 +22,30 @@
 // the hydro pass (GradhSph::ComputeSphHydroGravForces); the walk adds the direct 1/r^2 terms of
 // every other particle and the multipole terms, masking the neighbour pairs with the same range
 // test.  Without a hydro pass the walk evaluates the softened pairs itself.  Accepted cells and
-// direct particles are staged 64 at a time in LDS and every lane (one target particle) sweeps
-// the batch; the FP32 path sums each batch in registers and carries Kahan-compensated totals
-// across batches.
+// direct particles are staged 64 at a time in LDS, a batch a wavefront, and every lane (one target
+// particle) sweeps the batch; the FP32 path sums each batch in registers and carries
+// Kahan-compensated totals across batches.  The wavefronts' sums are added in order at the end.
+//
+// Bound by latency where the groups do not fill the device (each round and each batch waits for
+// its scattered node, cell or particle loads), and by vector issue beside the hydro pass where they
+// do.  20011 particles, FP64: 98 us with four wavefronts a group against 295 with one and the cell
+// term's products written out; a million, FP64, beside the hydro pass: 4.6 against 5.5 ms.
 #include <hip/hip_runtime.h>
 
 #include "gdf_internal.h"
 #include "gdf_device.h"
+#include "gdf_filter.h"
 
 namespace gdf {
 namespace {
 
-constexpr int PCAP = 1024;   // particle ring buffer (power of two); Nleafmax <= 14
-constexpr int CCAP = 256;    // cell ring buffer (power of two)
+// Wavefronts that share a walk group, and the group's ring buffers (powers of two): a round adds
+// at most 64 W cells or 64 W buckets to what is left of the last one, less than 64 W of either
+template <int W> struct GravRings {
+  static constexpr int cells = 2*kWave*W;
+  static constexpr int parts = W == 1 ? 1024 : 512*W;
+  static constexpr int wide = 4096;      // stack entries beyond which a round takes 64 nodes
+};
 
 struct GravArgs {
   int N, ngroups, nleaf;
@@ -106,8 +118,9 @@ __device__ __forceinline__ void pair_fp32(const KernelDesc& k, float d2, bool so
   }
 }
 
-// quadrupole cell term with dr = rp - com (NeighbourSearch.h:423-449); 1/|dr| from the
-// reciprocal square root instead of a division and a square root
+// quadrupole cell term with dr = rp - com (NeighbourSearch.h:423-449), q = (xx, xy, yy, xz, yz,
+// zz): Q dr once for the field and the scalar dr Q dr; 1/|dr| from the reciprocal square root
+// instead of a division and a square root
 template <typename T>
 __device__ __forceinline__ void quad_term(T dx, T dy, T dz, T mc, const T* q, T& ax, T& ay,
                                           T& az, T& pot, T soft2 = T(1.0e-20)) {
@@ -117,14 +130,16 @@ __device__ __forceinline__ void quad_term(T dx, T dy, T dz, T mc, const T* q, T&
   else invdrmag = (T) rsq_d((double) drsqd);
   const T invdrsqd = invdrmag*invdrmag;
   const T invdr5 = invdrsqd*invdrsqd*invdrmag;
-  const T mono = mc*invdrsqd*invdrmag;
-  const T qscalar = q[0]*dx*dx + q[2]*dy*dy - (q[0] + q[2])*dz*dz +
-                    T(2)*(q[1]*dx*dy + q[3]*dx*dz + q[4]*dy*dz);
-  const T qfactor = T(2.5)*qscalar*invdr5*invdrsqd;
-  ax += -mono*dx + (q[0]*dx + q[1]*dy + q[3]*dz)*invdr5 - qfactor*dx;
-  ay += -mono*dy + (q[1]*dx + q[2]*dy + q[4]*dz)*invdr5 - qfactor*dy;
-  az += -mono*dz + (q[3]*dx + q[4]*dy - (q[0] + q[2])*dz)*invdr5 - qfactor*dz;
-  pot += mc*invdrmag + T(0.5)*qscalar*invdr5;
+  const T qx = q[0]*dx + q[1]*dy + q[3]*dz;
+  const T qy = q[1]*dx + q[2]*dy + q[4]*dz;
+  const T qz = q[3]*dx + q[4]*dy + q[5]*dz;
+  const T qs5 = (qx*dx + qy*dy + qz*dz)*invdr5;
+  const T m1 = mc*invdrmag;
+  const T c = (m1 + T(2.5)*qs5)*invdrsqd;
+  ax += qx*invdr5 - c*dx;
+  ay += qy*invdr5 - c*dy;
+  az += qz*invdr5 - c*dz;
+  pot += m1 + T(0.5)*qs5;
 }
 
 // Tree::open_cell_for_gravity (Tree.h:413-432) past its geometric test, for a cell at squared
@@ -209,29 +224,39 @@ __device__ __forceinline__ void fast_add(double* f, double dx, double dy, double
 // that point divided by theta, so that the series converges for every target.  multipole
 // monopole: the cells' moments are staged as zeros (the quadrupole term reduces to
 // ComputeCellMonopoleForces, NeighbourSearch.h:350-377).
-template <bool MIXED, bool SOFT, bool PLUMMER, bool EWALD = false, bool FAST = false>
-__global__ __launch_bounds__(64) void k_gravity(GravArgs a) {
-  __shared__ int pbuf[PCAP];
-  __shared__ int cbuf[CCAP];
-  __shared__ int sidx[kWave];
-  // staged batch: particles (x, y, z, m, r2, h, zeta, hfactor) or cells (com x3, m, q x5).
-  // The FP32 path stages per lane two float4 records and one float, each read back with one
-  // broadcast LDS load: particles (dx, dy, dz, m), (h, zeta, hfactor, -), r2; cells
-  // (dx, dy, dz, m), (q0, q1, q2, q3), q4
-  __shared__ __align__(16) double stage[(MIXED ? 5 : 9)*kWave];
-  double (*sd)[kWave] = reinterpret_cast<double (*)[kWave]>(stage);
-  float4* s4a = reinterpret_cast<float4*>(stage);
-  float4* s4b = s4a + kWave;
-  float* s1 = reinterpret_cast<float*>(s4b + kWave);
+template <bool MIXED, bool SOFT, bool PLUMMER, bool EWALD = false, bool FAST = false, int W = 4>
+__global__ __launch_bounds__(64*W, EWALD || FAST || (SOFT && !PLUMMER) ? 2 : 3) void k_gravity(GravArgs a) {
+  typedef GravRings<W> R;
+  __shared__ int pbuf[R::parts];
+  __shared__ int cbuf[R::cells];
+  __shared__ int sidx[W][kWave];
+  // a wavefront's staged batch.  FP64: particles (x, y), (z, m), r2, (h, zeta), (hfactor, -) or
+  // cells (com x, y), (com z, m), (q0, q1), (q2, q3), (q4, q5).  FP32: two float4 records and a
+  // float2: particles (dx, dy, dz, m), (h, zeta, hfactor, -), (r2, -); cells (dx, dy, dz, m),
+  // (q0, q1, q2, q3), (q4, q5).  Each is read back with broadcast LDS loads.
+  __shared__ __align__(16) double stage[W][(MIXED ? 5 : 10)*kWave];
   __shared__ int lstk[kLdsStack];    // node stack; deeper entries go to the global region
-  const int lane = threadIdx.x;
+  __shared__ int count[W][3];        // a round's opened nodes, cells and particles
+  __shared__ int next;
+  const int lane = threadIdx.x & (kWave - 1), wv = W == 1 ? 0 : (int) threadIdx.x/kWave;
+  double2 (*sd)[kWave] = reinterpret_cast<double2 (*)[kWave]>(stage[wv]);
+  double* sr = stage[wv] + 8*kWave;
+  float4* s4a = reinterpret_cast<float4*>(stage[wv]);
+  float4* s4b = s4a + kWave;
+  float2* s2 = reinterpret_cast<float2*>(s4b + kWave);
+  int* sj = sidx[wv];
   int* stk = a.stacks + (size_t) blockIdx.x*kStackCap;
   const int N = a.N;
   const KernelDesc& K = a.p.kern;
   const double kr = K.range, krsqd = K.rangesqd;
   GroupQueue gq = group_queue(a.glist ? a.glist[a.ncap] : a.ngroups);
   for (;;) {
-    const int k = group_next(gq, a.counter);
+    // one lane alone fetches: every lane of a wavefront taking part in a divergent branch made 64
+    // atomics of each fetch, 0.4 ms over the device
+    if (threadIdx.x == 0) next = group_next(gq, a.counter);
+    __syncthreads();
+    const int k = __builtin_amdgcn_readfirstlane(next);
+    __syncthreads();
     if (k >= gq.nq) break;
     const int g = a.glist ? a.glist[k] : k;
     const int G = a.grp_node[g], gfirst = a.grp_first[g], gcnt = a.grp_count[g];
@@ -239,7 +264,7 @@ __global__ __launch_bounds__(64) void k_gravity(GravArgs a) {
     const int i = gfirst + lane;
     const int nact = __popcll(__ballot(has));
     if (nact == 0) {                 // no active target in this group
-      if (lane == 0) { a.gnc[g] = 0; a.gnn[g] = 0; }
+      if (threadIdx.x == 0) { a.gnc[g] = 0; a.gnn[g] = 0; }
       continue;
     }
     const double4 gc = a.geo_c[G], gh = a.geo_h[G];
@@ -264,23 +289,170 @@ __global__ __launch_bounds__(64) void k_gravity(GravArgs a) {
     if (has) { me = a.posm[i]; mr = a.grec[i]; }
     const double r2i = range2_rn(krsqd, mr.x);
     const float r2if = (float) r2i;
-    // accumulators; gpot starts at the self term (m/h) wpot(0) (GradhSphTree.cpp:512)
     double ax = 0.0, ay = 0.0, az = 0.0, pot = 0.0;
     KahanF fx, fy, fz, fp;
-    const double pot0 = (has && !PLUMMER) ? (me.w/mr.x)*kwpot<double>(K, 0.0) : 0.0;
     const double eps2 = a.p.eps2;
     const float eps2f = (float) eps2;
     // target position relative to the group centre (cell-relative frame of the FP32 path)
     const float rxi = (float) (me.x - gc.x), ryi = (float) (me.y - gc.y), rzi = (float) (me.z - gc.z);
+
+    // a batch of nb accepted cells from ring position c0
+    auto eval_cells = [&](int c0, int nb) {
+      if (lane < nb) {
+        const int c = cbuf[(c0 + lane) & (R::cells - 1)];
+        const double* m = a.mp + 10*(size_t) c;
+        double cx = m[0], cy = m[1], cz = m[2];
+        if (FAST) {
+#pragma clang fp contract(off)
+          // the cell relative to the expansion point, with the node test's replica
+          double dx = cx - gc.x, dy = cy - gc.y, dz = cz - gc.z;
+          nearest_image<double>(a.p, dx, dy, dz);
+          fast_add(fc, dx - rcx, dy - rcy, dz - rcz, m[3], m + 4,
+                   a.p.multipole == GDF_MULTIPOLE_FAST_QUADRUPOLE);
+        }
+        if (a.p.periodic) {
+          // nearest periodic replica of the cell relative to the group centre
+          double dx = cx - gc.x, dy = cy - gc.y, dz = cz - gc.z;
+          nearest_image<double>(a.p, dx, dy, dz);
+          cx = gc.x + dx; cy = gc.y + dy; cz = gc.z + dz;
+        }
+        const double qs = mono ? 0.0 : 1.0;      // monopole: no quadrupole moments
+        const double q0 = qs*m[4], q2 = qs*m[6];
+        if (MIXED) {
+          s4a[lane] = make_float4((float) (cx - gc.x), (float) (cy - gc.y),
+                                  (float) (cz - gc.z), (float) m[3]);
+          s4b[lane] = make_float4((float) q0, (float) (qs*m[5]), (float) q2, (float) (qs*m[7]));
+          s2[lane] = make_float2((float) (qs*m[8]), -((float) q0 + (float) q2));
+        } else {
+          sd[0][lane] = make_double2(cx, cy); sd[1][lane] = make_double2(cz, m[3]);
+          sd[2][lane] = make_double2(q0, qs*m[5]); sd[3][lane] = make_double2(q2, qs*m[7]);
+          sd[4][lane] = make_double2(qs*m[8], -(q0 + q2));
+        }
+      }
+      wave_lds_order();
+      // fast multipoles leave only the periodic corrections to the per-target sweep
+      if (has && (!FAST || EWALD)) {
+        if (MIXED) {
+          float bx = 0.f, by = 0.f, bz = 0.f, bp = 0.f;
+          #pragma unroll 4
+          for (int q = 0; q < nb; q++) {
+            const float4 c = s4a[q], qa = s4b[q];
+            const float2 qb = s2[q];
+            const float qq[6] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y};
+            if (!FAST)
+              quad_term<float>(rxi - c.x, ryi - c.y, rzi - c.z, c.w, qq, bx, by, bz, bp,
+                               PLUMMER ? eps2f : 1.0e-20f);
+            if (EWALD) ewald_corr<float>(a.p, c.x - rxi, c.y - ryi, c.z - rzi, c.w, bx, by, bz,
+                                         bp);
+          }
+          fx.add(bx); fy.add(by); fz.add(bz); fp.add(bp);
+        } else {
+          #pragma unroll 2
+          for (int q = 0; q < nb; q++) {
+            const double2 xy = sd[0][q], zm = sd[1][q], qa = sd[2][q], qb = sd[3][q], qc = sd[4][q];
+            const double qq[6] = {qa.x, qa.y, qb.x, qb.y, qc.x, qc.y};
+            if (!FAST)
+              quad_term<double>(me.x - xy.x, me.y - xy.y, me.z - zm.x, zm.y, qq, ax, ay, az, pot,
+                                PLUMMER ? eps2 : 1.0e-20);
+            if (EWALD) ewald_corr<double>(a.p, xy.x - me.x, xy.y - me.y, zm.x - me.z, zm.y, ax,
+                                          ay, az, pot);
+          }
+        }
+      }
+      wave_lds_order();
+    };
+    // a batch of nb direct particles from ring position p0
+    auto eval_parts = [&](int p0, int nb) {
+      if (lane < nb) {
+        const int j = pbuf[(p0 + lane) & (R::parts - 1)];
+        const double4 pj = a.posm[j];
+        const double4 rj = a.grec[j];
+        sj[lane] = j;
+        if (MIXED) {
+          double dx = pj.x - gc.x, dy = pj.y - gc.y, dz = pj.z - gc.z;
+          nearest_image<double>(a.p, dx, dy, dz);
+          s4a[lane] = make_float4((float) dx, (float) dy, (float) dz, (float) pj.w);
+          s2[lane] = make_float2((float) range2_rn(krsqd, rj.x), 0.f);
+          if (SOFT) s4b[lane] = make_float4((float) rj.x, (float) rj.y, (float) rj.z, 0.f);
+        } else {
+          sd[0][lane] = make_double2(pj.x, pj.y); sd[1][lane] = make_double2(pj.z, pj.w);
+          if (SOFT) { sd[2][lane] = make_double2(rj.x, rj.y); sd[3][lane].x = rj.z; }
+          sr[lane] = range2_rn(krsqd, rj.x);
+        }
+      }
+      wave_lds_order();
+      if (has) {
+        if (MIXED) {
+          const float hi = (float) mr.x, zi = (float) mr.y, hfi = (float) mr.z;
+          float bx = 0.f, by = 0.f, bz = 0.f, bp = 0.f;
+          // unrolled so that several LDS reads are in flight (same summation order)
+          #pragma unroll 8
+          for (int q = 0; q < nb; q++) {
+            // every record is loaded whatever the pair's branch: no LDS read under a mask
+            const float4 s = s4a[q];
+            const float r2j = s2[q].x;
+            const float dx = s.x - rxi, dy = s.y - ryi, dz = s.z - rzi;
+            const float d2 = dot3_f(dx, dy, dz);
+            const bool soft = (d2 < r2if) | (d2 < r2j);
+            if (PLUMMER) {
+              const float inv = rsq_f(d2 + eps2f);
+              const float mj = sj[q] == i ? 0.f : s.w;
+              const float minv3 = mj*inv*inv*inv;
+              bx += minv3*dx; by += minv3*dy; bz += minv3*dz; bp += mj*inv;
+            } else if (SOFT) {
+              const float4 hq = s4b[q];
+              pair_fp32(K, d2, soft, dx, dy, dz, s.w, hi, hq.x, zi, hq.y, hfi, hq.z, bx, by,
+                        bz, bp);
+            } else {
+              const float inv = rsq_f(d2 + 1.0e-20f);
+              const float mj = soft ? 0.f : s.w;
+              const float minv3 = mj*inv*inv*inv;
+              bx += minv3*dx; by += minv3*dy; bz += minv3*dz; bp += mj*inv;
+            }
+            if (EWALD) ewald_corr<float>(a.p, dx, dy, dz, s.w, bx, by, bz, bp);
+          }
+          fx.add(bx); fy.add(by); fz.add(bz); fp.add(bp);
+        } else {
+          #pragma unroll 2
+          for (int q = 0; q < nb; q++) {
+            const double2 xy = sd[0][q], zm = sd[1][q];
+            double dx = xy.x - me.x, dy = xy.y - me.y, dz = zm.x - me.z;
+            nearest_image<double>(a.p, dx, dy, dz);
+            if (PLUMMER) {
+              const double inv = rsq_d(dot3_rn(dx, dy, dz) + eps2);
+              const double mj = sj[q] == i ? 0.0 : zm.y;
+              const double minv3 = mj*inv*inv*inv;
+              ax += minv3*dx; ay += minv3*dy; az += minv3*dz; pot += mj*inv;
+            } else if (SOFT) {
+              const double2 hq = sd[2][q];
+              pair_fp64(K, krsqd, dx, dy, dz, zm.y, mr.x, hq.x, mr.y, hq.y, mr.z, sd[3][q].x, ax,
+                        ay, az, pot);
+            } else {
+              const double d2 = dot3_rn(dx, dy, dz);
+              const bool soft = (d2 < r2i) | (d2 < sr[q]);
+              const double inv = rsq_d(d2 + 1.0e-20);
+              const double mj = soft ? 0.0 : zm.y;
+              const double minv3 = mj*inv*inv*inv;
+              ax += minv3*dx; ay += minv3*dy; az += minv3*dz; pot += mj*inv;
+            }
+            if (EWALD) ewald_corr<double>(a.p, dx, dy, dz, zm.y, ax, ay, az, pot);
+          }
+        }
+      }
+      wave_lds_order();
+    };
+
     int sp = 1, phead = 0, ptail = 0, chead = 0, ctail = 0;
-    int nnear = 0, ncell = 0;
     bool overflow = false;
-    if (lane == 0) lstk[0] = a.grp_root ? a.grp_root[g] : 0;   // the group's segment subtree
+    // nodes a round may take: what the particle ring holds at the largest bucket
+    const int most = min(kWave*W, (R::parts - kWave*W)/max(a.nleaf, 1));
+    if (threadIdx.x == 0) lstk[0] = a.grp_root ? a.grp_root[g] : 0;  // the group's segment subtree
     __syncthreads();
     while (sp > 0) {
-      const int b = min(sp, kWave);
+      const int b = min(sp, sp > R::wide ? min(most, kWave) : most);
+      const int slot = wv*kWave + lane;
       int node = -1;
-      if (lane < b) node = stack_get(lstk, stk, sp - 1 - lane);
+      if (slot < b) node = stack_get(lstk, stk, sp - 1 - slot);
       sp -= b;
       bool open = false, near = false, cell = false;
       int ef = 0, ec = 0, cl = 0, cr = 0;
@@ -323,176 +495,54 @@ __global__ __launch_bounds__(64) void k_gravity(GravArgs a) {
         }
         if (open) { cl = nl.left; cr = nl.right; }
       }
-      // children onto the stack
-      const unsigned long long om = __ballot(open);
-      const int nopen = __popcll(om);
+      // places of the round's opened nodes, cells and particles, wavefront by wavefront
+      const unsigned long long om = __ballot(open), cm = __ballot(cell);
+      const int ecount = near ? ec : 0;
+      const int incl = wave_incl_scan(ecount);
+      int o0 = 0, c0 = ctail, p0 = ptail, nopen = __popcll(om);
+      if (W == 1) {
+        ctail += __popcll(cm);
+        ptail += __shfl(incl, 63, 64);
+      } else {
+        if (lane == 63) { count[wv][0] = nopen; count[wv][1] = __popcll(cm); count[wv][2] = incl; }
+        __syncthreads();
+        nopen = 0;
+        #pragma unroll
+        for (int w = 0; w < W; w++) {
+          if (w == wv) { o0 = nopen; c0 = ctail; p0 = ptail; }
+          nopen += count[w][0]; ctail += count[w][1]; ptail += count[w][2];
+        }
+      }
       if (sp + 2*nopen > kLdsStack + kStackCap) { overflow = true; break; }
       if (open) {
-        const int o = sp + 2*lanes_below(om);
+        const int o = sp + 2*(o0 + lanes_below(om));
         stack_put(lstk, stk, o, cr);
         stack_put(lstk, stk, o + 1, cl);
       }
       sp += 2*nopen;
       if (sp > kLdsStack) __threadfence_block();   // entries in the global overflow region
-      // accepted cells
-      const unsigned long long cm = __ballot(cell);
-      if (cell) cbuf[(ctail + lanes_below(cm)) & (CCAP - 1)] = node;
-      ctail += __popcll(cm);
-      ncell += __popcll(cm);
-      // direct particles
-      const int ecount = near ? ec : 0;
-      const int incl = wave_incl_scan(ecount);
-      const int tot = __shfl(incl, 63, 64);
-      for (int k = 0; k < ecount; k++) pbuf[(ptail + incl - ecount + k) & (PCAP - 1)] = ef + k;
-      ptail += tot;
-      nnear += tot;
+      if (cell) cbuf[(c0 + lanes_below(cm)) & (R::cells - 1)] = node;
+      for (int k = 0; k < ecount; k++) pbuf[(p0 + incl - ecount + k) & (R::parts - 1)] = ef + k;
       __syncthreads();
-      // evaluate full batches (and everything left once the walk is done)
-      while (ctail - chead >= kWave || (sp == 0 && ctail > chead)) {
-        const int nb = min(ctail - chead, kWave);
-        if (lane < nb) {
-          const int c = cbuf[(chead + lane) & (CCAP - 1)];
-          const double* m = a.mp + 10*(size_t) c;
-          double cx = m[0], cy = m[1], cz = m[2];
-          if (FAST) {
-#pragma clang fp contract(off)
-            // the cell relative to the expansion point, with the node test's replica
-            double dx = cx - gc.x, dy = cy - gc.y, dz = cz - gc.z;
-            nearest_image<double>(a.p, dx, dy, dz);
-            fast_add(fc, dx - rcx, dy - rcy, dz - rcz, m[3], m + 4,
-                     a.p.multipole == GDF_MULTIPOLE_FAST_QUADRUPOLE);
-          }
-          if (a.p.periodic) {
-            // nearest periodic replica of the cell relative to the group centre
-            double dx = cx - gc.x, dy = cy - gc.y, dz = cz - gc.z;
-            nearest_image<double>(a.p, dx, dy, dz);
-            cx = gc.x + dx; cy = gc.y + dy; cz = gc.z + dz;
-          }
-          const double qs = mono ? 0.0 : 1.0;      // monopole: no quadrupole moments
-          if (MIXED) {
-            s4a[lane] = make_float4((float) (cx - gc.x), (float) (cy - gc.y),
-                                    (float) (cz - gc.z), (float) m[3]);
-            s4b[lane] = make_float4((float) (qs*m[4]), (float) (qs*m[5]), (float) (qs*m[6]),
-                                    (float) (qs*m[7]));
-            s1[lane] = (float) (qs*m[8]);
-          } else {
-            sd[0][lane] = cx; sd[1][lane] = cy; sd[2][lane] = cz; sd[3][lane] = m[3];
-            for (int k = 4; k < 9; k++) sd[k][lane] = qs*m[k];
-          }
-        }
-        __syncthreads();
-        // fast multipoles leave only the periodic corrections to the per-target sweep
-        if (has && (!FAST || EWALD)) {
-          if (MIXED) {
-            float bx = 0.f, by = 0.f, bz = 0.f, bp = 0.f;
-            #pragma unroll 4
-            for (int q = 0; q < nb; q++) {
-              const float4 c = s4a[q], qa = s4b[q];
-              const float qq[5] = {qa.x, qa.y, qa.z, qa.w, s1[q]};
-              if (!FAST)
-                quad_term<float>(rxi - c.x, ryi - c.y, rzi - c.z, c.w, qq, bx, by, bz, bp,
-                                 PLUMMER ? eps2f : 1.0e-20f);
-              if (EWALD) ewald_corr<float>(a.p, c.x - rxi, c.y - ryi, c.z - rzi, c.w, bx, by, bz,
-                                           bp);
-            }
-            fx.add(bx); fy.add(by); fz.add(bz); fp.add(bp);
-          } else {
-            for (int q = 0; q < nb; q++) {
-              const double qq[5] = {sd[4][q], sd[5][q], sd[6][q], sd[7][q], sd[8][q]};
-              if (!FAST)
-                quad_term<double>(me.x - sd[0][q], me.y - sd[1][q], me.z - sd[2][q], sd[3][q],
-                                  qq, ax, ay, az, pot, PLUMMER ? eps2 : 1.0e-20);
-              if (EWALD) ewald_corr<double>(a.p, sd[0][q] - me.x, sd[1][q] - me.y,
-                                            sd[2][q] - me.z, sd[3][q], ax, ay, az, pot);
-            }
-          }
-        }
-        chead += nb;
-        __syncthreads();
+      // full batches, as many as the wavefronts share evenly; all that is left after the last
+      // round
+      const int cells = ctail - chead, parts = ptail - phead;
+      const int jc = sp == 0 ? (cells + kWave - 1)/kWave : cells/kWave;
+      int jobs = jc + (sp == 0 ? (parts + kWave - 1)/kWave : parts/kWave);
+      if (sp > 0) jobs -= jobs % W;
+      for (int j = wv; j < jobs; j += W) {
+        if (j < jc) eval_cells(chead + kWave*j, min(cells - kWave*j, kWave));
+        else eval_parts(phead + kWave*(j - jc), min(parts - kWave*(j - jc), kWave));
       }
-      while (ptail - phead >= kWave || (sp == 0 && ptail > phead)) {
-        const int nb = min(ptail - phead, kWave);
-        if (lane < nb) {
-          const int j = pbuf[(phead + lane) & (PCAP - 1)];
-          const double4 pj = a.posm[j];
-          const double4 rj = a.grec[j];
-          sidx[lane] = j;
-          if (MIXED) {
-            double dx = pj.x - gc.x, dy = pj.y - gc.y, dz = pj.z - gc.z;
-            nearest_image<double>(a.p, dx, dy, dz);
-            s4a[lane] = make_float4((float) dx, (float) dy, (float) dz, (float) pj.w);
-            s1[lane] = (float) range2_rn(krsqd, rj.x);
-            if (SOFT) s4b[lane] = make_float4((float) rj.x, (float) rj.y, (float) rj.z, 0.f);
-          } else {
-            sd[0][lane] = pj.x; sd[1][lane] = pj.y; sd[2][lane] = pj.z; sd[3][lane] = pj.w;
-            sd[4][lane] = range2_rn(krsqd, rj.x);
-            if (SOFT) { sd[5][lane] = rj.x; sd[6][lane] = rj.y; sd[7][lane] = rj.z; }
-          }
-        }
-        __syncthreads();
-        if (has) {
-          if (MIXED) {
-            const float hi = (float) mr.x, zi = (float) mr.y, hfi = (float) mr.z;
-            float bx = 0.f, by = 0.f, bz = 0.f, bp = 0.f;
-            // unrolled so that several LDS reads are in flight (same summation order)
-            #pragma unroll 8
-            for (int q = 0; q < nb; q++) {
-              // every record is loaded whatever the pair's branch: no LDS read under a mask
-              const float4 s = s4a[q];
-              const float r2j = s1[q];
-              const float dx = s.x - rxi, dy = s.y - ryi, dz = s.z - rzi;
-              const float d2 = dot3_f(dx, dy, dz);
-              const bool soft = (d2 < r2if) | (d2 < r2j);
-              if (PLUMMER) {
-                const float inv = rsq_f(d2 + eps2f);
-                const float mj = sidx[q] == i ? 0.f : s.w;
-                const float minv3 = mj*inv*inv*inv;
-                bx += minv3*dx; by += minv3*dy; bz += minv3*dz; bp += mj*inv;
-              } else if (SOFT) {
-                const float4 hq = s4b[q];
-                pair_fp32(K, d2, soft, dx, dy, dz, s.w, hi, hq.x, zi, hq.y, hfi, hq.z, bx, by,
-                          bz, bp);
-              } else {
-                const float inv = rsq_f(d2 + 1.0e-20f);
-                const float mj = soft ? 0.f : s.w;
-                const float minv3 = mj*inv*inv*inv;
-                bx += minv3*dx; by += minv3*dy; bz += minv3*dz; bp += mj*inv;
-              }
-              if (EWALD) ewald_corr<float>(a.p, dx, dy, dz, s.w, bx, by, bz, bp);
-            }
-            fx.add(bx); fy.add(by); fz.add(bz); fp.add(bp);
-          } else {
-            for (int q = 0; q < nb; q++) {
-              double dx = sd[0][q] - me.x, dy = sd[1][q] - me.y, dz = sd[2][q] - me.z;
-              nearest_image<double>(a.p, dx, dy, dz);
-              if (PLUMMER) {
-                const double inv = rsq_d(dot3_rn(dx, dy, dz) + eps2);
-                const double mj = sidx[q] == i ? 0.0 : sd[3][q];
-                const double minv3 = mj*inv*inv*inv;
-                ax += minv3*dx; ay += minv3*dy; az += minv3*dz; pot += mj*inv;
-              } else if (SOFT) {
-                pair_fp64(K, krsqd, dx, dy, dz, sd[3][q], mr.x, sd[5][q], mr.y, sd[6][q], mr.z,
-                          sd[7][q], ax, ay, az, pot);
-              } else {
-                const double d2 = dot3_rn(dx, dy, dz);
-                const bool soft = (d2 < r2i) | (d2 < sd[4][q]);
-                const double inv = rsq_d(d2 + 1.0e-20);
-                const double mj = soft ? 0.0 : sd[3][q];
-                const double minv3 = mj*inv*inv*inv;
-                ax += minv3*dx; ay += minv3*dy; az += minv3*dz; pot += mj*inv;
-              }
-              if (EWALD) ewald_corr<double>(a.p, dx, dy, dz, sd[3][q], ax, ay, az, pot);
-            }
-          }
-        }
-        phead += nb;
-        __syncthreads();
-      }
+      chead += min(cells, kWave*min(jobs, jc));
+      phead += min(parts, kWave*max(jobs - jc, 0));
     }
     if (overflow) {
-      if (lane == 0) atomicOr(&a.flags[2], 1);
+      if (threadIdx.x == 0) atomicOr(&a.flags[2], 1);
+      if (W > 1) __syncthreads();
       continue;
     }
+    if (MIXED) { ax = (double) fx.s; ay = (double) fy.s; az = (double) fz.s; pot = (double) fp.s; }
     if (FAST) {
       // the lanes' coefficient sums, reduced by a butterfly (every lane ends with the same sums)
       for (int k = 0; k < 10; k++) {
@@ -501,8 +551,28 @@ __global__ __launch_bounds__(64) void k_gravity(GravArgs a) {
         fc[k] = v;
       }
     }
-    if (has) {
-      if (MIXED) { ax = (double) fx.s; ay = (double) fy.s; az = (double) fz.s; pot = (double) fp.s; }
+    if (W > 1) {
+      // the wavefronts' sums, added in order by the first
+      double* red = &stage[0][0];
+      __syncthreads();
+      red[(4*wv + 0)*kWave + lane] = ax; red[(4*wv + 1)*kWave + lane] = ay;
+      red[(4*wv + 2)*kWave + lane] = az; red[(4*wv + 3)*kWave + lane] = pot;
+      double* redf = red + 4*kWave*W;
+      if (FAST && lane < 10) {
+        double v = 0.0;
+        for (int k = 0; k < 10; k++) v = lane == k ? fc[k] : v;
+        redf[10*wv + lane] = v;
+      }
+      __syncthreads();
+      if (wv == 0) {
+        for (int w = 1; w < W; w++) {
+          ax += red[(4*w + 0)*kWave + lane]; ay += red[(4*w + 1)*kWave + lane];
+          az += red[(4*w + 2)*kWave + lane]; pot += red[(4*w + 3)*kWave + lane];
+          if (FAST) for (int k = 0; k < 10; k++) fc[k] += redf[10*w + k];
+        }
+      }
+    }
+    if (has && wv == 0) {
       if (FAST) {
         // ApplyForcesTaylor (NeighbourSearch.h:735-760), first order about the expansion point
         const double* mG = a.mp + 10*(size_t) G;
@@ -512,6 +582,8 @@ __global__ __launch_bounds__(64) void k_gravity(GravArgs a) {
         az += fc[3] + fc[7]*d0 + fc[8]*d1 + fc[9]*d2;
         pot += fc[0] + fc[1]*d0 + fc[2]*d1 + fc[3]*d2;
       }
+      // the self term (m/h) wpot(0) (GradhSphTree.cpp:512)
+      const double pot0 = PLUMMER ? 0.0 : (me.w/mr.x)*kwpot<double>(K, 0.0);
       if (SOFT) {
         a.atx[i] = ax; a.aty[i] = ay; a.atz[i] = az;
         a.gpot[i] = pot0 + pot;
@@ -523,11 +595,11 @@ __global__ __launch_bounds__(64) void k_gravity(GravArgs a) {
         a.gpot[i] = pot0 + a.gpot[i] + pot;
       }
     }
-    if (lane == 0) {
-      a.gnc[g] = ncell;
-      a.gnn[g] = nnear;
-      atomicAdd((unsigned long long*) &a.icount[2], (unsigned long long) nnear*nact);
-      atomicAdd((unsigned long long*) &a.icount[3], (unsigned long long) ncell*(FAST ? 1 : nact));
+    if (threadIdx.x == 0) {
+      a.gnc[g] = ctail;
+      a.gnn[g] = ptail;
+      atomicAdd((unsigned long long*) &a.icount[2], (unsigned long long) ptail*nact);
+      atomicAdd((unsigned long long*) &a.icount[3], (unsigned long long) ctail*(FAST ? 1 : nact));
     }
   }
 }
@@ -725,13 +797,58 @@ int nbody_direct_stars(gdf_ctx* c, int smoothed) {
 
 namespace {
 
-// gas walks: the fast-multipole variant when the multipole option asks for it
-template <bool MIXED, bool SOFT, bool EWALD>
-void launch_gas(const GravArgs& a, int grid, hipStream_t s) {
-  if (a.p.multipole >= GDF_MULTIPOLE_FAST_MONOPOLE)
-    k_gravity<MIXED, SOFT, false, EWALD, true><<<grid, kWave, 0, s>>>(a);
-  else
-    k_gravity<MIXED, SOFT, false, EWALD, false><<<grid, kWave, 0, s>>>(a);
+// Wavefronts that share a walk group.  A group's walk is a chain of dependent loads, so while one
+// wavefront a group leaves SIMDs idle more of them finish sooner; with the device full they only
+// add barriers and partly filled rounds.  Walk (us) with 1, 2 and 4 wavefronts: 512 groups (20011
+// particles, FP64) 232 143 98, 1024 (FP64) 260 188 198, 2048 (FP32) 468 380 302, 2700 stars 397
+// 385 535; the whole force pass (ms): 4096 groups 2.88 2.73 2.81, 16384 10.3 10.6 11.1 (FP32),
+// 13.0 13.2 13.4 (FP64).  A serving batch keeps to two: a request's sums must not depend on what
+// else is resident.
+int grav_waves(const gdf_ctx* c) {
+  if (c->nseg > 0) return 2;
+  return c->ngroups <= 1024 ? 4 : c->ngroups <= 8192 ? 2 : 1;
+}
+
+template <bool MIXED, bool SOFT, bool PLUMMER, bool EWALD, bool FAST, int W>
+void launch_walk_w(const GravArgs& a, bool beside, hipStream_t s) {
+  // beside the hydro pass half the persistent wavefronts of a lone walk: at the full count they
+  // fill the CUs' LDS and the hydro pass waits for the walk to drain
+  const int most = (beside ? kGravSlots/2 : kGravSlots)/(W == 4 ? 2 : 1);
+  const int grid = std::min(a.ngroups, most);
+  k_gravity<MIXED, SOFT, PLUMMER, EWALD, FAST, W><<<grid, kWave*W, 0, s>>>(a);
+}
+
+// The walk's variant: stars, gas beside or after a hydro pass, or gas alone (SOFT); the options
+// off the main path (periodic corrections, fast multipoles, gas alone) take two wavefronts a group
+template <bool MIXED, bool SOFT>
+void launch_gas(const GravArgs& a, bool ewald, bool beside, int waves, hipStream_t s) {
+  const bool fast = a.p.multipole >= GDF_MULTIPOLE_FAST_MONOPOLE;
+  if (ewald) {
+    if (fast) launch_walk_w<MIXED, SOFT, false, true, true, 2>(a, beside, s);
+    else launch_walk_w<MIXED, SOFT, false, true, false, 2>(a, beside, s);
+  } else if (fast) {
+    launch_walk_w<MIXED, SOFT, false, false, true, 2>(a, beside, s);
+  } else if (SOFT || waves == 2) {
+    launch_walk_w<MIXED, SOFT, false, false, false, 2>(a, beside, s);
+  } else if (waves == 4) {
+    launch_walk_w<MIXED, SOFT, false, false, false, SOFT ? 2 : 4>(a, beside, s);
+  } else {
+    launch_walk_w<MIXED, SOFT, false, false, false, SOFT ? 2 : 1>(a, beside, s);
+  }
+}
+
+template <bool MIXED>
+void launch_grav(const gdf_ctx* c, const GravArgs& a, bool beside, hipStream_t s) {
+  const int waves = grav_waves(c);
+  if (c->phys.nbody) {
+    if (waves == 4) launch_walk_w<MIXED, true, true, false, false, 4>(a, beside, s);
+    else if (waves == 2) launch_walk_w<MIXED, true, true, false, false, 2>(a, beside, s);
+    else launch_walk_w<MIXED, true, true, false, false, 1>(a, beside, s);
+  } else if (c->phys.hydro_forces) {
+    launch_gas<MIXED, false>(a, c->phys.ewald, beside, waves, s);
+  } else {
+    launch_gas<MIXED, true>(a, c->phys.ewald, beside, waves, s);
+  }
 }
 
 GravArgs grav_args(gdf_ctx* c) {
@@ -790,18 +907,10 @@ int gravity_launch(gdf_ctx* c) {
     k_zero8<<<1, 64, 0, s2>>>(c->counters + 24);
     k_zero8<<<1, 64, 0, s2>>>(c->counters + 16);
   }
-  // half the persistent wavefronts of a lone walk: at the full count they fill every CU's LDS
-  // and the scatter-gather walk beside them waits for the gravity walk to drain
-  const int grid = std::min(c->ngroups, kGravSlots/2);
   const int kt = ktime_begin(c, s2, 5);
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
-  if (c->phys.ewald) {
-    if (mixed) launch_gas<true, false, true>(a, grid, s2);
-    else launch_gas<false, false, true>(a, grid, s2);
-  } else {
-    if (mixed) launch_gas<true, false, false>(a, grid, s2);
-    else launch_gas<false, false, false>(a, grid, s2);
-  }
+  if (mixed) launch_grav<true>(c, a, true, s2);
+  else launch_grav<false>(c, a, true, s2);
   GDF_HIP(c, hipGetLastError());
   ktime_end(c, s2, kt);
   GDF_HIP(c, hipMemcpyAsync(c->h_counters + 16, c->counters + 16, sizeof(int)*8,
@@ -838,27 +947,10 @@ int gravity_walk(gdf_ctx* c) {
     k_zero8<<<1, 64, 0, s>>>(c->counters);
   }
   GDF_TRY(rc);
-  const int grid = std::min(c->ngroups, kGravSlots);
   const int kt = ktime_begin(c, s, 5);
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
-  if (c->phys.nbody) {
-    if (mixed) k_gravity<true, true, true><<<grid, kWave, 0, s>>>(a);
-    else k_gravity<false, true, true><<<grid, kWave, 0, s>>>(a);
-  } else if (c->phys.hydro_forces) {
-    if (c->phys.ewald) {
-      if (mixed) launch_gas<true, false, true>(a, grid, s);
-      else launch_gas<false, false, true>(a, grid, s);
-    } else {
-      if (mixed) launch_gas<true, false, false>(a, grid, s);
-      else launch_gas<false, false, false>(a, grid, s);
-    }
-  } else if (c->phys.ewald) {
-    if (mixed) launch_gas<true, true, true>(a, grid, s);
-    else launch_gas<false, true, true>(a, grid, s);
-  } else {
-    if (mixed) launch_gas<true, true, false>(a, grid, s);
-    else launch_gas<false, true, false>(a, grid, s);
-  }
+  if (mixed) launch_grav<true>(c, a, false, s);
+  else launch_grav<false>(c, a, false, s);
   GDF_HIP(c, hipGetLastError());
   ktime_end(c, s, kt);
   GDF_HIP(c, hipMemcpyAsync(c->h_counters, c->counters, sizeof(int)*8, hipMemcpyDeviceToHost, s));

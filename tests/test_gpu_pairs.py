@@ -73,6 +73,17 @@ def test_cloud_passes_match_oracle(N, gmax, kern, precision):
     check(g, precision, gmax, True)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_gravity_walk_of_many_groups_matches_oracle(precision):
+    """More than 8192 walk groups: one wavefront a group in the gravity walk (the clouds above
+    have two and four)."""
+    g = ICS.rotating_m2_cloud(N=17011, seed=12)
+    g["params"].update(kernel="m4", thetamaxsqd=1e-12, gas_eos="energy_eqn")
+    s = passes(g, precision, 2)
+    assert s.tree_arrays()["group_first"].size > 8192
+    check(g, precision, 2, True)
+
+
 # The mixed path takes a candidate's image about the group's centre for all of its targets, so it
 # has no cases where a group's extent and range pass half the box, and none with the tabulated
 # kernel, where a lattice's nearly cancelling sums leave no bound on the effect of a shifted entry.

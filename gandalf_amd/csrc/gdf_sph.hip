@@ -38,6 +38,8 @@ constexpr double NODE_SLACK = 1.0 + 1e-12; // node tests err on the inclusive si
 // target's own test (FP32 tests of the mixed path included)
 constexpr double KEEP_SLACK = 1.0 + 1e-4;
 constexpr int kInitBatches = 16;           // initial candidate capacity per group, in batches
+constexpr int kMaxRounds = 64;             // search radii tried for a particle's h
+constexpr double kMaxGrowth = 23.26;       // between 1.05^64 and 1.05^65: beyond the last of them
 
 struct CandWalk {
   int N, ngroups, nleaf, capb;
@@ -468,7 +470,9 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
         state = 1;
       } else if (rc == 0) {
         if (wv == 0) {
-          a.hsearch[i] = hmax*1.05;     // GradhSphTree.cpp:154: hmax = 1.05 hmax per retry
+          // a larger search radius (k_hrho_finish, status 3) for an h past this one's
+          a.hfactor[i] = h;
+          a.status[i] = 3;
           atomicAdd(&a.flags[0], 1);
         }
         state = 0;
@@ -499,10 +503,25 @@ void launch_density(const DensArgs& d, int waves, hipStream_t s) {
 }
 
 // Final h, grad-h terms and EOS of the particles the h-rho pass has just converged (status 2:
-// rho, invomega and zeta hold the sums at the converged h, hfactor the bracket's lower end)
+// rho, invomega and zeta hold the sums at the converged h, hfactor the bracket's lower end), and
+// the next search radius of those that need one (status 3: hfactor holds the h that was past it)
 __global__ void k_hrho_finish(DensArgs a) {
   const int i = blockIdx.x*BS + threadIdx.x;
-  if (i >= a.N || a.status[i] != 2) return;
+  if (i >= a.N || a.status[i] < 2) return;
+  if (a.status[i] == 3) {
+    // GradhSphTree.cpp:154: hmax = 1.05 hmax per retry, here at once as often as it takes to reach
+    // the h that was past it: the iteration starts again from the same h and comes back to it, so
+    // the retries on the way would end where the last one did.  (An h of a first guess takes two
+    // or three instead of up to ten: six spheres set up and served 38.4 -> 36.8 ms.)
+    const double h = a.hfactor[i];
+    double hs = a.hsearch[i]*1.05;
+    for (int k = 0; k < kMaxRounds && hs < h; k++) hs *= 1.05;
+    a.hsearch[i] = hs;
+    a.status[i] = 1;
+    // past the last radius that a round each would try
+    if (hs > kMaxGrowth*a.h[i]) atomicOr(&a.flags[3], 4);
+    return;
+  }
   hrho_finish(a, a.p, i, a.posm[i].w, a.rho[i], a.invomega[i], a.zeta[i], a.hfactor[i]);
   a.status[i] = 0;
   // a final h past the search radius (h from rho after the convergence test can exceed it by
@@ -967,7 +986,7 @@ int sph_density(gdf_ctx* c, int nopbc) {
   const bool uni = !nopbc;
   const WalkKind kind = uni ? WALK_UNION : WALK_GATHER;
   bool grown = false, retried = false, outgrown = false;
-  for (int round = 0; round < 64; round++) {
+  for (int round = 0; round < kMaxRounds; round++) {
     // also clears the round's flags and the walk's queue counters
     GDF_TRY(group_list(c, c->status, c->glist, c->cs_g.ncand, nullptr, nullptr, c->counters,
                        12));
@@ -981,6 +1000,7 @@ int sph_density(gdf_ctx* c, int nopbc) {
     const int* f = c->h_counters;
     if (f[2]) return fail(c, GDF_ERR_CAPACITY, "tree walk stack overflow in gather pass");
     if (f[3] & 1) return fail(c, GDF_ERR_NOCONV, "Problem with convergence of h-rho iteration");
+    if (f[3] & 4) break;
     outgrown = outgrown || (f[3] & 2);
     retried = retried || f[0] > 0;
     // groups whose candidates overflowed skipped the density kernel and keep status 1

@@ -247,9 +247,7 @@ int ctx_get_field_range(gdf_ctx* c, const char* name, int i0, int n, double* out
                                                       p[2] ? p[2] + i0 : nullptr, c->iorig + i0,
                                                       c->tmpd);
   GDF_HIP(c, hipGetLastError());
-  GDF_HIP(c, hipMemcpyAsync(out, c->tmpd, sizeof(double)*w*(size_t) n, hipMemcpyDeviceToHost, c->stream));
-  GDF_HIP(c, hipStreamSynchronize(c->stream));
-  return GDF_OK;
+  return xfer_out(c, out, c->tmpd, (size_t) w*n);
 }
 
 int ctx_field_width(gdf_ctx* c, const char* name) {
@@ -423,6 +421,7 @@ void gdf_destroy(gdf_ctx* c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   free_particles(c);
   stars_free(c);
+  if (c->xfer) hipHostFree(c->xfer);
   if (c->counters) hipFree(c->counters);
   if (c->icount) hipFree(c->icount);
   if (c->red) hipFree(c->red);
@@ -458,30 +457,27 @@ int gdf_set_particles(gdf_ctx* c, int N, const double* r, const double* v, const
   if (N <= 0 || !r || !v || !m || !u) return fail(c, GDF_ERR_INVALID, "gdf_set_particles: bad arguments");
   if ((long long) N > (1LL << 30)) return fail(c, GDF_ERR_INVALID, "too many particles");
   c->snap_porig.clear();
-  for (int i = 0; i < N; i++)
-    if (!(m[i] > 0.0)) return fail(c, GDF_ERR_INVALID, "particle masses must be positive");
+  bool positive = true;
+  for (int i = 0; i < N; i++) positive &= m[i] > 0.0;
+  if (!positive) return fail(c, GDF_ERR_INVALID, "particle masses must be positive");
   if (N > c->Ncap) GDF_TRY(alloc_particles(c, N));
   c->N = N;
   const size_t n = (size_t) N;
-  std::vector<double> col(n);
-  auto up = [&](double* dst, const double* src, int stride, int off) -> int {
-    for (size_t i = 0; i < n; i++) col[i] = src ? src[i*stride + off] : 0.0;
-    GDF_HIP(c, hipMemcpy(dst, col.data(), sizeof(double)*n, hipMemcpyHostToDevice));
-    return GDF_OK;
+  ColSet z;
+  for (int f : {F_AX0, F_AY0, F_AZ0, F_DUDT0, F_TLAST, F_PDT, F_DTNEXT}) z.add(c->pf[f]);
+  if (!h) z.add(c->pf[F_H]);
+  for (int f = 0; f < D_NDERIVED; f++) z.add(c->df[f]);
+  for (int f = 0; f < I_NINT; f++) z.add(c->pi[f]);
+  GDF_TRY(cols_zero(c, z, N));
+  auto vec = [&](int a, int b) {
+    return XferCols{3, {c->pf[a], c->pf[a + 1], c->pf[a + 2]}, {c->pf[b], c->pf[b + 1], c->pf[b + 2]}};
   };
-  for (int k = 0; k < 3; k++) {
-    GDF_TRY(up(c->pf[F_X + k], r, 3, k)); GDF_TRY(up(c->pf[F_X0 + k], r, 3, k));
-    GDF_TRY(up(c->pf[F_VX + k], v, 3, k)); GDF_TRY(up(c->pf[F_VX0 + k], v, 3, k));
-    GDF_TRY(up(c->pf[F_AX0 + k], nullptr, 1, 0));
-  }
-  GDF_TRY(up(c->pf[F_M], m, 1, 0));
-  GDF_TRY(up(c->pf[F_H], h, 1, 0));
-  GDF_TRY(up(c->pf[F_U], u, 1, 0));
-  GDF_TRY(up(c->pf[F_U0], u, 1, 0));
-  GDF_TRY(up(c->pf[F_DUDT0], nullptr, 1, 0));
-  for (int f : {F_TLAST, F_PDT, F_DTNEXT}) GDF_TRY(up(c->pf[f], nullptr, 1, 0));
-  for (int f = 0; f < D_NDERIVED; f++) GDF_HIP(c, hipMemset(c->df[f], 0, sizeof(double)*n));
-  for (int f = 0; f < I_NINT; f++) GDF_HIP(c, hipMemset(c->pi[f], 0, sizeof(int)*n));
+  auto col = [&](int a, double* b) { return XferCols{1, {c->pf[a], nullptr, nullptr}, {b, nullptr, nullptr}}; };
+  GDF_TRY(xfer_in(c, r, 3*n, vec(F_X, F_X0)));
+  GDF_TRY(xfer_in(c, v, 3*n, vec(F_VX, F_VX0)));
+  GDF_TRY(xfer_in(c, m, n, col(F_M, nullptr)));
+  GDF_TRY(xfer_in(c, u, n, col(F_U, c->pf[F_U0])));
+  if (h) GDF_TRY(xfer_in(c, h, n, col(F_H, nullptr)));
   k_iota<<<nblocks(N, BS), BS, 0, c->stream>>>(N, c->iorig);
   GDF_HIP(c, hipStreamSynchronize(c->stream));
   c->tree_valid = false; c->topo_valid = false; c->sg_valid = false; c->sg_union = false; c->setup_done = false;
@@ -498,16 +494,12 @@ int gdf_get_field(gdf_ctx* c, const char* name, double* out) {
   if (fi >= 0) {
     k_scatter_out_int<<<nblocks(c->N, BS), BS, 0, c->stream>>>(c->N, c->pi[fi], c->iorig, c->tmpd);
     GDF_HIP(c, hipGetLastError());
-    GDF_HIP(c, hipMemcpyAsync(out, c->tmpd, sizeof(double)*(size_t) c->N, hipMemcpyDeviceToHost, c->stream));
-    GDF_HIP(c, hipStreamSynchronize(c->stream));
-    return GDF_OK;
+    return xfer_out(c, out, c->tmpd, (size_t) c->N);
   }
   if (!field_ptrs(c, name, p, &w)) return fail(c, GDF_ERR_INVALID, std::string("unknown field ") + name);
   k_scatter_out<<<nblocks(c->N, BS), BS, 0, c->stream>>>(c->N, w, p[0], p[1], p[2], c->iorig, c->tmpd);
   GDF_HIP(c, hipGetLastError());
-  GDF_HIP(c, hipMemcpyAsync(out, c->tmpd, sizeof(double)*w*(size_t) c->N, hipMemcpyDeviceToHost, c->stream));
-  GDF_HIP(c, hipStreamSynchronize(c->stream));
-  return GDF_OK;
+  return xfer_out(c, out, c->tmpd, (size_t) w*c->N);
 }
 
 int gdf_set_field(gdf_ctx* c, const char* name, const double* in) {
@@ -517,15 +509,14 @@ int gdf_set_field(gdf_ctx* c, const char* name, const double* in) {
   int w = 0;
   const int fi = int_field(name);
   if (fi >= 0) {
-    GDF_HIP(c, hipMemcpyAsync(c->tmpd, in, sizeof(double)*(size_t) c->N, hipMemcpyHostToDevice,
-                              c->stream));
+    GDF_TRY(xfer_in(c, in, (size_t) c->N, XferCols{1, {c->tmpd}, {}}, false));
     k_gather_in_int<<<nblocks(c->N, BS), BS, 0, c->stream>>>(c->N, c->pi[fi], c->iorig, c->tmpd);
     GDF_HIP(c, hipGetLastError());
     GDF_HIP(c, hipStreamSynchronize(c->stream));
     return GDF_OK;
   }
   if (!field_ptrs(c, name, p, &w)) return fail(c, GDF_ERR_INVALID, std::string("unknown field ") + name);
-  GDF_HIP(c, hipMemcpyAsync(c->tmpd, in, sizeof(double)*w*(size_t) c->N, hipMemcpyHostToDevice, c->stream));
+  GDF_TRY(xfer_in(c, in, (size_t) w*c->N, XferCols{1, {c->tmpd}, {}}, false));
   k_gather_in<<<nblocks(c->N, BS), BS, 0, c->stream>>>(c->N, w, p[0], p[1], p[2], c->iorig, c->tmpd);
   GDF_HIP(c, hipGetLastError());
   GDF_HIP(c, hipStreamSynchronize(c->stream));

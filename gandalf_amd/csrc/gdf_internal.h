@@ -191,6 +191,8 @@ struct gdf_ctx {
   double* red = nullptr;       // reduction partials
   double* h_red = nullptr;     // pinned
   double* tmpd = nullptr;      // scratch N*3 doubles for field export
+  double* xfer = nullptr;      // pinned staging of the transfers to and from the caller's memory
+                               // (2 MB, made by the first of them)
 
   // kernel tables
   double* ktab = nullptr; float* ktabf = nullptr;
@@ -292,6 +294,25 @@ void ktime_collect(gdf_ctx* c);
 int group_list(gdf_ctx* c, const int* status, int* list, int* ncand, int* gnc, int* gnn,
                int* zero = nullptr, int nzero = 0);
 TreeView tree_view(const gdf_ctx* c);
+
+// transfers and column fills (gdf_xfer.hip)
+struct XferCols {            // w interleaved components go to columns a[k], and to b[k] where set
+  int w;
+  double* a[3]; double* b[3];
+};
+struct ColSet {              // nd columns of doubles, ni of integers
+  int nd = 0, ni = 0;
+  double* d[64]; int* i[16];
+  void add(double* p) { d[nd++] = p; }
+  void add(int* p) { i[ni++] = p; }
+};
+static_assert(F_NPERSIST + D_NDERIVED <= 64 && I_NINT + 1 <= 16, "ColSet holds every column");
+// n doubles between the device and the caller's memory; both return when the copy is complete, or
+// with wait = false when it is in the stream, which the caller then waits for before it returns
+int xfer_out(gdf_ctx* c, double* out, const double* dev, size_t n);
+int xfer_in(gdf_ctx* c, const double* in, size_t n, const XferCols& to, bool wait = true);
+int cols_zero(gdf_ctx* c, const ColSet& s, int n);
+int cols_copy(gdf_ctx* c, const ColSet& to, const ColSet& from, int n);
 
 // SPH passes (gdf_sph.hip)
 int sph_alloc_lists(gdf_ctx* c);

@@ -70,6 +70,14 @@ int pool_ctx_fail(gdf_pool* P, gdf_ctx* c, int rc) {
   return rc;
 }
 
+// the persistent columns and the original indices from particle i0 on
+ColSet persistent(gdf_ctx* c, int i0) {
+  ColSet s;
+  for (int f = 0; f < F_NPERSIST; f++) s.add(c->pf[f] + i0);
+  s.add(c->iorig + i0);
+  return s;
+}
+
 // Fault injection for the failure-path tests: with GDF_FAULT_POOL_GROW=1 in the environment,
 // growing a batch reports an allocation failure after the grown arrays were allocated (the
 // state a failed hipMalloc part way through leaves behind).
@@ -114,22 +122,21 @@ int batch_reserve(gdf_ctx* c, int need, int64_t maxp, bool* lost) {
     }
     ncap = old_cap;
   }
-  hipError_t e = hipSuccess;
   // derived fields a class never computes (density of N-body) read 0
-  for (int f = 0; f < D_NDERIVED && e == hipSuccess; f++)
-    e = hipMemsetAsync(c->df[f], 0, sizeof(double)*ncap, c->stream);
-  if (N > 0) {
-    for (int f = 0; f < F_NPERSIST && e == hipSuccess; f++)
-      e = hipMemcpyAsync(c->pf[f], keep[f], sizeof(double)*N, hipMemcpyDeviceToDevice,
-                         c->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(c->iorig, keep_io, sizeof(int)*N, hipMemcpyDeviceToDevice, c->stream);
+  ColSet z;
+  for (int f = 0; f < D_NDERIVED; f++) z.add(c->df[f]);
+  int moved = cols_zero(c, z, ncap);
+  if (N > 0 && moved == GDF_OK) {
+    ColSet to = persistent(c, 0), from;
+    for (int f = 0; f < F_NPERSIST; f++) from.add(keep[f]);
+    from.add(keep_io);
+    moved = cols_copy(c, to, from, N);
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  const hipError_t e = hipStreamSynchronize(c->stream);
   release_kept();
-  if (e != hipSuccess) {
+  if (e != hipSuccess || moved != GDF_OK) {
     *lost = true;
-    return check_hip(c, e, "batch grow: copying the resident state");
+    return e != hipSuccess ? check_hip(c, e, "batch grow: copying the resident state") : moved;
   }
   c->N = N;
   // the new integer arrays need the resident segments' ids again
@@ -145,20 +152,15 @@ int batch_reserve(gdf_ctx* c, int need, int64_t maxp, bool* lost) {
 int batch_compact(gdf_ctx* c, const std::vector<int>& keep) {
   std::vector<int> off(1, 0);
   for (int sg : keep) off.push_back(off.back() + c->seg_off[sg + 1] - c->seg_off[sg]);
-  for (int f = 0; f <= F_NPERSIST; f++) {
-    double* src = f < F_NPERSIST ? c->pf[f] : nullptr;
-    for (size_t k = 0; k < keep.size(); k++) {
-      const int sg = keep[k], n = c->seg_off[sg + 1] - c->seg_off[sg];
-      if (f < F_NPERSIST)
-        GDF_HIP(c, hipMemcpyAsync(c->pf_alt[f] + off[k], src + c->seg_off[sg],
-                                  sizeof(double)*n, hipMemcpyDeviceToDevice, c->stream));
-      else
-        GDF_HIP(c, hipMemcpyAsync(c->iorig_alt + off[k], c->iorig + c->seg_off[sg],
-                                  sizeof(int)*n, hipMemcpyDeviceToDevice, c->stream));
-    }
-    if (f < F_NPERSIST) std::swap(c->pf[f], c->pf_alt[f]);
-    else std::swap(c->iorig, c->iorig_alt);
+  for (size_t k = 0; k < keep.size(); k++) {
+    const int sg = keep[k];
+    ColSet to;
+    for (int f = 0; f < F_NPERSIST; f++) to.add(c->pf_alt[f] + off[k]);
+    to.add(c->iorig_alt + off[k]);
+    GDF_TRY(cols_copy(c, to, persistent(c, c->seg_off[sg]), c->seg_off[sg + 1] - c->seg_off[sg]));
   }
+  for (int f = 0; f < F_NPERSIST; f++) std::swap(c->pf[f], c->pf_alt[f]);
+  std::swap(c->iorig, c->iorig_alt);
   c->N = off.back();
   c->seg_off = off;
   c->nseg = (int) keep.size();
@@ -275,12 +277,7 @@ int gdf_pool_admit(gdf_pool* P, int N, const double* r, const double* v, const d
     return pool_ctx_fail(P, c, rc);
   }
   if (rc == GDF_OK) {
-    for (int f = 0; f < F_NPERSIST && rc == GDF_OK; f++)
-      if (hipMemcpyAsync(c->pf[f] + N0, sc->pf[f], sizeof(double)*N, hipMemcpyDeviceToDevice,
-                         c->stream) != hipSuccess) rc = GDF_ERR_HIP;
-    if (rc == GDF_OK && hipMemcpyAsync(c->iorig + N0, sc->iorig, sizeof(int)*N,
-                                       hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
-      rc = GDF_ERR_HIP;
+    rc = cols_copy(c, persistent(c, N0), persistent(sc, 0), N);
   }
   PoolReq q;
   q.id = P->next_id; q.N = N; q.nsteps = nsteps; q.done = 0;

@@ -101,7 +101,7 @@ void free_particles(gdf_ctx* c) {
   for (int f = 0; f < I_NINT; f++) { hipFree(c->pi[f]); hipFree(c->pi_alt[f]); c->pi[f] = c->pi_alt[f] = nullptr; }
   void* ptrs[] = {c->iorig, c->iorig_alt, c->posm, c->hrecA, c->hrecB, c->grec, c->status,
                   c->keys, c->keys_alt, c->vals, c->vals_alt, c->sort_tmp, c->left, c->right,
-                  c->first, c->last, c->parent, c->lnk, c->visit, c->front, c->bbmin, c->bbmax, c->geo_c,
+                  c->first, c->last, c->parent, c->lnk, c->visit, c->front, c->geo_c,
                   c->geo_h, c->mp, c->gstart, c->grp_first, c->grp_count, c->grp_node, c->nsel,
                   c->sel_tmp, c->stacks, c->grav_nc,
                   c->grav_nn, c->tmpd, c->grp_root, c->stacks2, c->glist, c->grp_gmac};
@@ -110,7 +110,7 @@ void free_particles(gdf_ctx* c) {
   c->status = nullptr; c->keys = c->keys_alt = nullptr; c->vals = c->vals_alt = nullptr;
   c->sort_tmp = nullptr; c->left = c->right = c->first = c->last = c->parent = c->visit = c->front = nullptr;
   c->lnk = nullptr;
-  c->bbmin = c->bbmax = nullptr; c->geo_c = c->geo_h = nullptr; c->mp = nullptr;
+  c->geo_c = c->geo_h = nullptr; c->mp = nullptr;
   c->gstart = c->grp_first = c->grp_count = c->grp_node = c->nsel = nullptr; c->sel_tmp = nullptr;
   c->stacks = nullptr;
   sph_free_lists(c);
@@ -687,17 +687,18 @@ int gdf_tree_arrays(gdf_ctx* c, int32_t* perm, uint64_t* keys, int32_t* left, in
     if (first) GDF_HIP(c, hipMemcpy(first, c->first, sizeof(int)*ni, hipMemcpyDeviceToHost));
     if (last) GDF_HIP(c, hipMemcpy(last, c->last, sizeof(int)*ni, hipMemcpyDeviceToHost));
   }
-  std::vector<double> mpv(10*nn);
-  if (mass || com || quad) {
-    GDF_HIP(c, hipMemcpy(mpv.data(), c->mp, sizeof(double)*10*nn, hipMemcpyDeviceToHost));
+  if (mass || com || quad || bbmin || bbmax) {
+    std::vector<double> mpv(kMom*nn);
+    GDF_HIP(c, hipMemcpy(mpv.data(), c->mp, sizeof(double)*kMom*nn, hipMemcpyDeviceToHost));
     for (size_t n = 0; n < nn; n++) {
-      if (mass) mass[n] = mpv[10*n + 3];
-      if (com) for (int k = 0; k < 3; k++) com[3*n + k] = mpv[10*n + k];
-      if (quad) for (int k = 0; k < 5; k++) quad[5*n + k] = mpv[10*n + 4 + k];
+      const double* r = mpv.data() + kMom*n;
+      if (mass) mass[n] = r[3];
+      if (com) for (int k = 0; k < 3; k++) com[3*n + k] = r[k];
+      if (quad) for (int k = 0; k < 5; k++) quad[5*n + k] = r[4 + k];
+      if (bbmin) for (int k = 0; k < 3; k++) bbmin[3*n + k] = r[10 + k];
+      if (bbmax) for (int k = 0; k < 3; k++) bbmax[3*n + k] = r[13 + k];
     }
   }
-  if (bbmin) GDF_HIP(c, hipMemcpy(bbmin, c->bbmin, sizeof(double)*3*nn, hipMemcpyDeviceToHost));
-  if (bbmax) GDF_HIP(c, hipMemcpy(bbmax, c->bbmax, sizeof(double)*3*nn, hipMemcpyDeviceToHost));
   if (hmax) {
     std::vector<double4> gc(nn);
     GDF_HIP(c, hipMemcpy(gc.data(), c->geo_c, sizeof(double4)*nn, hipMemcpyDeviceToHost));

@@ -276,7 +276,7 @@ __global__ __launch_bounds__(64*W, EWALD || FAST || (SOFT && !PLUMMER) ? 2 : 3) 
     double fc[10];
     if (FAST) {
 #pragma clang fp contract(off)
-      const double* mG = a.mp + 10*(size_t) G;
+      const double* mG = a.mp + kMom*(size_t) G;
       rcx = mG[0] - gc.x; rcy = mG[1] - gc.y; rcz = mG[2] - gc.z;
       const double ex = fabs(rcx) + gh.x, ey = fabs(rcy) + gh.y, ez = fabs(rcz) + gh.z;
       rg2t = (ex*ex + ey*ey + ez*ez)/a.p.thetamaxsqd;
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(64*W, EWALD || FAST || (SOFT && !PLUMMER) ? 2 : 3) 
     auto eval_cells = [&](int c0, int nb) {
       if (lane < nb) {
         const int c = cbuf[(c0 + lane) & (R::cells - 1)];
-        const double* m = a.mp + 10*(size_t) c;
+        const double* m = a.mp + kMom*(size_t) c;
         double cx = m[0], cy = m[1], cz = m[2];
         if (FAST) {
 #pragma clang fp contract(off)
@@ -479,9 +479,9 @@ __global__ __launch_bounds__(64*W, EWALD || FAST || (SOFT && !PLUMMER) ? 2 : 3) 
           const double ez = fmax(fabs(dz) - gh.z, 0.0);
           const double dmac2 = ex*ex + ey*ey + ez*ez;
           bool accept = dmac2 >= nh.w;
-          if (gmac && accept) accept = !mac_opens(a.p, nh, a.mp + 10*(size_t) node, dmac2, gfac);
+          if (gmac && accept) accept = !mac_opens(a.p, nh, a.mp + kMom*(size_t) node, dmac2, gfac);
           if (FAST && accept) {
-            const double* mc = a.mp + 10*(size_t) node;
+            const double* mc = a.mp + kMom*(size_t) node;
             double cx = mc[0] - gc.x, cy = mc[1] - gc.y, cz = mc[2] - gc.z;
             nearest_image<double>(a.p, cx, cy, cz);
             cx -= rcx; cy -= rcy; cz -= rcz;
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(64*W, EWALD || FAST || (SOFT && !PLUMMER) ? 2 : 3) 
     if (has && wv == 0) {
       if (FAST) {
         // ApplyForcesTaylor (NeighbourSearch.h:735-760), first order about the expansion point
-        const double* mG = a.mp + 10*(size_t) G;
+        const double* mG = a.mp + kMom*(size_t) G;
         const double d0 = me.x - mG[0], d1 = me.y - mG[1], d2 = me.z - mG[2];
         ax += fc[1] + fc[4]*d0 + fc[5]*d1 + fc[7]*d2;
         ay += fc[2] + fc[5]*d0 + fc[6]*d1 + fc[8]*d2;

@@ -231,11 +231,6 @@ __global__ void k_diag_final(int nb, const double* __restrict__ part, int hydro,
   out[10] = acc[0];
 }
 
-__global__ void k_zero_d(int n, double* __restrict__ p) {
-  const int i = blockIdx.x*BS + threadIdx.x;
-  if (i < n) p[i] = 0.0;
-}
-
 __global__ void k_fill_i(int n, int* __restrict__ p, int v) {
   const int i = blockIdx.x*BS + threadIdx.x;
   if (i < n) p[i] = v;
@@ -432,9 +427,9 @@ int integ_zero_accelerations(gdf_ctx* c) {
 int integ_zero_forces(gdf_ctx* c) {
   const int n = c->N;
   const int fields[] = {D_AX, D_AY, D_AZ, D_ATX, D_ATY, D_ATZ, D_DUDT, D_DIVV, D_GPOT};
-  for (int f : fields) k_zero_d<<<nblocks(n, BS), BS, 0, c->stream>>>(n, c->df[f]);
-  GDF_HIP(c, hipGetLastError());
-  return GDF_OK;
+  ColSet z;
+  for (int f : fields) z.add(c->df[f]);
+  return cols_zero(c, z, n);
 }
 
 int integ_add_atree(gdf_ctx* c) {

@@ -101,8 +101,12 @@ struct TreeView {
   const int* left; const int* right; const int* first; const int* last;
   const double4* geo_c;   // (cx, cy, cz, hmax)
   const double4* geo_h;   // (hx, hy, hz, cdistsqd)
-  const double* mp;       // 10 doubles per node: comx comy comz m q0..q4 pad
+  const double* mp;       // kMom doubles per node
 };
+
+// A node's record, one 128-byte line: centre of mass, mass, quadrupole (xx, xy, yy, xz, yz), the
+// bound on h at the last full refit, box corners (low x y z, high x y z)
+constexpr int kMom = 16;
 
 // Candidate set of the SPH passes, per walk group g: idx[g][k] is candidate k in walk order,
 // ncand[g] their number; capb*64 are reserved per group.  The parity tap's set also holds
@@ -147,9 +151,8 @@ struct gdf_ctx {
   int* parent = nullptr; int* visit = nullptr;
   int4* lnk = nullptr;          // internal node: (first, last, left, right) in one 16-byte record
   int* front = nullptr;                                // refit frontier [N] + count
-  double* bbmin = nullptr; double* bbmax = nullptr;     // 3 per node
   double4* geo_c = nullptr; double4* geo_h = nullptr;
-  double* mp = nullptr;                                // 10 per node
+  double* mp = nullptr;                                // kMom per node
   int* gstart = nullptr;                               // per-slot group-start marker
   int* grp_first = nullptr; int* grp_count = nullptr; int* grp_node = nullptr;
   int* nsel = nullptr; void* sel_tmp = nullptr; size_t sel_tmp_bytes = 0;

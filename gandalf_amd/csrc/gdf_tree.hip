@@ -14,6 +14,7 @@
 
 #include "gdf_internal.h"
 #include "gdf_device.h"
+#include "gdf_filter.h"
 
 namespace gdf {
 namespace {
@@ -303,7 +304,7 @@ __global__ void k_lbvh(int N, const uint64_t* __restrict__ key, int* __restrict_
 }
 
 struct NodeArgs {
-  double* bbmin; double* bbmax; double4* geo_c; double4* geo_h; double* mp;
+  double4* geo_c; double4* geo_h; double* mp;
 };
 
 __global__ void k_leaves(int N, const double* __restrict__ x, const double* __restrict__ y,
@@ -316,10 +317,12 @@ __global__ void k_leaves(int N, const double* __restrict__ x, const double* __re
   if (N == 1) parent[0] = -1;
   const int n = N - 1 + l;
   const double r[3] = {x[l], y[l], z[l]};
-  for (int k = 0; k < 3; k++) { a.bbmin[3*n+k] = r[k]; a.bbmax[3*n+k] = r[k]; a.mp[10*n+k] = r[k]; }
-  a.mp[10*n+3] = m[l];
-  for (int k = 4; k < 10; k++) a.mp[10*n+k] = 0.0;
   const double hh = h[l];
+  double* mp = a.mp + (size_t) kMom*n;
+  for (int k = 0; k < 3; k++) mp[k] = mp[10 + k] = mp[13 + k] = r[k];
+  mp[3] = m[l];
+  for (int k = 4; k < 9; k++) mp[k] = 0.0;
+  mp[9] = hh;
   a.geo_c[n] = make_double4(r[0], r[1], r[2], hh);
   a.geo_h[n] = make_double4(0.0, 0.0, 0.0, __ddiv_rn(__dmul_rn(hh, hh), theta2));
 }
@@ -329,15 +332,6 @@ __global__ void k_leaves(int N, const double* __restrict__ x, const double* __re
 struct NodeD {
   double lo[3], hi[3], com[3], m, q[5], hmax;
 };
-
-__device__ __forceinline__ void load_node(int n, const NodeArgs& a, NodeD& d) {
-  for (int k = 0; k < 3; k++) {
-    d.lo[k] = a.bbmin[3*n+k]; d.hi[k] = a.bbmax[3*n+k]; d.com[k] = a.mp[10*n+k];
-  }
-  d.m = a.mp[10*n+3];
-  for (int k = 0; k < 5; k++) d.q[k] = a.mp[10*n+4+k];
-  d.hmax = a.geo_c[n].w;
-}
 
 // merge children L (left) and R (right) into o; operation order of KDTree.cpp:950-1051
 __device__ __forceinline__ void merge_d(const NodeD& L, const NodeD& R, NodeD& o) {
@@ -367,14 +361,9 @@ __device__ __forceinline__ void merge_d(const NodeD& L, const NodeD& R, NodeD& o
   }
 }
 
-__device__ __forceinline__ void store_node(int n, const NodeD& d, double theta2,
-                                           const NodeArgs& a) {
+// box centre and half-widths with the bound on h and the opening distance
+__device__ __forceinline__ void store_geo(int n, const NodeD& d, double theta2, const NodeArgs& a) {
 #pragma clang fp contract(off)
-  for (int k = 0; k < 3; k++) {
-    a.mp[10*n+k] = d.com[k]; a.bbmin[3*n+k] = d.lo[k]; a.bbmax[3*n+k] = d.hi[k];
-  }
-  a.mp[10*n+3] = d.m;
-  for (int k = 0; k < 5; k++) a.mp[10*n+4+k] = d.q[k];
   double c[3], hf[3];
   for (int k = 0; k < 3; k++) { c[k] = 0.5*(d.lo[k] + d.hi[k]); hf[k] = 0.5*(d.hi[k] - d.lo[k]); }
   const double rmaxsqd = hf[0]*hf[0] + hf[1]*hf[1] + hf[2]*hf[2];
@@ -382,271 +371,337 @@ __device__ __forceinline__ void store_node(int n, const NodeD& d, double theta2,
   a.geo_h[n] = make_double4(hf[0], hf[1], hf[2], fmax(rmaxsqd, d.hmax*d.hmax)/theta2);
 }
 
-// new smoothing-length bound of internal node n whose box is unchanged
-__device__ __forceinline__ void store_h(int n, double hmax, double theta2, const NodeArgs& a) {
+// Bottom-up refit.  A workgroup takes a contiguous run of finished nodes and merges the nodes whose
+// leaf range lies inside the run, level by level: the second child to finish puts its parent on the
+// next level's list, and the list's nodes are merged one a lane, so that the lanes of a wavefront
+// stay together however uneven the tree is.  The moments stay in LDS, each node's in the place of
+// its left child's.  Phase 1 runs over chunks of RB leaves; what it leaves (the maximal nodes inside
+// each chunk, in leaf order) is the input of the next phase, RS runs a workgroup, until one
+// workgroup reaches the root.  Every node is merged exactly once from finished children in the fixed
+// (left, right) operand order, and no two workgroups touch the same node, so there are no atomics
+// beyond LDS (device-scope ones would write back the per-XCD L2 on every level).
+//
+// Bound by the chain of levels at small runs and by vector issue before this: with a thread climbing
+// from every leaf each wavefront carried the whole merge through every level for a few lanes.  (us,
+// before and after, phase 1 and the rest)
+//   particles                4096     20011    131072   262144   1048576
+//   all moments, phase 1     37 23    58 29    54 36    65 39    240 148
+//   all moments, the rest     7  7    36 30   122 88   101 62    167  80
+//   h alone, phase 1         10  9    13 13             19 17     63  59
+//   h alone, the rest         5  6    18 18             42 38     61  47
+constexpr int RB = 1024;   // leaves per phase-1 workgroup
+constexpr int RS = 32;     // runs per workgroup of the later phases
+constexpr int RF = 768;    // nodes a workgroup of the later phases holds at a time
+constexpr int RT = 512;    // its threads (a level merges at most half of the nodes)
+
+// The moments in LDS, component by component in the order of a node's record in memory: one spare
+// slot in 32, as the slots of higher levels are multiples of ever higher powers of two, and an odd
+// stride, as a record's components are read together.  A record is one line, written and read by
+// eight lanes together: a lane writing its own node's would touch a line with every store.
+template <bool HONLY, int CAP> struct RefitSlots {
+  static constexpr int ND = HONLY ? 1 : kMom, STRIDE = CAP + CAP/32 + (CAP/32 & 1 ? 0 : 1);
+  double v[ND*STRIDE];
+  __device__ __forceinline__ static int at(int s) { return s + (s >> 5); }
+  __device__ __forceinline__ void put(int s, const NodeD& d) {
+    double* p = v + at(s);
+    if (HONLY) { p[0] = d.hmax; return; }
+    for (int k = 0; k < 3; k++) {
+      p[k*STRIDE] = d.com[k]; p[(10 + k)*STRIDE] = d.lo[k]; p[(13 + k)*STRIDE] = d.hi[k];
+    }
+    p[3*STRIDE] = d.m;
+    for (int k = 0; k < 5; k++) p[(4 + k)*STRIDE] = d.q[k];
+    p[9*STRIDE] = d.hmax;
+  }
+  __device__ __forceinline__ void get(int s, NodeD& d) const {
+    const double* p = v + at(s);
+    if (HONLY) { d.hmax = p[0]; return; }
+    for (int k = 0; k < 3; k++) {
+      d.com[k] = p[k*STRIDE]; d.lo[k] = p[(10 + k)*STRIDE]; d.hi[k] = p[(13 + k)*STRIDE];
+    }
+    d.m = p[3*STRIDE];
+    for (int k = 0; k < 5; k++) d.q[k] = p[(4 + k)*STRIDE];
+    d.hmax = p[9*STRIDE];
+  }
+  // record part k (two components of sixteen) of slot s, from or to node n's in memory
+  __device__ __forceinline__ void part_out(int s, int n, int k, const NodeArgs& a) const {
+    const double* p = v + at(s) + 2*k*STRIDE;
+    reinterpret_cast<double2*>(a.mp)[(size_t) n*(kMom/2) + k] = make_double2(p[0], p[STRIDE]);
+  }
+  __device__ __forceinline__ void part_in(int s, int n, int k, const NodeArgs& a) {
+    const double2 x = reinterpret_cast<const double2*>(a.mp)[(size_t) n*(kMom/2) + k];
+    double* p = v + at(s) + 2*k*STRIDE;
+    p[0] = x.x; p[STRIDE] = x.y;
+  }
+  // merge slots l and r into l as node n; rmax2: the squared half-diagonal of its box (HONLY).
+  // The record is left to part_out.
+  __device__ __forceinline__ void merge(int l, int r, int n, double rmax2, double theta2,
+                                        const NodeArgs& a) {
 #pragma clang fp contract(off)
-  double4 gc = a.geo_c[n];
-  double4 gh = a.geo_h[n];
-  const double rmaxsqd = gh.x*gh.x + gh.y*gh.y + gh.z*gh.z;
-  gc.w = hmax;
-  gh.w = fmax(rmaxsqd, hmax*hmax)/theta2;
-  a.geo_c[n] = gc;
-  a.geo_h[n] = gh;
+    NodeD L, R, o;
+    get(l, L);
+    get(r, R);
+    if (HONLY) {
+      o.hmax = fmax(L.hmax, R.hmax);
+      a.geo_c[n].w = o.hmax;
+      a.geo_h[n].w = fmax(rmax2, o.hmax*o.hmax)/theta2;
+    } else {
+      merge_d(L, R, o);
+      store_geo(n, o, theta2, a);
+    }
+    put(l, o);
+  }
+  // the records of a wavefront's merged nodes, the first `count` of which are node(j), slot(j)
+  template <class A, class B>
+  __device__ __forceinline__ void records_out(int count, A node, B slot, const NodeArgs& a) const {
+    if (HONLY) return;
+    wave_lds_order();
+    for (int j = lane_id()/(kMom/2); j < count; j += kWave/(kMom/2))
+      part_out(slot(j), node(j), lane_id() & (kMom/2 - 1), a);
+    wave_lds_order();
+  }
+};
+
+__device__ __forceinline__ double box_rmax2(const NodeArgs& a, int n) {
+#pragma clang fp contract(off)
+  const double4 gh = a.geo_h[n];
+  return gh.x*gh.x + gh.y*gh.y + gh.z*gh.z;
 }
 
-
-// Bottom-up refit in three phases.  The second child to reach a node merges it (an arrival
-// counter per node decides which), so every node is merged exactly once from finished children
-// in the fixed (left, right) operand order.  Synchronising through device-scope atomics would
-// write back and invalidate the per-XCD L2 on every tree level, so the counters stay within one
-// workgroup: phase 1 gives each workgroup a chunk of RB consecutive leaves and merges the nodes
-// whose particle range lies inside the chunk (an internal node is one end of its own range, so
-// its counter fits the chunk's LDS); the maximal such nodes form the chunk's frontier.  Phase 2
-// repeats this over RS chunks per workgroup starting from those frontiers, and phase 3 is one
-// workgroup that climbs the few remaining nodes to the root.
-constexpr int RB = 1024;   // leaves per phase-1 workgroup
-constexpr int RS = 32;     // phase-1 chunks per phase-2 workgroup
-
-// Phase 1, fused with the leaf moments.  The chunk's topology is staged in LDS, and each
-// climbing thread carries its node's moments in registers: before it counts its arrival at a
-// parent it leaves them in its own LDS slot, and the exchange that counts the arrival hands the
-// second arriver the first one's slot, so a merge reads nothing from global memory.  A slot is
-// read only after its owner has stopped climbing, hence is never overwritten while still needed.
+// Phase 1, fused with the leaf moments.
 template <bool HONLY>
 __global__ __launch_bounds__(RB) void k_refit_chunks(
     int N, const double* __restrict__ x, const double* __restrict__ y,
     const double* __restrict__ z, const double* __restrict__ mass, const double* __restrict__ h,
-    const int* __restrict__ parent, const int* __restrict__ left, const int* __restrict__ first,
-    const int* __restrict__ last, double theta2, NodeArgs a, int* __restrict__ visit,
-    int* __restrict__ front1, int* __restrict__ cnt1, int* __restrict__ front2_count) {
+    const int* __restrict__ parent, const int4* __restrict__ lnk, double theta2, NodeArgs a,
+    int* __restrict__ visit, int* __restrict__ front, int* __restrict__ nfront) {
 #pragma clang fp contract(off)
-  constexpr int ND = HONLY ? 1 : 16;    // doubles carried per node
-  __shared__ double sd[ND*RB];
-  __shared__ int arr[RB];               // 0, or 1 + slot of the first arrival
-  __shared__ int lpar[RB];              // parent of leaf c0 + t
-  __shared__ int ipar[RB];              // parent of internal node c0 + t
-  __shared__ int lft[RB];               // left child of internal node c0 + t, -1 if not inside
-  __shared__ int nfront;
+  __shared__ RefitSlots<HONLY, RB> sd;
+  __shared__ int arr[RB];               // arrivals at internal node c0 + t
+  __shared__ int ipar[RB];              // its parent
+  __shared__ int lr[RB];                // its children's slots, left | right << 16; -1 if not inside
+  __shared__ int fr[RB];                // the maximal node that starts at leaf c0 + t, or -1
+  __shared__ short list[2][RB/2];       // nodes to merge
+  __shared__ int cnt[3];
+  __shared__ int wsum[RB/kWave];
   const int t = threadIdx.x;
   const int c0 = blockIdx.x*RB;
   const int c1 = min(c0 + RB, N) - 1;
   const int l = c0 + t;
   arr[t] = 0;
-  if (t == 0) nfront = 0;
-  if (blockIdx.x == 0 && t == 0) *front2_count = 0;   // phase 2 counts its frontier here
-  NodeD d;
+  fr[t] = -1;
+  lr[t] = -1;
+  if (t < 3) cnt[t] = 0;
+  int up = -1;
+  double rmax2 = 0.0;                   // HONLY: of internal node c0 + t
   if (l <= c1) {
-    lpar[t] = parent[N - 1 + l];
+    up = parent[N - 1 + l];
     if (l < N - 1) {
       ipar[t] = parent[l];
-      lft[t] = (first[l] >= c0 && last[l] <= c1) ? left[l] : -1;
+      const int4 k = lnk[l];            // (first, last, left, right)
+      if (k.x >= c0 && k.y <= c1) {
+        const int split = k.z >= N - 1 ? k.z - (N - 1) : k.z;      // last leaf of the left child
+        lr[t] = (k.x - c0) | (split + 1 - c0) << 16;
+      }
       visit[l] = 0;
-    } else {
-      lft[t] = -1;
+      if (HONLY) rmax2 = box_rmax2(a, l);
     }
     const int n = N - 1 + l;
     const double hh = h[l];
+    NodeD d;
     d.hmax = hh;
     if (HONLY) {
-      double4 gc = a.geo_c[n]; gc.w = hh; a.geo_c[n] = gc;
-      double4 gh = a.geo_h[n]; gh.w = hh*hh/theta2; a.geo_h[n] = gh;
+      a.geo_c[n].w = hh;
+      a.geo_h[n].w = hh*hh/theta2;
     } else {
       const double r[3] = {x[l], y[l], z[l]};
       for (int k = 0; k < 3; k++) { d.lo[k] = r[k]; d.hi[k] = r[k]; d.com[k] = r[k]; }
       d.m = mass[l];
       for (int k = 0; k < 5; k++) d.q[k] = 0.0;
-      for (int k = 0; k < 3; k++) { a.bbmin[3*n+k] = r[k]; a.bbmax[3*n+k] = r[k]; a.mp[10*n+k] = r[k]; }
-      a.mp[10*n+3] = d.m;
-      for (int k = 4; k < 10; k++) a.mp[10*n+k] = 0.0;
       a.geo_c[n] = make_double4(r[0], r[1], r[2], hh);
       a.geo_h[n] = make_double4(0.0, 0.0, 0.0, hh*hh/theta2);
     }
+    sd.put(t, d);
   }
+  // HONLY: the half-diagonals wait for their merge in LDS
+  __shared__ double rm[HONLY ? RB : 1];
+  if (HONLY) rm[t] = rmax2;
   __syncthreads();
-  if (l <= c1) {
-    int n = N - 1 + l;
-    int p = lpar[t];
-    while (p >= 0) {
-      const int lf = (p >= c0 && p <= c1) ? lft[p - c0] : -1;
-      if (lf < 0) {
-        // n is a maximal node of this chunk: at most RB of them
-        front1[c0 + atomicAdd(&nfront, 1)] = n;
-        break;
-      }
-      if (HONLY) {
-        sd[t] = d.hmax;
-      } else {
-        for (int k = 0; k < 3; k++) {
-          sd[k*RB + t] = d.lo[k]; sd[(3 + k)*RB + t] = d.hi[k]; sd[(6 + k)*RB + t] = d.com[k];
-        }
-        sd[9*RB + t] = d.m;
-        for (int k = 0; k < 5; k++) sd[(10 + k)*RB + t] = d.q[k];
-        sd[15*RB + t] = d.hmax;
-      }
-      const int old = __hip_atomic_exchange(&arr[p - c0], t + 1, __ATOMIC_ACQ_REL,
-                                            __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (old == 0) break;
-      const int o = old - 1;
-      if (HONLY) {
-        d.hmax = fmax(d.hmax, sd[o]);
-        store_h(p, d.hmax, theta2, a);
-      } else {
-        NodeD e, r;
-        for (int k = 0; k < 3; k++) {
-          e.lo[k] = sd[k*RB + o]; e.hi[k] = sd[(3 + k)*RB + o]; e.com[k] = sd[(6 + k)*RB + o];
-        }
-        e.m = sd[9*RB + o];
-        for (int k = 0; k < 5; k++) e.q[k] = sd[(10 + k)*RB + o];
-        e.hmax = sd[15*RB + o];
-        if (lf == n) merge_d(d, e, r);
-        else merge_d(e, d, r);
-        store_node(p, r, theta2, a);
-        d = r;
-      }
-      n = p;
-      p = ipar[p - c0];
-    }
-  }
+  // node n with parent p, starting at slot s, is finished
+  auto arrive = [&](int n, int p, int s, int b) {
+    if (p < 0) return;
+    if (p < c0 || p > c1 || lr[p - c0] < 0) fr[s] = n;
+    else if (atomicAdd(&arr[p - c0], 1) == 1) list[b & 1][atomicAdd(&cnt[b % 3], 1)] = (short) (p - c0);
+  };
+  if (l <= c1) arrive(N - 1 + l, up, t, 0);
+  if (!HONLY)
+    for (int k = t; k <= (c1 - c0)*(kMom/2) + kMom/2 - 1; k += RB)
+      sd.part_out(k/(kMom/2), N - 1 + c0 + k/(kMom/2), k & (kMom/2 - 1), a);
   __syncthreads();
-  if (t == 0) cnt1[blockIdx.x] = nfront;
-}
-
-// Topology of the next node of a climb, loaded together with the moments of the current
-// merge so that each level of phases 2 and 3 waits on global memory about once.
-struct Topo {
-  int first, last, left, right, parent;
-  double rmax2;   // squared half-diagonal of the node's box (smoothing-length refit only)
-};
-
-template <bool HONLY>
-__device__ __forceinline__ void load_topo(int p, const int* __restrict__ parent,
-                                          const int* __restrict__ left,
-                                          const int* __restrict__ right,
-                                          const int* __restrict__ first,
-                                          const int* __restrict__ last, const NodeArgs& a,
-                                          Topo& q) {
-#pragma clang fp contract(off)
-  q.first = first[p]; q.last = last[p]; q.left = left[p]; q.right = right[p];
-  q.parent = parent[p];
-  if (HONLY) {
-    // the box only: another thread may be writing the node's .w bound
-    const double hx = a.geo_h[p].x, hy = a.geo_h[p].y, hz = a.geo_h[p].z;
-    q.rmax2 = hx*hx + hy*hy + hz*hz;
-  }
-}
-
-// Climb from node n through the nodes whose leaf range lies in [lo, hi] (phase 2) or up to
-// the root (phase 3, lo = 0 and hi = N - 1).  The second arrival at a node, counted in
-// cnt[p - cbase], merges it from its own moments (registers) and its sibling's (global memory,
-// written before the sibling's thread counted its arrival).  A node whose parent leaves the
-// range goes to the next frontier.
-template <bool HONLY>
-__device__ __forceinline__ void climb(int n, int lo, int hi, int* cnt, int cbase,
-                                      const int* __restrict__ parent,
-                                      const int* __restrict__ left,
-                                      const int* __restrict__ right,
-                                      const int* __restrict__ first,
-                                      const int* __restrict__ last, double theta2,
-                                      const NodeArgs& a, int* __restrict__ front_next,
-                                      int* __restrict__ front_count) {
-#pragma clang fp contract(off)
-  NodeD d;
-  if (HONLY) d.hmax = a.geo_c[n].w;
-  else load_node(n, a, d);
-  int p = parent[n];
-  Topo q;
-  if (p >= 0) load_topo<HONLY>(p, parent, left, right, first, last, a, q);
-  while (p >= 0) {
-    if (q.first < lo || q.last > hi) {
-      front_next[atomicAdd(front_count, 1)] = n;
-      break;
+  for (int b = 0; ; b++) {
+    const int n = cnt[b % 3];
+    if (n == 0) break;
+    if (t == 0) cnt[(b + 2) % 3] = 0;
+    if (t < n) {
+      const int q = list[b & 1][t], w = lr[q], L = w & 0xffff;
+      sd.merge(L, w >> 16, c0 + q, HONLY ? rm[q] : 0.0, theta2, a);
+      arrive(c0 + q, ipar[q], L, b + 1);
     }
-    const int old = __hip_atomic_fetch_add(&cnt[p - cbase], 1, __ATOMIC_ACQ_REL,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (old == 0) break;
-    const bool isleft = q.left == n;
-    const int sib = isleft ? q.right : q.left;
-    const int pp = q.parent;
-    Topo qn;
-    if (pp >= 0) load_topo<HONLY>(pp, parent, left, right, first, last, a, qn);
-    if (HONLY) {
-      d.hmax = fmax(d.hmax, a.geo_c[sib].w);
-      a.geo_c[p].w = d.hmax;
-      a.geo_h[p].w = fmax(q.rmax2, d.hmax*d.hmax)/theta2;
-    } else {
-      NodeD e, r;
-      load_node(sib, a, e);
-      if (isleft) merge_d(d, e, r);
-      else merge_d(e, d, r);
-      store_node(p, r, theta2, a);
-      d = r;
-    }
-    n = p;
-    p = pp;
-    q = qn;
+    const short* w = list[b & 1] + t/kWave*kWave;
+    sd.records_out(min(n - t/kWave*kWave, kWave), [&](int j) { return c0 + w[j]; },
+                   [&](int j) { return lr[w[j]] & 0xffff; }, a);
+    __syncthreads();
   }
+  // the maximal nodes in leaf order
+  const int node = fr[t];
+  const unsigned long long m = __ballot(node >= 0);
+  if (lane_id() == 0) wsum[t/kWave] = __popcll(m);
+  __syncthreads();
+  int o = 0, total = 0;
+  for (int w = 0; w < RB/kWave; w++) {
+    if (w < t/kWave) o += wsum[w];
+    total += wsum[w];
+  }
+  if (node >= 0) front[c0 + o + lanes_below(m)] = node;
+  if (t == 0) nfront[blockIdx.x] = total;
 }
 
-// Phase 2: one workgroup per RS consecutive phase-1 chunks climbs from their frontier nodes
-// through the nodes inside its leaf range.  Every arrival at such a node comes from this
-// workgroup, and the node's index lies in the range, so the arrival counters live in LDS.
+// Later phases: runs [blk RS, blk RS + RS) of `span` leaves each, the run starting at leaf f having
+// its maximal nodes at in[f ...], nin of them; their merge leaves out[lo ...] and nout.  More nodes
+// than the workgroup holds are merged a window at a time until they fit (a window of RF adjacent
+// nodes leaves at most two a level of the tree).
 template <bool HONLY>
-__global__ __launch_bounds__(RB) void k_refit_mid(
-    int N, int nchunks, const int* __restrict__ parent, const int* __restrict__ left,
-    const int* __restrict__ right, const int* __restrict__ first, const int* __restrict__ last,
-    double theta2, NodeArgs a, const int* __restrict__ front1, const int* __restrict__ cnt1,
-    int* __restrict__ front2) {
-  __shared__ int arr[RB*RS];
+__global__ __launch_bounds__(RT) void k_refit_runs(
+    int N, int nruns, long long span, const int* __restrict__ parent, const int4* __restrict__ lnk,
+    double theta2, NodeArgs a, const int* __restrict__ in, const int* __restrict__ nin,
+    int* __restrict__ out, int* __restrict__ nout) {
+#pragma clang fp contract(off)
+  struct Ready { int node, parent; short left, right; };
+  __shared__ RefitSlots<HONLY, RF> sd;
+  __shared__ int nd[RF];                // the node starting at slot s, or -1
+  __shared__ short en[RF];              // one past its last slot
+  __shared__ int arr[RF + 1];           // arrivals at the node whose right child starts at slot s
+  __shared__ short lft[RF + 1];         // ... and the slot of its left child, once that arrived
+  __shared__ Ready list[2][RF/2];
+  __shared__ double rm[HONLY ? RF + 1 : 1];      // ... and its box's squared half-diagonal
+  __shared__ int cnt[3];
   __shared__ int pre[RS + 1];
-  const int k0 = blockIdx.x*RS, k1 = min(k0 + RS, nchunks);
-  const int lo = k0*RB, hi = min(k1*RB, N) - 1;
-  for (int i = threadIdx.x; i < RB*RS; i += RB) arr[i] = 0;
-  if (threadIdx.x == 0) {
+  const int t = threadIdx.x;
+  const int k0 = blockIdx.x*RS, k1 = min(k0 + RS, nruns);
+  const int lo = (int) (k0*span), hi = (int) min(k1*span, (long long) N) - 1;
+  if (t == 0) {
     pre[0] = 0;
-    for (int c = 0; c < RS; c++) pre[c + 1] = pre[c] + (k0 + c < k1 ? cnt1[k0 + c] : 0);
+    for (int c = 0; c < RS; c++) pre[c + 1] = pre[c] + (k0 + c < k1 ? nin[k0 + c] : 0);
   }
   __syncthreads();
-  const int total = pre[RS];
-  for (int e = threadIdx.x; e < total; e += RB) {
-    int c = 0;
-    while (pre[c + 1] <= e) c++;
-    climb<HONLY>(front1[(k0 + c)*RB + (e - pre[c])], lo, hi, arr, lo, parent, left, right,
-                 first, last, theta2, a, front2, &front2[N]);
+  int total = pre[RS];
+  bool first = true;                    // nodes still in `in`, run by run; else in out[lo ...]
+  for (;;) {
+    int done = 0;                       // nodes left by the windows so far
+    for (int w0 = 0; w0 < total; w0 += RF) {
+      const int F = min(RF, total - w0);
+      if (t < 3) cnt[t] = 0;
+      for (int s = t; s < F; s += RT) {
+        int n;
+        if (first) {
+          int c = 0;
+          while (pre[c + 1] <= w0 + s) c++;
+          n = in[(size_t) ((k0 + c)*span) + (w0 + s - pre[c])];
+        } else {
+          n = out[lo + w0 + s];
+        }
+        nd[s] = n;
+        en[s] = (short) (s + 1);
+        if (HONLY) sd.v[sd.at(s)] = a.geo_c[n].w;
+      }
+      for (int s = t; s <= F; s += RT) arr[s] = 0;
+      __syncthreads();
+      if (!HONLY) {
+        for (int k = t; k < F*(kMom/2); k += RT)
+          sd.part_in(k/(kMom/2), nd[k/(kMom/2)], k & (kMom/2 - 1), a);
+      }
+      // node n with parent p and its topology, slots [s, e), is finished
+      struct Up { int4 k; int parent; double rmax2; };
+      auto above = [&](int p) {
+        Up u = {make_int4(0, 0, 0, 0), -1, 0.0};
+        if (p < 0) return u;
+        u.k = lnk[p];                   // (first, last, left, right)
+        u.parent = parent[p];
+        if (HONLY) u.rmax2 = box_rmax2(a, p);
+        return u;
+      };
+      auto arrive = [&](int n, int p, const Up& u, int s, int e, int b) {
+        if (p < 0 || u.k.x < lo || u.k.y > hi) return;
+        const bool isleft = u.k.z == n;
+        const int r = isleft ? e : s;
+        if (isleft) lft[r] = (short) s;
+        if (__hip_atomic_fetch_add(&arr[r], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+          return;
+        if (HONLY) rm[r] = u.rmax2;
+        list[b & 1][atomicAdd(&cnt[b % 3], 1)] = {p, u.parent, lft[r], (short) r};
+      };
+      for (int s = t; s < F; s += RT) {
+        const int p = parent[nd[s]];
+        arrive(nd[s], p, above(p), s, s + 1, 0);
+      }
+      __syncthreads();
+      for (int b = 0; ; b++) {
+        const int n = cnt[b % 3];
+        if (n == 0) break;
+        if (t == 0) cnt[(b + 2) % 3] = 0;
+        if (t < n) {
+          const Ready q = list[b & 1][t];
+          const Up u = above(q.parent);    // in flight during the merge
+          sd.merge(q.left, q.right, q.node, HONLY ? rm[q.right] : 0.0, theta2, a);
+          const int e = en[q.right];
+          nd[q.right] = -1;
+          nd[q.left] = q.node;
+          en[q.left] = (short) e;
+          arrive(q.node, q.parent, u, q.left, e, b + 1);
+        }
+        const Ready* w = list[b & 1] + t/kWave*kWave;
+        sd.records_out(min(n - t/kWave*kWave, kWave), [&](int j) { return w[j].node; },
+                       [&](int j) { return (int) w[j].left; }, a);
+        __syncthreads();
+      }
+      // what is left, in leaf order, by the first wavefront
+      int left = 0;
+      for (int s0 = 0; s0 < F; s0 += kWave) {
+        const int s = s0 + (t & (kWave - 1));
+        const int n = s < F ? nd[s] : -1;
+        const unsigned long long m = __ballot(n >= 0);
+        if (t < kWave && n >= 0) out[lo + done + left + lanes_below(m)] = n;
+        left += __popcll(m);
+      }
+      done += left;
+      __syncthreads();
+    }
+    const bool more = total > RF && done < total;
+    total = done;
+    first = false;
+    if (!more) break;
   }
-}
-
-// Phase 3: one workgroup climbs from the phase-3 frontier to the root, counting arrivals in
-// global memory (the nodes above the frontier may have any index).
-template <bool HONLY>
-__global__ __launch_bounds__(RB) void k_refit_top(
-    int N, const int* __restrict__ parent, const int* __restrict__ left,
-    const int* __restrict__ right, const int* __restrict__ first, const int* __restrict__ last,
-    double theta2, NodeArgs a, const int* __restrict__ front2, int* __restrict__ visit) {
-  const int nf = front2[N];
-  // every range lies in [0, N - 1], so the climb never reaches its frontier branch
-  for (int k = threadIdx.x; k < nf; k += RB)
-    climb<HONLY>(front2[k], 0, N - 1, visit, 0, parent, left, right, first, last, theta2, a,
-                 nullptr, nullptr);
+  if (t == 0) nout[blockIdx.x] = total;
 }
 
 template <bool HONLY>
 void launch_refit(gdf_ctx* c, const NodeArgs& na, double theta2) {
   const int N = c->N;
   hipStream_t s = c->stream;
-  const int nch = (N + RB - 1)/RB;
-  int* front1 = c->front;                          // nch*RB entries
-  int* cnt1 = front1 + (size_t) nch*RB;            // nch counts
-  int* front2 = cnt1 + nch;                        // N entries + count
-  k_refit_chunks<HONLY><<<nch, RB, 0, s>>>(N, c->pf[F_X], c->pf[F_Y], c->pf[F_Z], c->pf[F_M],
-                                           c->pf[F_H], c->parent, c->left, c->first, c->last,
-                                           theta2, na, c->visit, front1, cnt1, front2 + N);
-  if (nch > 1) {
-    const int nmid = (nch + RS - 1)/RS;
-    k_refit_mid<HONLY><<<nmid, RB, 0, s>>>(N, nch, c->parent, c->left, c->right, c->first,
-                                           c->last, theta2, na, front1, cnt1, front2);
-    if (nmid > 1)
-      k_refit_top<HONLY><<<1, RB, 0, s>>>(N, c->parent, c->left, c->right, c->first, c->last,
-                                          theta2, na, front2, c->visit);
+  int nrun = (N + RB - 1)/RB;
+  int* from = c->front;                            // N entries a buffer, and a count a run
+  int* to = from + N;
+  int* nfrom = to + N;
+  int* nto = nfrom + nrun;
+  k_refit_chunks<HONLY><<<nrun, RB, 0, s>>>(N, c->pf[F_X], c->pf[F_Y], c->pf[F_Z], c->pf[F_M],
+                                            c->pf[F_H], c->parent, c->lnk, theta2, na, c->visit,
+                                            from, nfrom);
+  for (long long span = RB; nrun > 1; span *= RS) {
+    const int nb = (nrun + RS - 1)/RS;
+    k_refit_runs<HONLY><<<nb, RT, 0, s>>>(N, nrun, span, c->parent, c->lnk, theta2, na, from, nfrom,
+                                          to, nto);
+    std::swap(from, to);
+    std::swap(nfrom, nto);
+    nrun = nb;
   }
 }
 
@@ -755,7 +810,7 @@ TreeView tree_view(const gdf_ctx* c) {
 }
 
 static NodeArgs node_args(gdf_ctx* c) {
-  NodeArgs a; a.bbmin = c->bbmin; a.bbmax = c->bbmax; a.geo_c = c->geo_c; a.geo_h = c->geo_h;
+  NodeArgs a; a.geo_c = c->geo_c; a.geo_h = c->geo_h;
   a.mp = c->mp;
   return a;
 }
@@ -806,12 +861,10 @@ int tree_alloc(gdf_ctx* c) {
   GDF_HIP(c, hipMalloc(&c->lnk, sizeof(int4)*N));
   GDF_HIP(c, hipMalloc(&c->visit, sizeof(int)*(N + 16)));   // also 16-byte-padded flags
   // refit frontiers: phase 1 (one RB slot per chunk), chunk counts, phase 2 (N + count)
-  GDF_HIP(c, hipMalloc(&c->front, sizeof(int)*(2*N + 1024 + N/1024 + 16)));
-  GDF_HIP(c, hipMalloc(&c->bbmin, sizeof(double)*3*nn));
-  GDF_HIP(c, hipMalloc(&c->bbmax, sizeof(double)*3*nn));
+  GDF_HIP(c, hipMalloc(&c->front, sizeof(int)*(2*N + 2*(N/1024 + 16))));
   GDF_HIP(c, hipMalloc(&c->geo_c, sizeof(double4)*nn));
   GDF_HIP(c, hipMalloc(&c->geo_h, sizeof(double4)*nn));
-  GDF_HIP(c, hipMalloc(&c->mp, sizeof(double)*10*nn));
+  GDF_HIP(c, hipMalloc(&c->mp, sizeof(double)*kMom*nn));
   GDF_HIP(c, hipMalloc(&c->gstart, sizeof(int)*N));
   GDF_HIP(c, hipMalloc(&c->grp_first, sizeof(int)*N));
   GDF_HIP(c, hipMalloc(&c->grp_count, sizeof(int)*N));
@@ -999,7 +1052,7 @@ std::vector<const void*> build_key(const gdf_ctx* c) {
   // every other buffer and value the launches take
   const void* other[] = {c->d_seg_off, c->seg_bnd, c->red, c->sort_tmp, c->sel_tmp, c->nsel,
                          c->left, c->right, c->first, c->last, c->parent, c->lnk, c->visit, c->front,
-                         c->bbmin, c->bbmax, c->geo_c, c->geo_h, c->mp, c->gstart, c->grp_first,
+                         c->geo_c, c->geo_h, c->mp, c->gstart, c->grp_first,
                          c->grp_count, c->grp_node};
   for (const void* q : other) k.push_back(q);
   uint64_t theta_bits;

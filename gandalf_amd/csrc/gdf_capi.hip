@@ -394,7 +394,7 @@ int gdf_create(const gdf_config* cfg, gdf_ctx** out) {
   p.ewald = cfg->periodic && cfg->self_gravity && !cfg->nbody;
   if (rc == GDF_OK && p.ewald) rc = upload_ewald_table(c);
   if (rc == GDF_OK) {
-    if (hipMalloc(&c->counters, sizeof(int)*32) != hipSuccess ||
+    if (hipMalloc(&c->counters, sizeof(int)*(16 + kGravZero)) != hipSuccess ||
         hipMalloc(&c->icount, sizeof(long long)*8) != hipSuccess ||
         hipMalloc(&c->red, sizeof(double)*16384) != hipSuccess ||
         hipHostMalloc(&c->h_counters, sizeof(int)*32) != hipSuccess ||
@@ -402,7 +402,7 @@ int gdf_create(const gdf_config* cfg, gdf_ctx** out) {
       rc = GDF_ERR_NOMEM;
   }
   if (rc == GDF_OK) {
-    hipMemset(c->counters, 0, sizeof(int)*32);
+    hipMemset(c->counters, 0, sizeof(int)*(16 + kGravZero));
     if (hipStreamCreate(&c->stream2) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_dens, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_grav, hipEventDisableTiming) != hipSuccess)

@@ -448,18 +448,6 @@ __device__ __forceinline__ void eos_state(const PhysParams& p, double rho, doubl
   press = p.gammam1*rho*u;
 }
 
-// Next work item for a persistent wavefront.  Every active lane takes part in the atomic (the
-// first active lane adds one, the others zero) and the result is broadcast with readfirstlane,
-// so the index is a scalar and the loop that consumes it has uniform control flow.  Fetching
-// behind `if (lane == 0)` and broadcasting with a shuffle instead lets the compiler treat the
-// loop exit as divergent and re-enter the loop body with lane 0 split off, where the shuffle
-// then reads a stale index.
-__device__ __forceinline__ int wave_next_item(int* counter) {
-  const int first = lanes_below(__ballot(1)) == 0;
-  const int old = atomicAdd(counter, first ? 1 : 0);
-  return __builtin_amdgcn_readfirstlane(old);
-}
-
 // MI355X has 8 XCDs, each with its own L2, and workgroups are dispatched to them round-robin by
 // workgroup id.  Work that neighbours other work in memory (Morton-ordered particles, walk
 // groups) is therefore remapped so each XCD takes one contiguous eighth.
@@ -470,21 +458,6 @@ constexpr int kXcds = 8;
 __device__ __forceinline__ int xcd_block(int b, int nb) {
   const int x = b % kXcds, k = b / kXcds, q = nb / kXcds, r = nb % kXcds;
   return x*q + min(x, r) + k;
-}
-
-// Next walk group for a persistent wavefront: the groups are split into 8 contiguous ranges with
-// one counter each (counters[0..7]); a wave starts on its own XCD's range and moves to the next
-// range when that is exhausted.  `range` carries the current range between calls; returns
-// ngroups when every range is exhausted.
-__device__ __forceinline__ int wave_next_group(int* counters, int ngroups, int& range) {
-  for (int t = 0; t < kXcds; t++) {
-    const int r = (range + t) % kXcds;
-    const int lo = (int) (((long long) ngroups*r)/kXcds);
-    const int hi = (int) (((long long) ngroups*(r + 1))/kXcds);
-    const int k = wave_next_item(&counters[r]);
-    if (lo + k < hi) { range = r; return lo + k; }
-  }
-  return ngroups;
 }
 
 // ---- tree walks ----
@@ -515,27 +488,32 @@ __device__ __forceinline__ void load_links(int n, int N, const int4* __restrict_
   }
 }
 
-// Queue of walk groups for a grid of persistent wavefronts.  nq entries (all groups, or a
-// compacted list of the groups with targets): when they fit the grid, wavefront b takes entry b
-// and stops, with no atomics and the work spread over every XCD; otherwise the entries come from
-// the per-XCD ranged queues of wave_next_group.  Returns nq when the wavefront is done.
+// The walk groups of a persistent workgroup: nq entries (all groups, or a compacted list of the
+// groups with targets) in eight contiguous ranges, one an XCD, whose workgroups take every
+// (their number)-th entry of it.  Neighbouring groups are walked at the same time and share the
+// XCD's L2.  (Fetching each entry from a counter a range, and on from the other ranges', took an
+// atomic an entry and eight a workgroup on one line: 0.1 ms of a walk of 2048 groups.)
 struct GroupQueue {
-  int nq;
-  int range;
-  bool once;
+  int first, end, step;
 };
 __device__ __forceinline__ GroupQueue group_queue(int nq) {
-  GroupQueue q;
-  q.nq = nq; q.range = blockIdx.x % kXcds; q.once = false;
-  return q;
+  const int x = blockIdx.x % kXcds, nb = gridDim.x;
+  const int q = nq/kXcds, r = nq % kXcds, lo = x*q + min(x, r);
+  return {lo + (int) blockIdx.x/kXcds, lo + q + (x < r), nb/kXcds + (x < nb % kXcds)};
 }
-__device__ __forceinline__ int group_next(GroupQueue& q, int* counters) {
-  if (q.nq <= (int) gridDim.x) {
-    if (q.once) return q.nq;
-    q.once = true;
-    return (int) blockIdx.x < q.nq ? (int) blockIdx.x : q.nq;
+
+// The same ranges handed out entry by entry, for walks whose groups cost unequally: one counter a
+// range, kQueueStride apart (the line is the unit that atomics are serialised by), and from the
+// other ranges once a workgroup's own is empty.  Called by one lane; returns nq at the end.
+constexpr int kQueueStride = 32;
+__device__ __forceinline__ int group_fetch(int* counters, int nq, int& range) {
+  const int q = nq/kXcds, r = nq % kXcds;
+  for (int t = 0; t < kXcds; t++) {
+    const int x = (range + t) % kXcds;
+    const int k = atomicAdd(&counters[x*kQueueStride], 1);
+    if (k < q + (x < r)) { range = x; return x*q + min(x, r) + k; }
   }
-  return wave_next_group(counters, q.nq, q.range);
+  return nq;
 }
 
 // Kahan-compensated accumulator for the mixed-precision pair sums

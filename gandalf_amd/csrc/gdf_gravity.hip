@@ -29,7 +29,9 @@
 // Bound by latency where the groups do not fill the device (each round and each batch waits for
 // its scattered node, cell or particle loads), and by vector issue beside the hydro pass where they
 // do.  20011 particles, FP64: 98 us with four wavefronts a group against 295 with one and the cell
-// term's products written out; a million, FP64, beside the hydro pass: 4.6 against 5.5 ms.
+// term's products written out; a million, FP64, beside the hydro pass: 4.4 against 5.5 ms.  Groups
+// cost unequally, so they are fetched one by one (dealt out beforehand they took 3.4 ms instead of
+// 2.65, FP32), from counters a line apart (on one line: 560 us at 262144 particles instead of 455).
 #include <hip/hip_runtime.h>
 
 #include "gdf_internal.h"
@@ -47,6 +49,8 @@ template <int W> struct GravRings {
   static constexpr int wide = 4096;      // stack entries beyond which a round takes 64 nodes
 };
 
+static_assert(kGravQueue + (kXcds - 1)*kQueueStride < 16 + kGravZero, "range counters are cleared");
+
 struct GravArgs {
   int N, ngroups, nleaf;
   const int* grp_node; const int* grp_first; const int* grp_count;
@@ -54,7 +58,7 @@ struct GravArgs {
   const double4* geo_c; const double4* geo_h; const double* mp;
   const double4* posm; const double4* grec;     // grec: (h, zeta, hfactor, 0)
   double* atx; double* aty; double* atz; double* gpot;
-  int* stacks; int* counter; int* flags; long long* icount;
+  int* stacks; int* queue; int* flags; long long* icount;
   const int* glist; int ncap;   // groups to walk (count at glist[ncap]); NULL = all groups
   int32_t* gnc; int32_t* gnn;
   const int* act;         // block timesteps: only active targets (NULL = all)
@@ -237,7 +241,6 @@ __global__ __launch_bounds__(64*W, EWALD || FAST || (SOFT && !PLUMMER) ? 2 : 3) 
   __shared__ __align__(16) double stage[W][(MIXED ? 5 : 10)*kWave];
   __shared__ int lstk[kLdsStack];    // node stack; deeper entries go to the global region
   __shared__ int count[W][3];        // a round's opened nodes, cells and particles
-  __shared__ int next;
   const int lane = threadIdx.x & (kWave - 1), wv = W == 1 ? 0 : (int) threadIdx.x/kWave;
   double2 (*sd)[kWave] = reinterpret_cast<double2 (*)[kWave]>(stage[wv]);
   double* sr = stage[wv] + 8*kWave;
@@ -249,15 +252,20 @@ __global__ __launch_bounds__(64*W, EWALD || FAST || (SOFT && !PLUMMER) ? 2 : 3) 
   const int N = a.N;
   const KernelDesc& K = a.p.kern;
   const double kr = K.range, krsqd = K.rangesqd;
-  GroupQueue gq = group_queue(a.glist ? a.glist[a.ncap] : a.ngroups);
-  for (;;) {
-    // one lane alone fetches: every lane of a wavefront taking part in a divergent branch made 64
-    // atomics of each fetch, 0.4 ms over the device
-    if (threadIdx.x == 0) next = group_next(gq, a.counter);
+  __shared__ int next;
+  const int nq = a.glist ? a.glist[a.ncap] : a.ngroups;
+  int range = blockIdx.x % kXcds;
+  for (bool once = nq <= (int) gridDim.x; ; ) {
+    if (once) {
+      if (range < 0 || (int) blockIdx.x >= nq) break;
+      range = -1;
+    }
+    // one lane alone fetches: in a divergent branch every active lane's part is an atomic
+    else if (threadIdx.x == 0) next = group_fetch(a.queue, nq, range);
     __syncthreads();
-    const int k = __builtin_amdgcn_readfirstlane(next);
+    const int k = once ? (int) blockIdx.x : __builtin_amdgcn_readfirstlane(next);
     __syncthreads();
-    if (k >= gq.nq) break;
+    if (k >= nq) break;
     const int g = a.glist ? a.glist[k] : k;
     const int G = a.grp_node[g], gfirst = a.grp_first[g], gcnt = a.grp_count[g];
     const bool has = lane < gcnt && (!a.act || a.act[gfirst + lane]);
@@ -736,7 +744,7 @@ __global__ void k_pack_grav(int N, const double* __restrict__ h, const double* _
   if (i < N) g[i] = make_double4(h[i], zeta[i], hf[i], 0.0);
 }
 
-__global__ void k_zero8(int* p) { if (threadIdx.x < 8) p[threadIdx.x] = 0; }
+__global__ void k_zero_ints(int* p) { p[threadIdx.x] = 0; }
 
 // the walk's sums joined to the hydro pass's in the order of the single-stream update
 // (atx += walk; gpot = self + gpot + walk), then a += atree (GradhSphTree.cpp:615-617)
@@ -800,9 +808,9 @@ namespace {
 // Wavefronts that share a walk group.  A group's walk is a chain of dependent loads, so while one
 // wavefront a group leaves SIMDs idle more of them finish sooner; with the device full they only
 // add barriers and partly filled rounds.  Walk (us) with 1, 2 and 4 wavefronts: 512 groups (20011
-// particles, FP64) 232 143 98, 1024 (FP64) 260 188 198, 2048 (FP32) 468 380 302, 2700 stars 397
-// 385 535; the whole force pass (ms): 4096 groups 2.88 2.73 2.81, 16384 10.3 10.6 11.1 (FP32),
-// 13.0 13.2 13.4 (FP64).  A serving batch keeps to two: a request's sums must not depend on what
+// particles, FP64) 230 147 100, 1024 (FP64) 253 183 200, 2048 (FP32) 320 283 300, 2700 of stars
+// 397 390 450; the whole force pass (ms): 4096 groups 2.16 2.15 2.26, 16384 9.38 9.57 9.99 (FP32),
+// 11.6 12.1 12.3 (FP64).  A serving batch keeps to two: a request's sums must not depend on what
 // else is resident.
 int grav_waves(const gdf_ctx* c) {
   if (c->nseg > 0) return 2;
@@ -859,7 +867,7 @@ GravArgs grav_args(gdf_ctx* c) {
   a.geo_c = c->geo_c; a.geo_h = c->geo_h; a.mp = c->mp;
   a.posm = c->posm; a.grec = c->grec;
   a.atx = c->df[D_ATX]; a.aty = c->df[D_ATY]; a.atz = c->df[D_ATZ]; a.gpot = c->df[D_GPOT];
-  a.stacks = c->stacks; a.counter = c->counters + 4; a.flags = c->counters;
+  a.stacks = c->stacks; a.flags = c->counters + 16; a.queue = c->counters + kGravQueue;
   a.icount = c->icount; a.gnc = c->grav_nc; a.gnn = c->grav_nn;
   a.act = c->nlevels > 1 ? c->pi[I_ACT] : nullptr;
   a.grp_root = c->nseg > 0 ? c->grp_root : nullptr;
@@ -871,7 +879,7 @@ GravArgs grav_args(gdf_ctx* c) {
 }
 
 // in a block step, the compacted list of groups with active particles (built on the main stream)
-// zero[0, nzero): the flags and queue counters of the walk, cleared with the list (or by the
+// zero[0, nzero): the flags of the walk, cleared with the list (or by the
 // caller when there is no list: returns false)
 bool grav_group_list(gdf_ctx* c, GravArgs& a, int* zero, int nzero, int& rc) {
   rc = GDF_OK;
@@ -894,18 +902,17 @@ int gravity_launch(gdf_ctx* c) {
   hipStream_t s2 = c->stream2;
   GravArgs a = grav_args(c);
   int rc = GDF_OK;
-  const bool listed = grav_group_list(c, a, c->counters + 16, 16, rc);   // flags and queue
+  const bool listed = grav_group_list(c, a, c->counters + 16, kGravZero, rc);
   GDF_TRY(rc);
   GDF_HIP(c, hipEventRecord(c->ev_dens, c->stream));        // h, zeta, tree, posm are ready
   GDF_HIP(c, hipStreamWaitEvent(s2, c->ev_dens, 0));
   k_pack_grav<<<nblocks(N, 256), 256, 0, s2>>>(N, c->pf[F_H], c->df[D_ZETA], c->df[D_HFACTOR],
                                                  c->grec);
-  a.stacks = c->stacks2; a.counter = c->counters + 24; a.flags = c->counters + 16;
+  a.stacks = c->stacks2;
   a.gwx = c->df[D_GWX]; a.gwy = c->df[D_GWY]; a.gwz = c->df[D_GWZ];
   a.gwp = c->df[D_GWP]; a.gwp0 = c->df[D_GWP0];
   if (!listed) {
-    k_zero8<<<1, 64, 0, s2>>>(c->counters + 24);
-    k_zero8<<<1, 64, 0, s2>>>(c->counters + 16);
+    k_zero_ints<<<1, kGravZero, 0, s2>>>(c->counters + 16);
   }
   const int kt = ktime_begin(c, s2, 5);
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
@@ -942,9 +949,8 @@ int gravity_walk(gdf_ctx* c) {
                                                 c->grec);
   GravArgs a = grav_args(c);
   int rc = GDF_OK;
-  if (!grav_group_list(c, a, c->counters, 12, rc)) {
-    k_zero8<<<1, 64, 0, s>>>(c->counters + 4);
-    k_zero8<<<1, 64, 0, s>>>(c->counters);
+  if (!grav_group_list(c, a, c->counters + 16, kGravZero, rc)) {
+    k_zero_ints<<<1, kGravZero, 0, s>>>(c->counters + 16);
   }
   GDF_TRY(rc);
   const int kt = ktime_begin(c, s, 5);
@@ -953,9 +959,10 @@ int gravity_walk(gdf_ctx* c) {
   else launch_grav<false>(c, a, false, s);
   GDF_HIP(c, hipGetLastError());
   ktime_end(c, s, kt);
-  GDF_HIP(c, hipMemcpyAsync(c->h_counters, c->counters, sizeof(int)*8, hipMemcpyDeviceToHost, s));
+  GDF_HIP(c, hipMemcpyAsync(c->h_counters + 16, c->counters + 16, sizeof(int)*8,
+                            hipMemcpyDeviceToHost, s));
   GDF_HIP(c, hipStreamSynchronize(s));
-  if (c->h_counters[2]) return fail(c, GDF_ERR_CAPACITY, "tree walk stack overflow in gravity pass");
+  if (c->h_counters[16 + 2]) return fail(c, GDF_ERR_CAPACITY, "tree walk stack overflow in gravity pass");
   return GDF_OK;
 }
 

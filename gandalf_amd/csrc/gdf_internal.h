@@ -14,11 +14,15 @@ namespace gdf {
 // Walk groups hold at most one wavefront of targets.
 constexpr int kWave = 64;
 constexpr int kMaxGroup = 64;
-// Persistent wavefronts of the candidate walks (3 per SIMD: 4, 6 and 8 were slower, more walks
-// in flight contending for the caches) and of the gravity walk (4 per SIMD); walk kernels grab
-// groups from a counter.
+// Wavefronts a walk group of the candidate walks, and the persistent workgroups of those and of the
+// gravity walk
+constexpr int kWalkWaves = 2;
 constexpr int kWalkSlots = 3072;
 constexpr int kGravSlots = 4096;
+// The gravity walk's range counters in gdf_ctx::counters, each in a line of its own, and the
+// integers cleared before a walk (its flags, from 16 on, and the range counters)
+constexpr int kGravQueue = 31;
+constexpr int kGravZero = 256;
 // Per-slot stack capacity of the tree walks (node indices); the stack regions serve both walks.
 constexpr int kStackCap = 8192;
 constexpr int kStackSlots = kWalkSlots > kGravSlots ? kWalkSlots : kGravSlots;
@@ -183,9 +187,8 @@ struct gdf_ctx {
   // of the h-rho rounds, [Ncap + 1, 2 Ncap + 1] for the active particles of a block step (the
   // scatter-gather walk and the gravity walk); each list's count follows its Ncap entries
   int* glist = nullptr;
-  int* counters = nullptr;     // [0..7] flags, [4..11] walk range counters, [12..13] block
-                               // reductions; [16..23] flags and [24..31] range counters of the
-                               // gravity walk on the second stream
+  int* counters = nullptr;     // [0..3] flags, [12..13] block reductions; [16..23] flags and
+                               // from kGravQueue on range counters of the gravity walk
   hipStream_t stream2 = nullptr;             // gravity walk beside the hydro pass
   hipEvent_t ev_dens = nullptr, ev_grav = nullptr;
   int* h_counters = nullptr;   // pinned mirror
@@ -293,7 +296,7 @@ void ktime_end(gdf_ctx* c, hipStream_t s, int slot);
 void ktime_collect(gdf_ctx* c);
 // compacted list of the walk groups holding a particle with status[i] == 1 (ascending, count at
 // list[Ncap]); the optional per-group outputs of every other group are cleared, and so are
-// zero[0, nzero) (nzero <= 256: the flags and queue counters of the walk that follows)
+// zero[0, nzero) (nzero <= 256: the flags of the walk that follows)
 int group_list(gdf_ctx* c, const int* status, int* list, int* ncand, int* gnc, int* gnn,
                int* zero = nullptr, int nzero = 0);
 TreeView tree_view(const gdf_ctx* c);

@@ -38,6 +38,8 @@ constexpr double NODE_SLACK = 1.0 + 1e-12; // node tests err on the inclusive si
 // target's own test (FP32 tests of the mixed path included)
 constexpr double KEEP_SLACK = 1.0 + 1e-4;
 constexpr int kInitBatches = 16;           // initial candidate capacity per group, in batches
+constexpr int kMaxLeaf = 14;               // largest bucket (Nleafmax)
+constexpr int kWideStack = 4096;           // stack entries beyond which a round takes 64 nodes
 constexpr int kMaxRounds = 64;             // search radii tried for a particle's h
 constexpr double kMaxGrowth = 23.26;       // between 1.05^64 and 1.05^65: beyond the last of them
 
@@ -52,7 +54,7 @@ struct CandWalk {
   const int* glist;                  // groups to walk (count at glist[Ncap]); NULL = all groups
   int ncap;
   int* idx; unsigned long long* mask; int* ncand;
-  int* stacks; int* counter; int* flags;
+  int* stacks; int* flags;
   PhysParams p;
 };
 
@@ -62,26 +64,33 @@ struct CandWalk {
 // radius reaches the targets' box (hcand = the search radii hs_j = 1.05 h_j; a node's hs bound is
 // 1.05 times its h maximum), so that while no smoothing length outgrows its search radius the
 // list holds the scatter-gather set of the converged smoothing lengths as well.  The lists err on
-// the inclusive side; the pair passes test every pair.  MASKS (the parity tap): also each target's exact scatter-gather set as masks over the list, MODE 1 in FP64 with
+// the inclusive side; the pair passes test every pair.  W wavefronts share a group: a round tests up
+// to 64 W nodes of the group's stack, each wavefront the members of its own buckets.  Bound by the
+// chain of rounds (stack, node, member loads), so wavefronts in flight count: one a group and 3072
+// in all, fetching groups from eight counters on one line, took 870 us at a million particles, 405
+// at 262144 (M4) and 97 at 100003; two a group and 6144 in all take 570, 108 and 67 (20011: 42 and
+// 37; one a group and 4096: 567, 108, 79, 42; four and 8192: 975, 205, 88, 35).  MASKS (the parity tap): also each target's exact scatter-gather set as masks over the list, MODE 1 in FP64 with
 // the oracle's operation order, MODE 2 in FP32 in the frame of the mixed path's pair kernels with
 // their expression.  PER: periodic nearest images.
-template <int MODE, bool PER, bool MASKS = false, bool UNION = false>
-__global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
+template <int MODE, bool PER, int W, bool MASKS = false, bool UNION = false>
+__global__ __launch_bounds__(64*W) void k_walk_cand(CandWalk a) {
+  static_assert(!MASKS || W == 1, "the masks' tests are a lone wavefront's");
   constexpr bool F32 = MODE == 2;      // group-frame FP32 tests
   constexpr bool GATHER = MODE == 0;
   __shared__ double4 sc[MASKS && !F32 ? kWave : 1];   // MODE 1: (x, y, z, (k h_j)^2)
   __shared__ float4 fc[MASKS && F32 ? kWave : 1];     // MODE 2: the same in the FP32 frame
   __shared__ int lstk[kLdsStack];    // node stack; deeper entries go to the global region
-  const int lane = threadIdx.x;
+  __shared__ int kept[W > 1 ? W : 1][W > 1 ? kWave*kMaxLeaf : 1];    // a round's candidates
+  __shared__ int count[W][2];        // a round's opened nodes and candidates
+  const int lane = threadIdx.x & (kWave - 1), wv = W == 1 ? 0 : (int) threadIdx.x/kWave;
   int* stk = a.stacks + (size_t) blockIdx.x*kStackCap;
   const int N = a.N;
   const double krsqd = a.p.kern.rangesqd, kr = a.p.kern.range;
   PhysParams pp = a.p;
   pp.periodic = PER ? 1 : 0;
-  GroupQueue q = group_queue(a.glist ? a.glist[a.ncap] : a.ngroups);
-  for (;;) {
-    const int k = group_next(q, a.counter);
-    if (k >= q.nq) break;
+  const GroupQueue q = group_queue(a.glist ? a.glist[a.ncap] : a.ngroups);
+  for (int k = q.first; k < q.end; k += q.step) {
+    __syncthreads();                 // the last group's stack is done with
     const int g = a.glist ? a.glist[k] : k;
     const int G = a.grp_node[g], gfirst = a.grp_first[g], gcnt = a.grp_count[g];
     // tc, th: the box the walk tests nodes and members against, that of the group's targets
@@ -98,7 +107,7 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
       r2i = range2_rn(krsqd, hG);
     }
     if (__ballot(has) == 0) {        // nothing left to do in this group
-      if (lane == 0) a.ncand[g] = 0;
+      if (threadIdx.x == 0) a.ncand[g] = 0;
       continue;
     }
     hG = wave_max_d(hG);
@@ -115,13 +124,15 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
     const int cap = a.capb*kWave;
     int sp = 1, tail = 0;
     bool overflow = false;
-    if (lane == 0) lstk[0] = a.grp_root ? a.grp_root[g] : 0;   // the group's segment subtree
+    if (threadIdx.x == 0) lstk[0] = a.grp_root ? a.grp_root[g] : 0;  // the group's segment subtree
     __syncthreads();
-    // 1. traversal: the particles of every bucket within range, in walk order, into idx
+    // 1. traversal: the particles of every bucket within range, round by round and wavefront by
+    // wavefront, into idx
     while (sp > 0) {
-      const int b = min(sp, kWave);
+      const int b = min(sp, sp > kWideStack ? kWave : kWave*W);
+      const int slot = wv*kWave + lane;
       int node = -1;
-      if (lane < b) node = stack_get(lstk, stk, sp - 1 - lane);
+      if (slot < b) node = stack_get(lstk, stk, sp - 1 - slot);
       sp -= b;
       bool open = false, emit = false;
       int ef = 0, ec = 0, cl = 0, cr = 0;
@@ -144,15 +155,6 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
         }
       }
       const unsigned long long om = __ballot(open);
-      const int nopen = __popcll(om);
-      if (sp + 2*nopen > kLdsStack + kStackCap) { overflow = true; break; }
-      if (open) {
-        const int o = sp + 2*lanes_below(om);
-        stack_put(lstk, stk, o, cr);
-        stack_put(lstk, stk, o + 1, cl);
-      }
-      sp += 2*nopen;
-      if (sp > kLdsStack) __threadfence_block();   // entries in the global overflow region
       // a bucket's members that lie beyond the largest range from the group box fail every
       // target's test below: they are dropped here, once per member, instead of being tested
       // on all 64 lanes and staged by every pair pass (about a quarter of the members of the
@@ -161,6 +163,7 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
       const int mcount = emit ? ec : 0;
       const int mincl = wave_incl_scan(mcount);
       const int mtot = __shfl(mincl, 63, 64);
+      int nkept = 0;
       for (int base = 0; base < mtot; base += kWave) {
         const int s = base + lane;
         // the lane whose bucket holds member s: the first with an inclusive count above s
@@ -182,23 +185,50 @@ __global__ __launch_bounds__(64) void k_walk_cand(CandWalk a) {
         }
         const unsigned long long km = __ballot(kp);
         if (kp) {
-          const int slot = tail + lanes_below(km);
-          if (slot < cap) idx[slot] = j;
+          const int o = nkept + lanes_below(km);
+          if (W > 1) kept[wv][o] = j;
+          else if (tail + o < cap) idx[tail + o] = j;
         }
-        tail += __popcll(km);
+        nkept += __popcll(km);
       }
+      // places of the round's opened nodes and candidates, wavefront by wavefront
+      int nopen = __popcll(om), o0 = 0;
+      if (W == 1) {
+        tail += nkept;
+      } else {
+        if (lane == 0) { count[wv][0] = nopen; count[wv][1] = nkept; }
+        __syncthreads();
+        int t0 = 0;
+        nopen = 0;
+        #pragma unroll
+        for (int w = 0; w < W; w++) {
+          if (w == wv) { o0 = nopen; t0 = tail; }
+          nopen += count[w][0]; tail += count[w][1];
+        }
+        for (int o = lane; o < nkept; o += kWave)
+          if (t0 + o < cap) idx[t0 + o] = kept[wv][o];
+      }
+      if (sp + 2*nopen > kLdsStack + kStackCap) { overflow = true; break; }
+      if (open) {
+        const int o = sp + 2*(o0 + lanes_below(om));
+        stack_put(lstk, stk, o, cr);
+        stack_put(lstk, stk, o + 1, cl);
+      }
+      sp += 2*nopen;
+      if (sp > kLdsStack) __threadfence_block();   // entries in the global overflow region
+      __syncthreads();
     }
     if (overflow) {
-      if (lane == 0) atomicOr(&a.flags[2], 1);
+      if (threadIdx.x == 0) atomicOr(&a.flags[2], 1);
       continue;
     }
     const int nbat = (tail + kWave - 1)/kWave;
     if (tail > cap) {                // candidates beyond the set's capacity: grow and repeat
-      if (lane == 0) { a.ncand[g] = tail; atomicMax(&a.flags[1], nbat); }
+      if (threadIdx.x == 0) { a.ncand[g] = tail; atomicMax(&a.flags[1], nbat); }
       continue;
     }
     if (!MASKS) {
-      if (lane == 0) a.ncand[g] = tail;
+      if (threadIdx.x == 0) a.ncand[g] = tail;
       continue;
     }
     __threadfence_block();
@@ -896,7 +926,6 @@ int grow_cand(gdf_ctx* c, CandSet& cs, int ng, int need, bool masks) {
 enum WalkKind { WALK_GATHER, WALK_UNION, WALK_SG, WALK_MASKS };
 
 // glist: the groups holding targets (from group_list), or NULL to walk every group
-// (the walk's queue counters, counters[4, 12), must be zero: the list builder clears them)
 int launch_walk(gdf_ctx* c, WalkKind kind, int nopbc, CandSet& cs, const int* status,
                 const int* glist) {
   CandWalk w;
@@ -912,25 +941,26 @@ int launch_walk(gdf_ctx* c, WalkKind kind, int nopbc, CandSet& cs, const int* st
   w.grp_root = c->nseg > 0 ? c->grp_root : nullptr;
   w.glist = glist; w.ncap = c->Ncap;
   w.idx = cs.idx; w.mask = cs.mask; w.ncand = cs.ncand;
-  w.stacks = c->stacks; w.counter = c->counters + 4; w.flags = c->counters;
+  w.stacks = c->stacks; w.flags = c->counters;
   w.p = c->phys;
   if (nopbc) w.p.periodic = 0;
-  if (!glist) k_zero_ints<<<1, BS, 0, c->stream>>>(8, c->counters + 4);
   const int grid = std::min(ng, kWalkSlots);
+  constexpr int W = kWalkWaves;
+  const int nt = kind == WALK_MASKS ? kWave : kWave*W;
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
   hipStream_t st = c->stream;
   if (w.p.periodic) {
-    if (kind == WALK_GATHER) k_walk_cand<0, true><<<grid, kWave, 0, st>>>(w);
-    else if (kind == WALK_UNION) k_walk_cand<0, true, false, true><<<grid, kWave, 0, st>>>(w);
-    else if (kind == WALK_SG) k_walk_cand<1, true><<<grid, kWave, 0, st>>>(w);
-    else if (mixed) k_walk_cand<2, true, true><<<grid, kWave, 0, st>>>(w);
-    else k_walk_cand<1, true, true><<<grid, kWave, 0, st>>>(w);
+    if (kind == WALK_GATHER) k_walk_cand<0, true, W><<<grid, nt, 0, st>>>(w);
+    else if (kind == WALK_UNION) k_walk_cand<0, true, W, false, true><<<grid, nt, 0, st>>>(w);
+    else if (kind == WALK_SG) k_walk_cand<1, true, W><<<grid, nt, 0, st>>>(w);
+    else if (mixed) k_walk_cand<2, true, 1, true><<<grid, nt, 0, st>>>(w);
+    else k_walk_cand<1, true, 1, true><<<grid, nt, 0, st>>>(w);
   } else {
-    if (kind == WALK_GATHER) k_walk_cand<0, false><<<grid, kWave, 0, st>>>(w);
-    else if (kind == WALK_UNION) k_walk_cand<0, false, false, true><<<grid, kWave, 0, st>>>(w);
-    else if (kind == WALK_SG) k_walk_cand<1, false><<<grid, kWave, 0, st>>>(w);
-    else if (mixed) k_walk_cand<2, false, true><<<grid, kWave, 0, st>>>(w);
-    else k_walk_cand<1, false, true><<<grid, kWave, 0, st>>>(w);
+    if (kind == WALK_GATHER) k_walk_cand<0, false, W><<<grid, nt, 0, st>>>(w);
+    else if (kind == WALK_UNION) k_walk_cand<0, false, W, false, true><<<grid, nt, 0, st>>>(w);
+    else if (kind == WALK_SG) k_walk_cand<1, false, W><<<grid, nt, 0, st>>>(w);
+    else if (mixed) k_walk_cand<2, false, 1, true><<<grid, nt, 0, st>>>(w);
+    else k_walk_cand<1, false, 1, true><<<grid, nt, 0, st>>>(w);
   }
   GDF_HIP(c, hipGetLastError());
   return GDF_OK;
@@ -987,9 +1017,9 @@ int sph_density(gdf_ctx* c, int nopbc) {
   const WalkKind kind = uni ? WALK_UNION : WALK_GATHER;
   bool grown = false, retried = false, outgrown = false;
   for (int round = 0; round < kMaxRounds; round++) {
-    // also clears the round's flags and the walk's queue counters
+    // also clears the round's flags
     GDF_TRY(group_list(c, c->status, c->glist, c->cs_g.ncand, nullptr, nullptr, c->counters,
-                       12));
+                       4));
     GDF_TRY(launch_walk(c, kind, nopbc, c->cs_g, c->status, c->glist));
     d.capb = c->cs_g.capb; d.idx = c->cs_g.idx; d.ncand = c->cs_g.ncand;
     if (mixed) launch_density<float>(d, waves, s);
@@ -1017,7 +1047,7 @@ int sph_density(gdf_ctx* c, int nopbc) {
       // first round would have made them with room enough (the radii and the nodes' bounds are
       // still those of its start)
       if (act) GDF_TRY(group_list(c, act, c->glist, c->cs_g.ncand, nullptr, nullptr,
-                                  c->counters, 12));
+                                  c->counters, 4));
       else k_zero_ints<<<1, BS, 0, s>>>(4, c->counters);
       GDF_TRY(launch_walk(c, kind, nopbc, c->cs_g, act, act ? c->glist : nullptr));
       GDF_TRY(read_flags(c));
@@ -1042,7 +1072,7 @@ int sph_build_sg(gdf_ctx* c, bool masks) {
   for (int round = 0; round < 8; round++) {
     const int* act = c->nlevels > 1 ? c->pi[I_ACT] : nullptr;
     int* sl = c->glist + (c->Ncap + 1);
-    if (act) GDF_TRY(group_list(c, act, sl, c->cs_s.ncand, nullptr, nullptr, c->counters, 12));
+    if (act) GDF_TRY(group_list(c, act, sl, c->cs_s.ncand, nullptr, nullptr, c->counters, 4));
     else k_zero_ints<<<1, BS, 0, c->stream>>>(4, c->counters);
     GDF_TRY(launch_walk(c, masks ? WALK_MASKS : WALK_SG, 0, c->cs_s, act, act ? sl : nullptr));
     GDF_TRY(read_flags(c));

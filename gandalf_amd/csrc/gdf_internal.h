@@ -152,7 +152,7 @@ struct gdf_ctx {
   int* vals = nullptr; int* vals_alt = nullptr;
   void* sort_tmp = nullptr; size_t sort_tmp_bytes = 0;
   int* left = nullptr; int* right = nullptr; int* first = nullptr; int* last = nullptr;
-  int* parent = nullptr; int* visit = nullptr;
+  int* parent = nullptr; int* visit = nullptr;   // visit: scratch of the group selections
   int4* lnk = nullptr;          // internal node: (first, last, left, right) in one 16-byte record
   int* front = nullptr;                                // refit frontier [N] + count
   double4* geo_c = nullptr; double4* geo_h = nullptr;

@@ -74,7 +74,7 @@ __global__ __launch_bounds__(BS) void k_bounds_final(int nb, const double* __res
 // ---- serving batches: per-segment bounds and segment-prefixed keys ----
 // partial-reduction blocks per segment: kMaxSeg x 16 x 6 partials fit the reduction buffer
 constexpr int kSegBlocks = 16;
-constexpr int kSelBlock = 256;      // workgroup of the flag selection; 16 flags per thread
+constexpr int kSelBlock = 256;      // workgroup of the group selection
 
 // grid (kSegBlocks, nseg): block (b, s) folds a strided share of segment s
 __global__ void k_seg_bounds_partial(const int* __restrict__ off, const double* __restrict__ x,
@@ -133,9 +133,11 @@ __device__ __forceinline__ uint64_t spread3(uint64_t x) {
 
 __global__ void k_morton(int N, const double* __restrict__ x, const double* __restrict__ y,
                          const double* __restrict__ z, const double* __restrict__ bnd,
-                         uint64_t* __restrict__ keys, int* __restrict__ vals) {
+                         uint64_t* __restrict__ keys, int* __restrict__ vals,
+                         int* __restrict__ gstart) {
   const int i = blockIdx.x*BS + threadIdx.x;
   if (i >= N) return;
+  gstart[i] = -1;                       // k_lbvh marks the group starts
   const double scale = bnd[3];
   const double v[3] = {x[i], y[i], z[i]};
   uint64_t q[3];
@@ -192,9 +194,10 @@ __device__ __forceinline__ int delta(const uint64_t* __restrict__ key, int N, in
 __global__ void k_morton_seg(int N, const double* __restrict__ x, const double* __restrict__ y,
                              const double* __restrict__ z, const int* __restrict__ seg,
                              const double* __restrict__ bnd, uint64_t* __restrict__ keys,
-                             int* __restrict__ vals) {
+                             int* __restrict__ vals, int* __restrict__ gstart) {
   const int i = blockIdx.x*BS + threadIdx.x;
   if (i >= N) return;
+  gstart[i] = -1;                       // k_lbvh marks the group starts
   const int sg = seg[i];
   const double scale = bnd[4*sg + 3];
   const double v[3] = {x[i], y[i], z[i]};
@@ -271,8 +274,10 @@ __global__ void k_grp_roots(int ngroups, const int* __restrict__ grp_first,
   if (g < ngroups) grp_root[g] = root[seg[grp_first[g]]];
 }
 
-// Karras 2012, "Maximizing parallelism in the construction of BVHs, octrees, and k-d trees"
-__global__ void k_lbvh(int N, const uint64_t* __restrict__ key, int* __restrict__ left,
+// Karras 2012, "Maximizing parallelism in the construction of BVHs, octrees, and k-d trees".  The
+// walk groups are the maximal nodes of at most gmax particles: a node of more marks those of its
+// children that are groups, with their sizes, at their first particles.
+__global__ void k_lbvh(int N, int gmax, int* __restrict__ gstart, int* __restrict__ gsize, const uint64_t* __restrict__ key, int* __restrict__ left,
                        int* __restrict__ right, int* __restrict__ first, int* __restrict__ last,
                        int* __restrict__ parent, int4* __restrict__ lnk) {
   const int i = blockIdx.x*BS + threadIdx.x;
@@ -301,6 +306,13 @@ __global__ void k_lbvh(int N, const uint64_t* __restrict__ key, int* __restrict_
   lnk[i] = make_int4(f, la, L, R);
   parent[L] = i; parent[R] = i;
   if (i == 0) parent[0] = -1;
+  if (la - f + 1 > gmax) {
+    if (gamma - f + 1 <= gmax) { gstart[f] = L; gsize[f] = gamma - f + 1; }
+    if (la - gamma <= gmax) { gstart[gamma + 1] = R; gsize[gamma + 1] = la - gamma; }
+  } else if (i == 0) {
+    gstart[0] = 0;
+    gsize[0] = N;
+  }
 }
 
 struct NodeArgs {
@@ -310,11 +322,11 @@ struct NodeArgs {
 __global__ void k_leaves(int N, const double* __restrict__ x, const double* __restrict__ y,
                          const double* __restrict__ z, const double* __restrict__ m,
                          const double* __restrict__ h, double theta2, NodeArgs a,
-                         int* __restrict__ visit, int* __restrict__ parent) {
+                         int* __restrict__ parent, int* __restrict__ gstart,
+                         int* __restrict__ gsize) {
   const int l = blockIdx.x*BS + threadIdx.x;
   if (l >= N) return;
-  if (l < N - 1) visit[l] = 0;
-  if (N == 1) parent[0] = -1;
+  if (N == 1) { parent[0] = -1; gstart[0] = 0; gsize[0] = 1; }
   const int n = N - 1 + l;
   const double r[3] = {x[l], y[l], z[l]};
   const double hh = h[l];
@@ -473,7 +485,7 @@ __global__ __launch_bounds__(RB) void k_refit_chunks(
     int N, const double* __restrict__ x, const double* __restrict__ y,
     const double* __restrict__ z, const double* __restrict__ mass, const double* __restrict__ h,
     const int* __restrict__ parent, const int4* __restrict__ lnk, double theta2, NodeArgs a,
-    int* __restrict__ visit, int* __restrict__ front, int* __restrict__ nfront) {
+    int* __restrict__ front, int* __restrict__ nfront) {
 #pragma clang fp contract(off)
   __shared__ RefitSlots<HONLY, RB> sd;
   __shared__ int arr[RB];               // arrivals at internal node c0 + t
@@ -502,7 +514,6 @@ __global__ __launch_bounds__(RB) void k_refit_chunks(
         const int split = k.z >= N - 1 ? k.z - (N - 1) : k.z;      // last leaf of the left child
         lr[t] = (k.x - c0) | (split + 1 - c0) << 16;
       }
-      visit[l] = 0;
       if (HONLY) rmax2 = box_rmax2(a, l);
     }
     const int n = N - 1 + l;
@@ -693,8 +704,8 @@ void launch_refit(gdf_ctx* c, const NodeArgs& na, double theta2) {
   int* nfrom = to + N;
   int* nto = nfrom + nrun;
   k_refit_chunks<HONLY><<<nrun, RB, 0, s>>>(N, c->pf[F_X], c->pf[F_Y], c->pf[F_Z], c->pf[F_M],
-                                            c->pf[F_H], c->parent, c->lnk, theta2, na, c->visit,
-                                            from, nfrom);
+                                            c->pf[F_H], c->parent, c->lnk, theta2, na, from,
+                                            nfrom);
   for (long long span = RB; nrun > 1; span *= RS) {
     const int nb = (nrun + RS - 1)/RS;
     k_refit_runs<HONLY><<<nb, RT, 0, s>>>(N, nrun, span, c->parent, c->lnk, theta2, na, from, nfrom,
@@ -705,43 +716,13 @@ void launch_refit(gdf_ctx* c, const NodeArgs& na, double theta2) {
   }
 }
 
-__global__ void k_hleaves(int N, const double* __restrict__ h, double theta2, NodeArgs a,
-                          int* __restrict__ visit) {
+__global__ void k_hleaves(int N, const double* __restrict__ h, double theta2, NodeArgs a) {
   const int l = blockIdx.x*BS + threadIdx.x;
   if (l >= N) return;
-  if (l < N - 1) visit[l] = 0;
   const int n = N - 1 + l;
   const double hh = h[l];
   double4 gc = a.geo_c[n]; gc.w = hh; a.geo_c[n] = gc;
   double4 gh = a.geo_h[n]; gh.w = __ddiv_rn(__dmul_rn(hh, hh), theta2); a.geo_h[n] = gh;
-}
-
-// a node is a walk group iff it holds <= gmax particles and its parent holds more
-__global__ void k_groups_mark(int N, int gmax, const int* __restrict__ parent,
-                              const int* __restrict__ first, const int* __restrict__ last,
-                              int* __restrict__ gstart, unsigned char* __restrict__ gflag) {
-  const int n = blockIdx.x*BS + threadIdx.x;
-  if (n >= 2*N - 1) return;
-  const int cnt = n >= N - 1 ? 1 : last[n] - first[n] + 1;
-  const int fst = n >= N - 1 ? n - (N - 1) : first[n];
-  if (cnt > gmax) return;
-  const int p = parent[n];
-  const int pcnt = p < 0 ? 0x7fffffff : last[p] - first[p] + 1;
-  if (p >= 0 && pcnt <= gmax) return;
-  gstart[fst] = n;
-  gflag[fst] = 1;
-}
-
-__global__ void k_groups_fill(int N, const int* __restrict__ nsel, const int* __restrict__ slots,
-                              const int* __restrict__ gstart, const int* __restrict__ first,
-                              const int* __restrict__ last, int* __restrict__ gnode,
-                              int* __restrict__ gcount) {
-  const int g = blockIdx.x*BS + threadIdx.x;
-  if (g >= *nsel) return;
-  const int s = slots[g];
-  const int n = gstart[s];
-  gnode[g] = n;
-  gcount[g] = n >= N - 1 ? 1 : last[n] - first[n] + 1;
 }
 
 // Order-preserving compaction of n byte flags (0 or 1) into the indices of the set ones
@@ -859,7 +840,7 @@ int tree_alloc(gdf_ctx* c) {
   GDF_HIP(c, hipMalloc(&c->last, sizeof(int)*N));
   GDF_HIP(c, hipMalloc(&c->parent, sizeof(int)*nn));
   GDF_HIP(c, hipMalloc(&c->lnk, sizeof(int4)*N));
-  GDF_HIP(c, hipMalloc(&c->visit, sizeof(int)*(N + 16)));   // also 16-byte-padded flags
+  GDF_HIP(c, hipMalloc(&c->visit, sizeof(int)*(N + 16)));   // 16-byte-padded byte flags
   // refit frontiers: phase 1 (one RB slot per chunk), chunk counts, phase 2 (N + count)
   GDF_HIP(c, hipMalloc(&c->front, sizeof(int)*(2*N + 2*(N/1024 + 16))));
   GDF_HIP(c, hipMalloc(&c->geo_c, sizeof(double4)*nn));
@@ -886,76 +867,109 @@ int tree_alloc(gdf_ctx* c) {
 
 namespace {
 
-// Order-preserving selection of the set bytes of n 0/1 byte flags (zero-padded to whole
-// 16-byte words): per-block counts, an exclusive scan of the block counts by one workgroup, and
-// a per-block scatter of the indices.  No memset and no library call, so the tree build's
-// launches capture into a graph of kernel nodes only.
-__device__ __forceinline__ int bytes_set(uint4 w) {
-  // each byte is 0 or 1: the byte sum of a word is its top byte after multiplying by 0x01010101
-  return (int) (((w.x*0x01010101u) >> 24) + ((w.y*0x01010101u) >> 24) +
-                ((w.z*0x01010101u) >> 24) + ((w.w*0x01010101u) >> 24));
+// The marked group starts (gstart[i] >= 0: the group's node) in ascending order: per-block counts,
+// an exclusive scan of them by one workgroup, and a scatter of the groups' first particles, nodes
+// and sizes; up to kSelSmall particles all in one workgroup.  No memset and no library call, so the
+// tree build's launches capture into a graph of kernel nodes only.  (Marked by a pass over all
+// nodes into cleared byte flags, with a pass over the groups for their nodes, it was six launches, 21
+// to 28 us and the gaps between them; now 4 us for 4096 particles, 14 for 20011, 17 in three launches
+// for 131072.)
+constexpr int kSelPer = 16;                // particles a thread
+constexpr int kSelSmall = 32768;
+
+struct SelOut { int* first; int* node; int* count; };
+
+// marks i .. i + 3 of N (unmarked past the end)
+__device__ __forceinline__ int4 sel_marks(int N, int i, const int* __restrict__ gstart) {
+  if (i + 3 < N) return *reinterpret_cast<const int4*>(gstart + i);
+  return make_int4(i < N ? gstart[i] : -1, i + 1 < N ? gstart[i + 1] : -1,
+                   i + 2 < N ? gstart[i + 2] : -1, -1);
+}
+__device__ __forceinline__ int sel_count(int4 m) {
+  return (m.x >= 0) + (m.y >= 0) + (m.z >= 0) + (m.w >= 0);
+}
+__device__ __forceinline__ int sel_write(int4 m, int i, int o, const int* __restrict__ gsize,
+                                         const SelOut& out) {
+  const int n[4] = {m.x, m.y, m.z, m.w};
+  #pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (n[k] >= 0) {
+      out.first[o] = i + k; out.node[o] = n[k]; out.count[o] = gsize[i + k];
+      o++;
+    }
+  return o;
 }
 
-__global__ __launch_bounds__(kSelBlock) void k_sel_count(int nw, const uint4* __restrict__ flags,
+// exclusive scan over a workgroup of up to 16 wavefronts, its sum into total
+__device__ __forceinline__ int block_scan(int v, int& total) {
+  __shared__ int sum[16];
+  const int w = threadIdx.x/kWave;
+  const int incl = wave_incl_scan(v);
+  if ((threadIdx.x & (kWave - 1)) == kWave - 1) sum[w] = incl;
+  __syncthreads();
+  int before = 0;
+  total = 0;
+  for (int k = 0; k < (int) blockDim.x/kWave; k++) {
+    if (k < w) before += sum[k];
+    total += sum[k];
+  }
+  __syncthreads();
+  return before + incl - v;
+}
+
+__global__ __launch_bounds__(1024) void k_sel_small(int N, const int* __restrict__ gstart,
+                                                    const int* __restrict__ gsize,
+                                                    int* __restrict__ ngroups, SelOut out) {
+  int run = 0;
+  int4 next = sel_marks(N, 4*threadIdx.x, gstart);
+  for (int base = 0; base < N; base += 4096) {
+    const int i = base + 4*threadIdx.x;
+    const int4 m = next;
+    next = sel_marks(N, i + 4096, gstart);
+    int total;
+    const int o = run + block_scan(sel_count(m), total);
+    sel_write(m, i, o, gsize, out);
+    run += total;
+  }
+  if (threadIdx.x == 0) *ngroups = run;
+}
+
+__global__ __launch_bounds__(kSelBlock) void k_sel_count(int N, const int* __restrict__ gstart,
                                                          int* __restrict__ bcount) {
-  __shared__ int red[kSelBlock];
-  const int w = blockIdx.x*kSelBlock + threadIdx.x;
-  red[threadIdx.x] = w < nw ? bytes_set(flags[w]) : 0;
-  __syncthreads();
-  for (int st = kSelBlock/2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) bcount[blockIdx.x] = red[0];
+  const int i0 = (blockIdx.x*kSelBlock + threadIdx.x)*kSelPer;
+  int c = 0, total;
+  for (int i = i0; i < i0 + kSelPer; i += 4) c += sel_count(sel_marks(N, i, gstart));
+  (void) block_scan(c, total);
+  if (threadIdx.x == 0) bcount[blockIdx.x] = total;
 }
 
-// exclusive scan of nb block counts in place, the total into *total; one workgroup
-__global__ __launch_bounds__(kSelBlock) void k_sel_scan(int nb, int* __restrict__ bcount,
-                                                        int* __restrict__ total) {
-  __shared__ int part[kSelBlock];
-  const int per = (nb + kSelBlock - 1)/kSelBlock;
-  const int b0 = min(threadIdx.x*per, nb), b1 = min(b0 + per, nb);
-  int sum = 0;
+// exclusive scan of nb block counts in place, the total into *ngroups; one workgroup
+__global__ __launch_bounds__(1024) void k_sel_scan(int nb, int* __restrict__ bcount,
+                                                   int* __restrict__ ngroups) {
+  const int per = (nb + 1023)/1024;
+  const int b0 = min((int) threadIdx.x*per, nb), b1 = min(b0 + per, nb);
+  int sum = 0, total;
   for (int b = b0; b < b1; b++) sum += bcount[b];
-  part[threadIdx.x] = sum;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int t = 0; t < kSelBlock; t++) { const int v = part[t]; part[t] = run; run += v; }
-    *total = run;
-  }
-  __syncthreads();
-  int run = part[threadIdx.x];
+  int run = block_scan(sum, total);
   for (int b = b0; b < b1; b++) { const int v = bcount[b]; bcount[b] = run; run += v; }
+  if (threadIdx.x == 0) *ngroups = total;
 }
 
-__global__ __launch_bounds__(kSelBlock) void k_sel_scatter(int nw, const uint4* __restrict__ flags,
+__global__ __launch_bounds__(kSelBlock) void k_sel_scatter(int N, const int* __restrict__ gstart,
+                                                           const int* __restrict__ gsize,
                                                            const int* __restrict__ boff,
-                                                           int* __restrict__ out) {
-  __shared__ int pre[kSelBlock];
-  const int w = blockIdx.x*kSelBlock + threadIdx.x;
-  const uint4 x = w < nw ? flags[w] : make_uint4(0u, 0u, 0u, 0u);
-  const int cnt = bytes_set(x);
-  pre[threadIdx.x] = cnt;
-  __syncthreads();
-  for (int st = 1; st < kSelBlock; st <<= 1) {          // inclusive scan (Hillis-Steele)
-    const int v = threadIdx.x >= st ? pre[threadIdx.x - st] : 0;
-    __syncthreads();
-    pre[threadIdx.x] += v;
-    __syncthreads();
+                                                           SelOut out) {
+  const int i0 = (blockIdx.x*kSelBlock + threadIdx.x)*kSelPer;
+  int4 m[kSelPer/4];
+  int c = 0, total;
+  #pragma unroll
+  for (int k = 0; k < kSelPer/4; k++) {
+    m[k] = sel_marks(N, i0 + 4*k, gstart);
+    c += sel_count(m[k]);
   }
-  if (cnt == 0) return;
-  int o = boff[blockIdx.x] + pre[threadIdx.x] - cnt;
-  const unsigned int word[4] = {x.x, x.y, x.z, x.w};
-  for (int k = 0; k < 16; k++)
-    if ((word[k >> 2] >> (8*(k & 3))) & 0xffu) out[o++] = 16*w + k;
-}
-
-// The byte flags of the group selection, cleared by a kernel (a memset would become a memset
-// node of the captured graph)
-__global__ void k_zero_words(int n, uint4* __restrict__ p) {
-  const int i = blockIdx.x*BS + threadIdx.x;
-  if (i < n) p[i] = make_uint4(0u, 0u, 0u, 0u);
+  int o = boff[blockIdx.x] + block_scan(c, total);
+  #pragma unroll
+  for (int k = 0; k < kSelPer/4; k++) o = sel_write(m[k], i0 + 4*k, o, gsize, out);
 }
 
 // Steps 1-6 of a tree build: every launch that needs no value back on the host.  The host's
@@ -973,12 +987,12 @@ int build_body(gdf_ctx* c, hipStream_t s, bool launch) {
                                                                     c->red);
       k_seg_bounds_final<<<c->nseg, 64, 0, s>>>(c->red, c->seg_bnd);
       k_morton_seg<<<nblocks(N, BS), BS, 0, s>>>(N, c->pf[F_X], c->pf[F_Y], c->pf[F_Z],
-                                                 c->pi[I_SEG], c->seg_bnd, c->keys, c->vals);
+                                                 c->pi[I_SEG], c->seg_bnd, c->keys, c->vals, c->gstart);
     } else {
       k_bounds_partial<<<nbp, BS, 0, s>>>(N, c->pf[F_X], c->pf[F_Y], c->pf[F_Z], c->red);
       k_bounds_final<<<1, BS, 0, s>>>(nbp, c->red, c->red + 6*1024);
       k_morton<<<nblocks(N, BS), BS, 0, s>>>(N, c->pf[F_X], c->pf[F_Y], c->pf[F_Z],
-                                             c->red + 6*1024, c->keys, c->vals);
+                                             c->red + 6*1024, c->keys, c->vals, c->gstart);
     }
     // 2. stable radix sort of (key, index)
     size_t bytes = c->sort_tmp_bytes;
@@ -1011,7 +1025,7 @@ int build_body(gdf_ctx* c, hipStream_t s, bool launch) {
   if (!launch) return GDF_OK;
   // 4. topology
   if (N > 1)
-    k_lbvh<<<nblocks(N - 1, BS), BS, 0, s>>>(N, c->keys, c->left, c->right, c->first, c->last,
+    k_lbvh<<<nblocks(N - 1, BS), BS, 0, s>>>(N, c->cfg.group_max, c->gstart, c->visit, c->keys, c->left, c->right, c->first, c->last,
                                              c->parent, c->lnk);
   // 5. moments, bottom-up
   NodeArgs na = node_args(c);
@@ -1020,21 +1034,18 @@ int build_body(gdf_ctx* c, hipStream_t s, bool launch) {
     launch_refit<false>(c, na, theta2);
   else
     k_leaves<<<1, BS, 0, s>>>(N, c->pf[F_X], c->pf[F_Y], c->pf[F_Z], c->pf[F_M], c->pf[F_H],
-                              theta2, na, c->visit, c->parent);
+                              theta2, na, c->parent, c->gstart, c->visit);
   // 6. walk groups in ascending first-particle order
-  const int nw = (N + 15)/16;                // N byte flags, padded to 16 bytes
-  k_zero_words<<<nblocks(nw, BS), BS, 0, s>>>(nw, reinterpret_cast<uint4*>(c->visit));
-  k_groups_mark<<<nblocks(2*N - 1, BS), BS, 0, s>>>(N, c->cfg.group_max, c->parent, c->first,
-                                                    c->last, c->gstart,
-                                                    (unsigned char*) c->visit);
-  const int nsb = nblocks(nw, kSelBlock);
-  int* bcount = reinterpret_cast<int*>(c->sel_tmp);
-  const uint4* fw = reinterpret_cast<const uint4*>(c->visit);
-  k_sel_count<<<nsb, kSelBlock, 0, s>>>(nw, fw, bcount);
-  k_sel_scan<<<1, kSelBlock, 0, s>>>(nsb, bcount, c->nsel);
-  k_sel_scatter<<<nsb, kSelBlock, 0, s>>>(nw, fw, bcount, c->grp_first);
-  k_groups_fill<<<nblocks(N, BS), BS, 0, s>>>(N, c->nsel, c->grp_first, c->gstart, c->first,
-                                              c->last, c->grp_node, c->grp_count);
+  const SelOut out = {c->grp_first, c->grp_node, c->grp_count};
+  if (N <= kSelSmall) {
+    k_sel_small<<<1, 1024, 0, s>>>(N, c->gstart, c->visit, c->nsel, out);
+  } else {
+    const int nsb = nblocks(nblocks(N, kSelPer), kSelBlock);
+    int* bcount = reinterpret_cast<int*>(c->sel_tmp);
+    k_sel_count<<<nsb, kSelBlock, 0, s>>>(N, c->gstart, bcount);
+    k_sel_scan<<<1, 1024, 0, s>>>(nsb, bcount, c->nsel);
+    k_sel_scatter<<<nsb, kSelBlock, 0, s>>>(N, c->gstart, c->visit, bcount, out);
+  }
   GDF_HIP(c, hipGetLastError());
   return GDF_OK;
 }
@@ -1208,7 +1219,7 @@ int tree_restock(gdf_ctx* c) {
     launch_refit<false>(c, na, theta2);
   else
     k_leaves<<<1, BS, 0, s>>>(N, c->pf[F_X], c->pf[F_Y], c->pf[F_Z], c->pf[F_M], c->pf[F_H],
-                              theta2, na, c->visit, c->parent);
+                              theta2, na, c->parent, c->gstart, c->visit);
   GDF_HIP(c, hipGetLastError());
   GDF_TRY(group_mac(c, nullptr));
   GDF_TRY(integ_pack_posm(c));
@@ -1222,7 +1233,6 @@ int group_list(gdf_ctx* c, const int* status, int* list, int* ncand, int* gnc, i
                int* zero, int nzero) {
   const int ng = c->ngroups;
   hipStream_t s = c->stream;
-  // the refit's arrival counters are free between tree passes (phase 1 clears them)
   unsigned char* flags = reinterpret_cast<unsigned char*>(c->visit);
   constexpr int gpb = BS/kWave;   // groups per block
   k_group_flags<<<(ng + gpb - 1)/gpb, BS, 0, s>>>(ng, c->grp_first, c->grp_count, status, flags,
@@ -1241,7 +1251,7 @@ int tree_refit_h(gdf_ctx* c) {
   if (N > 1)
     launch_refit<true>(c, na, theta2);
   else
-    k_hleaves<<<1, BS, 0, s>>>(N, c->pf[F_H], theta2, na, c->visit);
+    k_hleaves<<<1, BS, 0, s>>>(N, c->pf[F_H], theta2, na);
   GDF_HIP(c, hipGetLastError());
   return GDF_OK;
 }

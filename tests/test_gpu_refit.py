@@ -1,7 +1,7 @@
 """The tree's bottom-up passes at the edges of their phases: one chunk of 1024 leaves, the first
 leaf of a second one, one workgroup of 32 chunks and the first leaf past it, and a cloud of nearly
 chain-like subtrees whose chunks leave more nodes than a workgroup of the later phases holds at a
-time.  Every node's moments, box and smoothing-length bound equal the twin's bit for bit (the
+time.  The walk groups (selected by one workgroup up to 32768 particles), every node's moments, box and smoothing-length bound equal the twin's bit for bit (the
 quadrupoles to rounding, as in the twin's other comparisons); so do the bounds after the h-rho pass
 (the pass over the smoothing lengths alone)."""
 import numpy as np
@@ -49,7 +49,8 @@ def test_moments_match_twin_at_phase_edges(kind, N):
     if kind == "chains":
         assert left_by_chunks(t, N) > 768
     a = s.tree_arrays()
-    for k in ("perm", "first", "last", "mass", "com", "quad", "bbmin", "bbmax", "hmax"):
+    for k in ("perm", "first", "last", "mass", "com", "quad", "bbmin", "bbmax", "hmax",
+              "group_first", "group_count", "group_node"):
         if k == "quad":
             assert np.max(np.abs(a[k] - t[k])) <= 1e-14 * max(np.max(np.abs(t[k])), 1e-300), k
         else:

@@ -385,8 +385,12 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
   if (nc <= 0 || nc > a.capb*kWave) return;   // no active target, or the walk overflowed
   const int gfirst = a.grp_first[g], gcnt = a.grp_count[g];
   Rec* const st = stage[wv];
-  const int i = gfirst + lane;
-  const bool has = lane < gcnt && a.status[i] == 1;
+  const unsigned long long on = __ballot(lane < gcnt && a.status[gfirst + lane] == 1);
+  if (on == 0) return;
+  const TargetLanes tl(on);
+  const bool has = tl.has, writes = wv == 0 && tl.copy == 0;
+  const int i = has ? gfirst + tl.member : 0;
+  const unsigned mine = tl.share();
   int state = has ? 2 : 3;                    // 2 iterating, 3 not a target
   PhysParams p = a.p;
   if (a.nopbc) p.periodic = 0;
@@ -451,7 +455,7 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
         f.state = !pb.filled(b, l) ? 1 : all ? -1 : 0;
         return f;
       });
-      hq.stage(b == 0, run ? hit : make_uint2(0u, 0u));
+      hq.stage(b == 0, run ? make_uint2(hit.x & mine, hit.y & mine) : make_uint2(0u, 0u));
       const int need = b + 1 < pb.nb ? hq.older : hq.staged;
       if constexpr (F64) {
         hq.run(need, rec, [&](int q) { return st[q]; }, [&](const Rec& pj, bool take) {
@@ -474,7 +478,8 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
       wave_lds_order();
     }
     evals += hq.staged;
-    double r_ = sum.r, om_ = sum.o, z_ = sum.z;
+    double r_ = tl.over_copies(sum.r), om_ = tl.over_copies(sum.o), z_ = tl.over_copies(sum.z);
+    inside = tl.over_copies(inside);
     if (W > 1) {
       red[wv][0][lane] = r_; red[wv][1][lane] = om_; red[wv][2][lane] = z_;
       __syncthreads();
@@ -492,14 +497,14 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
       if (rc == 1) {
         // converged: the sums and the bracket go to k_hrho_finish (status 2), which keeps
         // the final h, grad-h terms and EOS out of this kernel's register budget
-        if (wv == 0) {
+        if (writes) {
           a.rho[i] = rho; a.invomega[i] = invomega; a.zeta[i] = zeta; a.hfactor[i] = h_lower;
           a.status[i] = 2;
         }
-        ngather = inside;
+        ngather = tl.copy == 0 ? inside : 0;
         state = 1;
       } else if (rc == 0) {
-        if (wv == 0) {
+        if (writes) {
           // a larger search radius (k_hrho_finish, status 3) for an h past this one's
           a.hfactor[i] = h;
           a.status[i] = 3;
@@ -507,7 +512,7 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
         }
         state = 0;
       } else if (rc < 0) {
-        if (wv == 0) {
+        if (writes) {
           a.status[i] = 0;
           atomicOr(&a.flags[3], 1);
         }
@@ -659,8 +664,12 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
   if (nc <= 0) return;                        // no target in this group
   const int gfirst = a.grp_first[g], gcnt = a.grp_count[g];
   HydroStage<T, VAR, BLK>& st = stage[wv];
-  const int i = gfirst + lane;
-  const bool has = lane < gcnt && (!BLK || a.act[i] != 0);
+  const unsigned long long on = __ballot(lane < gcnt && (!BLK || a.act[gfirst + lane] != 0));
+  if (on == 0) return;
+  const TargetLanes tl(on);
+  const bool has = tl.has, writes = wv == 0 && tl.copy == 0;
+  const int i = has ? gfirst + tl.member : 0;
+  const unsigned mine = tl.share();
   const PhysParams& p = a.p;
   const double krsqd = p.kern.rangesqd;
   const double4 gc = a.geo_c[a.grp_node[g]], gh = a.geo_h[a.grp_node[g]];
@@ -742,7 +751,7 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
       f.thr = filter_thr((float) ((double) r2*fs*fs));
       return f;
     });
-    hq.stage(b == 0, has ? hit : make_uint2(0u, 0u));
+    hq.stage(b == 0, has ? make_uint2(hit.x & mine, hit.y & mine) : make_uint2(0u, 0u));
     const int need = b + 1 < pb.nb ? hq.older : hq.staged;
     HydroSums<T> part;
     if (F64) sum.to(part);
@@ -797,6 +806,15 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
     else sum.add(part);
     wave_lds_order();
   }
+  if (tl.copies > 1) {
+    sum.ax = tl.over_copies(sum.ax); sum.ay = tl.over_copies(sum.ay); sum.az = tl.over_copies(sum.az);
+    sum.du = tl.over_copies(sum.du); sum.dv = tl.over_copies(sum.dv);
+    if (VAR == 1) {
+      sum.gx = tl.over_copies(sum.gx); sum.gy = tl.over_copies(sum.gy);
+      sum.gz = tl.over_copies(sum.gz); sum.gp = tl.over_copies(sum.gp);
+    }
+    if (BLK) for (int o = tl.span; o < kWave; o <<= 1) lmax = max(lmax, __shfl_xor(lmax, o, kWave));
+  }
   if (W > 1) {
     // the wavefronts' sums, added in order by the first
     double v[NS] = {sum.ax, sum.ay, sum.az, sum.du, sum.dv};
@@ -823,8 +841,8 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
   }
   wave_add_ll(&a.icount[1], npairs);
   // the filter's candidate-target tests (counted for the mixed path)
-  if (!F64) wave_add_ll(&a.icount[5], has && wv == 0 ? nc : 0);
-  if (!has || wv != 0) return;
+  if (!F64) wave_add_ll(&a.icount[5], has && writes ? nc : 0);
+  if (!has || !writes) return;
   if (BLK) a.levelneib[i] = lmax;
   const double dvd = sum.dv*mB.x;
   const double dud = sum.du - a.pressure[i]*dvd*mB.x*a.invomega[i];

@@ -473,7 +473,7 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
           inside += take & (ssqd < (float) rsq);
           part.add(p.kern, ssqd, take ? pj.w : 0.f);
         });
-        sum.r += (double) part.r; sum.o += (double) part.o; sum.z += (double) part.z;
+        sum.r += part.r; sum.o += (double) part.o; sum.z += (double) part.z;
       }
       wave_lds_order();
     }

@@ -180,8 +180,8 @@ struct HitQueue {
   // pair(record, take) until every lane has taken `need` hits; rec: the record of the hit popped
   // last, read while the one before it is evaluated.  Every lane runs every trip (no execution
   // mask changes): with !take the record is slot 0's.  The test stands at the loop's end: with it
-  // at the head the compiler kept the sums before and after a pair apart, 22 of a hydro trip's
-  // 190 vector instructions being moves (1M particles, quintic, FP32: 9.34 against 9.09 ms a
+  // at the head the compiler kept the sums before and after a pair apart, 32 of a hydro trip's
+  // 204 vector instructions more (1M particles, quintic, FP32: 9.34 against 9.09 ms a
   // force evaluation; FP64 11.57 against 11.33).
   template <class R, class L, class P>
   __device__ __forceinline__ void run(int need, R& rec, L load, P pair) {

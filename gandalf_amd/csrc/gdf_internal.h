@@ -326,8 +326,8 @@ void sph_free_lists(gdf_ctx* c);
 int sph_copy_sg(gdf_ctx* c, std::vector<int>& idx, std::vector<unsigned long long>& mask,
                 std::vector<int>& ncand, int& capb);
 int sph_density(gdf_ctx* c, int nopbc);
-// masks: also record each target's candidate masks (the mixed path's hydro kernel otherwise
-// tests its candidates itself)
+// masks: also record each target's exact set as masks over the candidates (the parity tap; the
+// hydro kernel tests its candidates itself)
 int sph_build_sg(gdf_ctx* c, bool masks = false);
 int sph_hydro(gdf_ctx* c, int variant);
 

@@ -5,10 +5,9 @@
 // per-particle physics of GradhSph::ComputeH (src/GradhSph/GradhSph.cpp:142-326) and
 // ComputeSphHydroForces / ComputeSphHydroGravForces (:361-460, :474-585).
 //
-// Work mapping: a walk pass (one wavefront per walk group, a tree node of up to 64
+// Work mapping: a walk pass (two wavefronts per walk group, a tree node of up to 64
 // Morton-consecutive particles) resolves the group's candidate particles from the tree: the
-// members of every bucket that come within the group's search range, in walk order.  The h-rho
-// pass walks with bounds that also hold the scatter-gather sets of the converged smoothing
+// members of every bucket that come within the group's search range.  The h-rho pass walks with bounds that also hold the scatter-gather sets of the converged smoothing
 // lengths, so the force pass reads the same lists.  A pair pass takes one walk group per
 // workgroup, one target a lane, and its wavefronts share the group's candidates: each stages its
 // own in LDS batch by batch, filters them against the 64 targets on the matrix cores
@@ -18,9 +17,9 @@
 //
 // The lists hold no masks: exact 64-bit masks per batch and target, made by the walk with 64
 // distance tests a candidate and read back by the pair passes, cost 12 to 19 VALU instructions a
-// test and 640 bytes a batch, and the FP64 force pass a walk of its own.  One FP64 force
-// evaluation of a million particles (quintic, 64-particle groups) takes 13.2 ms against 17.2 ms
-// with them: walks 0.88 against 1.51 + 1.52 ms, h-rho pass 1.51 (1.59), hydro pass 3.45 (5.06).
+// test and 640 bytes a batch, and the FP64 force pass a walk of its own.  Without them one FP64
+// force evaluation of a million particles (quintic, 64-particle groups) went from 17.2 to 13.2 ms
+// (11.3 with the later changes described at each kernel).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -69,9 +68,10 @@ struct CandWalk {
 // chain of rounds (stack, node, member loads), so wavefronts in flight count: one a group and 3072
 // in all, fetching groups from eight counters on one line, took 870 us at a million particles, 405
 // at 262144 (M4) and 97 at 100003; two a group and 6144 in all take 570, 108 and 67 (20011: 42 and
-// 37; one a group and 4096: 567, 108, 79, 42; four and 8192: 975, 205, 88, 35).  MASKS (the parity tap): also each target's exact scatter-gather set as masks over the list, MODE 1 in FP64 with
-// the oracle's operation order, MODE 2 in FP32 in the frame of the mixed path's pair kernels with
-// their expression.  PER: periodic nearest images.
+// 37; one a group and 4096: 567, 108, 79, 42; four and 8192: 975, 205, 88, 35).  MASKS (the parity
+// tap): also each target's exact scatter-gather set as masks over the list, MODE 1 in FP64 with the
+// oracle's operation order, MODE 2 in FP32 in the frame of the mixed path's pair kernels with their
+// expression.  PER: periodic nearest images.
 template <int MODE, bool PER, int W, bool MASKS = false, bool UNION = false>
 __global__ __launch_bounds__(64*W) void k_walk_cand(CandWalk a) {
   static_assert(!MASKS || W == 1, "the masks' tests are a lone wavefront's");
@@ -366,9 +366,9 @@ __device__ void hrho_finish(const DensArgs& a, const PhysParams& p, int i, doubl
 // h-rho pass, one walk group per workgroup, its W wavefronts sharing the candidates.  A sweep
 // stages the candidates' positions batch by batch, filters them against the targets' current
 // ranges and sums the hits; every wavefront adds the W partial sums in the same order and takes
-// the same step of the iteration.  T = double: FP64 sums; T = float: FP32 pair terms in the group-centred frame summed
-// batch by batch, FP64 totals (the convergence test and the final h are always FP64).  KT:
-// DensSums' kernel.
+// the same step of the iteration.  T = double: FP64 throughout; T = float: FP32 pair terms in the
+// group-centred frame, the density's added up in FP64, the other sums batch by batch (the
+// convergence test and the final h are always FP64).  KT: DensSums' kernel.
 // Bound by vector issue where the device is full (1M particles, quintic: 0.25 VALU instructions
 // a cycle and SIMD), by the latency of the dependent loads and of each sweep's reduction below;
 // 3 wavefronts a SIMD, as 4 spill.  1M, quintic: 0.95 ms against 1.20 with masks (FP32), 1.51

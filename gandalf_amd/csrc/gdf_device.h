@@ -476,9 +476,10 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 struct TargetLanes {
   int span, copies, slot, copy, member;    // span: a power of two, at least the number of targets
   bool has;
-  __device__ __forceinline__ TargetLanes(unsigned long long on) {
+  // alone: no copies, whatever the number of targets
+  __device__ __forceinline__ explicit TargetLanes(unsigned long long on, bool alone = false) {
     const int n = __popcll(on), lane = lane_id();
-    span = n <= 2 ? 2 : 1 << (32 - __clz(n - 1));
+    span = alone ? kWave : n <= 2 ? 2 : 1 << (32 - __clz(n - 1));
     copies = kWave/span;
     slot = lane & (span - 1);
     copy = lane/span;

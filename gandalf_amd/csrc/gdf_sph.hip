@@ -308,6 +308,7 @@ struct DensArgs {
   int* status; int* flags; long long* icount;
   // stars of a gas + star run for their zeta terms (nstar = 0: none, or the terms are off)
   int nstar, star_soft;
+  int ordered;             // tabulated FP32 kernels: see k_density
   const double* sx; const double* sy; const double* sz; const double* sm; const double* sh;
   PhysParams p;
 };
@@ -369,13 +370,20 @@ __device__ void hrho_finish(const DensArgs& a, const PhysParams& p, int i, doubl
 // the same step of the iteration.  T = double: FP64 throughout; T = float: FP32 pair terms in the
 // group-centred frame, the density's added up in FP64, the other sums batch by batch (the
 // convergence test and the final h are always FP64).  KT: DensSums' kernel.
+// Tabulated FP32 kernels take the nearest lower entry, so that an h rounded otherwise moves one pair
+// in 10^4 to the next entry, 1 % of a particle's acceleration where it nearly cancels.  These
+// passes keep to one order of summation, whatever the group: every batch of a lone wavefront's list
+// by itself in FP32, batch after batch compensated, one lane a target (ORDER).  A force evaluation
+// of 72^3 particles, ms, with masks, in this order and in any order: M4 3.20, 2.41, 2.44, quintic
+// 3.79, 3.29, 2.83; of 14^3, M4, 0.57, 0.36, 0.33.
 // Bound by vector issue where the device is full (1M particles, quintic: 0.25 VALU instructions
 // a cycle and SIMD), by the latency of the dependent loads and of each sweep's reduction below;
 // 3 wavefronts a SIMD, as 4 spill.  1M, quintic: 0.95 ms against 1.20 with masks (FP32), 1.51
 // against 1.59 (FP64).
 template <typename T, int KT, int W>
 __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
-  constexpr bool F64 = sizeof(T) == 8;
+  constexpr bool F64 = sizeof(T) == 8, ORDER = !F64 && KT == 2;
+  static_assert(!ORDER || W == 1, "one wavefront's order");
   typedef typename std::conditional<F64, double4, float4>::type Rec;
   __shared__ Rec stage[W][kPairSlots];
   __shared__ double red[W > 1 ? W : 1][3][W > 1 ? kWave : 1];
@@ -387,7 +395,7 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
   Rec* const st = stage[wv];
   const unsigned long long on = __ballot(lane < gcnt && a.status[gfirst + lane] == 1);
   if (on == 0) return;
-  const TargetLanes tl(on);
+  const TargetLanes tl(on, ORDER);
   const bool has = tl.has, writes = wv == 0 && tl.copy == 0;
   const int i = has ? gfirst + tl.member : 0;
   const unsigned mine = tl.share();
@@ -423,6 +431,8 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
     ft.range(rxi*fs, ryi*fs, rzi*fs, run ? (float) rsq*hs*hs : -1.f);
     int inside = 0;
     DensSums<double, KT> sum;
+    KahanF kr, kom, kz;
+    const float invhf = (float) invh;
     HitQueue hq;
     Rec rec{};
     // the next batch's record and the indices of the one after it are in flight
@@ -456,7 +466,7 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
         return f;
       });
       hq.stage(b == 0, run ? make_uint2(hit.x & mine, hit.y & mine) : make_uint2(0u, 0u));
-      const int need = b + 1 < pb.nb ? hq.older : hq.staged;
+      const int need = b + 1 < pb.nb && !ORDER ? hq.older : hq.staged;
       if constexpr (F64) {
         hq.run(need, rec, [&](int q) { return st[q]; }, [&](const Rec& pj, bool take) {
           double dx = pj.x - me.x, dy = pj.y - me.y, dz = pj.z - me.z;
@@ -465,6 +475,21 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
           inside += take & (ssqd < rsq);
           sum.add(p.kern, ssqd, take ? pj.w : 0.0);
         });
+      } else if constexpr (ORDER) {
+        float br = 0.f, bom = 0.f, bz = 0.f;
+        hq.run(need, rec, [&](int q) { return st[q]; }, [&](const Rec& pj, bool take) {
+          const float dx = pj.x - rxi, dy = pj.y - ryi, dz = pj.z - rzi;
+          const float ssqd = invhsqdf*(dx*dx + dy*dy + dz*dz);
+          if (take && ssqd < (float) rsq) {
+            inside++;
+            const float* t = ktab<float>(p.kern) + (int) (ssqd*(float) p.kern.resinvsqd);
+            const int res = p.kern.res;
+            br += pj.w*t[KW0S2*res];
+            bom += pj.w*invhf*t[KWOMEGAS2*res];
+            bz += pj.w*t[KWZETAS2*res];
+          }
+        });
+        kr.add(br); kom.add(bom); kz.add(bz);
       } else {
         DensSums<float, KT> part;
         hq.run(need, rec, [&](int q) { return st[q]; }, [&](const Rec& pj, bool take) {
@@ -477,6 +502,7 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
       }
       wave_lds_order();
     }
+    if (ORDER) { sum.r = (double) kr.s; sum.o = (double) kom.s; sum.z = (double) kz.s; }
     evals += hq.staged;
     double r_ = tl.over_copies(sum.r), om_ = tl.over_copies(sum.o), z_ = tl.over_copies(sum.z);
     inside = tl.over_copies(inside);
@@ -492,7 +518,7 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
     if (run) {
       const double hfac3 = invh*invhsqd;
       DensSums<T, KT>::finish(p.kern, r_, om_, z_);
-      const double rho = r_*hfac3, invomega = om_*invh*hfac3, zeta = z_*invhsqd;
+      const double rho = r_*hfac3, invomega = (ORDER ? om_ : om_*invh)*hfac3, zeta = z_*invhsqd;
       const int rc = hrho_step(p, m, hmax, iteration, rho, h, h_lower, h_upper);
       if (rc == 1) {
         // converged: the sums and the bracket go to k_hrho_finish (status 2), which keeps
@@ -526,7 +552,8 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
 
 template <typename T, int KT>
 void launch_density_k(const DensArgs& d, int waves, hipStream_t s) {
-  if (waves == 4) k_density<T, KT, 4><<<d.ngroups, 4*kWave, 0, s>>>(d);
+  constexpr int many = sizeof(T) == 4 && KT == 2 ? 1 : 4;     // (waves is then 1)
+  if (waves == 4) k_density<T, KT, many><<<d.ngroups, many*kWave, 0, s>>>(d);
   else k_density<T, KT, 1><<<d.ngroups, kWave, 0, s>>>(d);
 }
 
@@ -547,10 +574,11 @@ __global__ void k_hrho_finish(DensArgs a) {
     // GradhSphTree.cpp:154: hmax = 1.05 hmax per retry, here at once as often as it takes to reach
     // the h that was past it: the iteration starts again from the same h and comes back to it, so
     // the retries on the way would end where the last one did.  (An h of a first guess takes two
-    // or three instead of up to ten: six spheres set up and served 38.4 -> 36.8 ms.)
+    // or three instead of up to ten: six spheres set up and served 38.4 -> 36.8 ms.)  One step at a
+    // time where the order of the sums counts (ordered): it follows the targets' common search.
     const double h = a.hfactor[i];
     double hs = a.hsearch[i]*1.05;
-    for (int k = 0; k < kMaxRounds && hs < h; k++) hs *= 1.05;
+    for (int k = 0; k < kMaxRounds && hs < h && !a.ordered; k++) hs *= 1.05;
     a.hsearch[i] = hs;
     a.status[i] = 1;
     // past the last radius that a round each would try
@@ -655,7 +683,8 @@ template <typename T, int VAR, bool BLK> struct HydroStage {
 // 3.45 against 5.06 (FP64) with masks.
 template <typename T, int KT, int VAR, bool BLK, int W>
 __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArgs a) {
-  constexpr bool F64 = sizeof(T) == 8;
+  constexpr bool F64 = sizeof(T) == 8, ORDER = !F64 && KT == 2;       // see k_density
+  static_assert(!ORDER || W == 1, "one wavefront's order");
   constexpr int NS = VAR == 1 ? 9 : 5;
   __shared__ HydroStage<T, VAR, BLK> stage[W];
   const int g = xcd_block(blockIdx.x, gridDim.x);
@@ -666,7 +695,7 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
   HydroStage<T, VAR, BLK>& st = stage[wv];
   const unsigned long long on = __ballot(lane < gcnt && (!BLK || a.act[gfirst + lane] != 0));
   if (on == 0) return;
-  const TargetLanes tl(on);
+  const TargetLanes tl(on, ORDER);
   const bool has = tl.has, writes = wv == 0 && tl.copy == 0;
   const int i = has ? gfirst + tl.member : 0;
   const unsigned mine = tl.share();
@@ -701,6 +730,7 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
   ft.position(rxf*fs, ryf*fs, rzf*fs);
   ft.range(rxf*fs, ryf*fs, rzf*fs, has ? (float) ((double) r2i*fs*fs) : -1.f);
   HydroSums<double> sum;
+  KahanF kx, ky, kz, ku, kv;
   const PairBatches pb((nc - wv + W - 1)/W);
   const int* idx = a.idx + (size_t) g*a.capb*kWave + wv;
   const double w1f = HydroKern<T, KT>::w1_factor(p.kern);
@@ -752,7 +782,7 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
       return f;
     });
     hq.stage(b == 0, has ? make_uint2(hit.x & mine, hit.y & mine) : make_uint2(0u, 0u));
-    const int need = b + 1 < pb.nb ? hq.older : hq.staged;
+    const int need = b + 1 < pb.nb && !ORDER ? hq.older : hq.staged;
     HydroSums<T> part;
     if (F64) sum.to(part);
     hq.run(need, rec, [&](int q) { return q; }, [&](int q, bool take) {
@@ -771,8 +801,13 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
       // unit separation; the particle itself has none
       const T tiny = F64 ? T(1.0e-280) : T(1.0e-36);
       const T d2e = VAR == 1 ? d2 + T(1.0e-20) : (d2 > tiny ? d2 : tiny);
-      const T inv = rsq_t(d2e);
-      const T drmag = d2e*inv;
+      T inv = rsq_t(d2e), drmag = d2e*inv;
+      if constexpr (ORDER) {
+        // a fixed rounding: it decides the table's entry
+        const float s2 = fmaf(dz, dz, fmaf(dx, dx, dy*dy));
+        drmag = sqrt_f(VAR == 1 ? s2 + 1.0e-20f : s2);
+        inv = drmag > 0.f ? rcp_f(drmag) : 0.f;
+      }
       dx *= inv; dy *= inv; dz *= inv;
       const T invh_j = V.w;
       HydroKern<T, KT> ki, kj;
@@ -784,12 +819,22 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
       T paux = pterm_i*wkerni + B.y*wkernj;
       if (dvdr < T(0)) {
         const T winvrho = T(0.25)*(wkerni + wkernj)*(invrho_i + B.x);
-        const T q2 = alpha*(snd_i + B.z - beta*alpha*dvdr)*dvdr*winvrho;
-        paux -= q2;
-        part.du -= T(0.5)*mj*q2*dvdr;
+        if constexpr (ORDER) {
+          const float vsignal = snd_i + B.z - beta*alpha*dvdr;
+          paux -= alpha*vsignal*dvdr*winvrho;
+          part.du -= 0.5f*mj*alpha*vsignal*dvdr*dvdr*winvrho;
+        } else {
+          const T q2 = alpha*(snd_i + B.z - beta*alpha*dvdr)*dvdr*winvrho;
+          paux -= q2;
+          part.du -= T(0.5)*mj*q2*dvdr;
+        }
       }
-      const T ma = mj*paux;
-      part.ax += ma*dx; part.ay += ma*dy; part.az += ma*dz;
+      if constexpr (ORDER) {
+        part.ax += mj*dx*paux; part.ay += mj*dy*paux; part.az += mj*dz*paux;
+      } else {
+        const T ma = mj*paux;
+        part.ax += ma*dx; part.ay += ma*dy; part.az += ma*dz;
+      }
       if (VAR == 1) {
         T mi, poti, mjj, potj;
         ki.grav(p.kern, mi, poti);
@@ -802,9 +847,17 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
         part.gp += mj*(M*inv + (invh_i*poti + invh_j*potj));
       }
     });
+    if (ORDER) {
+      kx.add((float) part.ax); ky.add((float) part.ay); kz.add((float) part.az);
+      ku.add((float) part.du); kv.add((float) part.dv);
+    }
     if (F64) part.to(sum);
     else sum.add(part);
     wave_lds_order();
+  }
+  if (ORDER) {
+    sum.ax = (double) kx.s; sum.ay = (double) ky.s; sum.az = (double) kz.s;
+    sum.du = (double) ku.s; sum.dv = (double) kv.s;
   }
   if (tl.copies > 1) {
     sum.ax = tl.over_copies(sum.ax); sum.ay = tl.over_copies(sum.ay); sum.az = tl.over_copies(sum.az);
@@ -868,8 +921,9 @@ void launch_hydro_w(const HydroArgs& h, int variant, bool blk, hipStream_t s) {
 
 template <typename T, int KT>
 void launch_hydro_k(const HydroArgs& h, int variant, bool blk, int waves, hipStream_t s) {
-  if (waves == 4) launch_hydro_w<T, KT, 4>(h, variant, blk, s);
-  else if (waves == 2) launch_hydro_w<T, KT, 2>(h, variant, blk, s);
+  constexpr bool ordered = sizeof(T) == 4 && KT == 2;         // waves is 1
+  if (waves == 4) launch_hydro_w<T, KT, ordered ? 1 : 4>(h, variant, blk, s);
+  else if (waves == 2) launch_hydro_w<T, KT, ordered ? 1 : 2>(h, variant, blk, s);
   else launch_hydro_w<T, KT, 1>(h, variant, blk, s);
 }
 
@@ -889,9 +943,15 @@ void launch_hydro(const HydroArgs& h, int variant, bool blk, int waves, hipStrea
 //   h-rho    36 24 20     46 43 61     91  89 133    164 183 257   198 319 589
 //   hydro    48 32 22     94 63 70    159 153 177    575 474 456   547 560 668
 // A serving batch keeps to one: a request's sums must not depend on what else is resident.
-int density_waves(const gdf_ctx* c) { return c->ngroups <= 256 && c->nseg == 0 ? 4 : 1; }
+// Nor may a tabulated FP32 kernel's passes depend on the number (see k_density).
+bool ordered_sums(const gdf_ctx* c) {
+  return c->cfg.precision == GDF_PREC_MIXED && c->phys.kern.tabulated;
+}
+int density_waves(const gdf_ctx* c) {
+  return c->ngroups <= 256 && c->nseg == 0 && !ordered_sums(c) ? 4 : 1;
+}
 int hydro_waves(const gdf_ctx* c) {
-  if (c->nseg > 0 || c->ngroups > 2048) return 1;
+  if (c->nseg > 0 || c->ngroups > 2048 || ordered_sums(c)) return 1;
   return c->ngroups <= 256 ? 4 : 2;
 }
 
@@ -964,10 +1024,19 @@ int launch_walk(gdf_ctx* c, WalkKind kind, int nopbc, CandSet& cs, const int* st
   if (nopbc) w.p.periodic = 0;
   const int grid = std::min(ng, kWalkSlots);
   constexpr int W = kWalkWaves;
-  const int nt = kind == WALK_MASKS ? kWave : kWave*W;
+  // (lists in the order of a lone wavefront's rounds where the order of the sums counts)
+  const bool lone = ordered_sums(c) && kind != WALK_MASKS;
+  const int nt = kind == WALK_MASKS || lone ? kWave : kWave*W;
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
   hipStream_t st = c->stream;
-  if (w.p.periodic) {
+  if (lone) {
+    if (kind == WALK_GATHER && w.p.periodic) k_walk_cand<0, true, 1><<<grid, nt, 0, st>>>(w);
+    else if (kind == WALK_GATHER) k_walk_cand<0, false, 1><<<grid, nt, 0, st>>>(w);
+    else if (kind == WALK_SG && w.p.periodic) k_walk_cand<1, true, 1><<<grid, nt, 0, st>>>(w);
+    else if (kind == WALK_SG) k_walk_cand<1, false, 1><<<grid, nt, 0, st>>>(w);
+    else if (w.p.periodic) k_walk_cand<0, true, 1, false, true><<<grid, nt, 0, st>>>(w);
+    else k_walk_cand<0, false, 1, false, true><<<grid, nt, 0, st>>>(w);
+  } else if (w.p.periodic) {
     if (kind == WALK_GATHER) k_walk_cand<0, true, W><<<grid, nt, 0, st>>>(w);
     else if (kind == WALK_UNION) k_walk_cand<0, true, W, false, true><<<grid, nt, 0, st>>>(w);
     else if (kind == WALK_SG) k_walk_cand<1, true, W><<<grid, nt, 0, st>>>(w);
@@ -1028,6 +1097,7 @@ int sph_density(gdf_ctx* c, int nopbc) {
   d.p = c->phys;
   c->sg_union = false;
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
+  d.ordered = ordered_sums(c);
   const int waves = density_waves(c);
   // with periodic images the walk makes the union lists, which the force pass reads if they
   // still bound its set: no search radius may have grown (a retry) or been outgrown

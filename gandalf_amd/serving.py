@@ -24,8 +24,8 @@ from .gpu import GpuPool, GpuSim
 # particle of capacity: 23 persistent FP64 fields and their permutation targets (368 B), 25
 # derived fields (200 B), integer state and ids (64 B), packed records and export scratch
 # (96 B), tree arrays over 2N nodes (~400 B), and the two candidate sets at their initial 16
-# batches of 64 per walk group (~512 B): ~1.65 KB; the admission budget divided by this gives
-# a pool's particle limit
+# batches of 64 indices per walk group (~190 B): ~1.3 KB; the admission budget divided by this
+# gives a pool's particle limit
 BYTES_PER_PARTICLE = 2048
 
 CLASSES = ("box", "sphere", "plummer")

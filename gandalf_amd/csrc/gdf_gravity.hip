@@ -320,47 +320,41 @@ __global__ __launch_bounds__(64*W, EWALD || FAST || (SOFT && !PLUMMER) ? 2 : 3) 
     // target position relative to the group centre (cell-relative frame of the FP32 path)
     const float rxi = (float) (me.x - gc.x), ryi = (float) (me.y - gc.y), rzi = (float) (me.z - gc.z);
 
-    // a batch of nb accepted cells from ring position c0, massless ones up to the copies' last
+    // a batch of nb accepted cells from ring position c0.  The copies' last trip goes past the batch:
+    // the slots there hold its last cell again without mass and moments.  (A fixed place can be a
+    // target's, where the term overflows in FP32 and is 0 times infinity: massless cells one code unit
+    // from the centre left NaN in the forces of lattices of unit spacing.)
     auto eval_cells = [&](int c0, int nb) {
-      if (lane >= nb) {
-        if (MIXED) {
-          s4a[lane] = make_float4(1.f, 0.f, 0.f, 0.f);
-          s4b[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-          s2[lane] = make_float2(0.f, 0.f);
-        } else {
-          sd[0][lane] = make_double2(gc.x, gc.y); sd[1][lane] = make_double2(gc.z, 0.0);
-          for (int k = 2; k < 5; k++) sd[k][lane] = make_double2(0.0, 0.0);
-        }
-      } else {
-        const int c = cbuf[(c0 + lane) & (R::cells - 1)];
-        const double* m = a.mp + kMom*(size_t) c;
-        double cx = m[0], cy = m[1], cz = m[2];
-        if (FAST) {
+      const bool fill = lane >= nb;
+      const int c = cbuf[(c0 + min(lane, nb - 1)) & (R::cells - 1)];
+      const double* m = a.mp + kMom*(size_t) c;
+      double cx = m[0], cy = m[1], cz = m[2];
+      const double mc = fill ? 0.0 : m[3];
+      if (FAST && !fill) {
 #pragma clang fp contract(off)
-          // the cell relative to the expansion point, with the node test's replica
-          double dx = cx - gc.x, dy = cy - gc.y, dz = cz - gc.z;
-          nearest_image<double>(a.p, dx, dy, dz);
-          fast_add(fc, dx - rcx, dy - rcy, dz - rcz, m[3], m + 4,
-                   a.p.multipole == GDF_MULTIPOLE_FAST_QUADRUPOLE);
-        }
-        if (a.p.periodic) {
-          // nearest periodic replica of the cell relative to the group centre
-          double dx = cx - gc.x, dy = cy - gc.y, dz = cz - gc.z;
-          nearest_image<double>(a.p, dx, dy, dz);
-          cx = gc.x + dx; cy = gc.y + dy; cz = gc.z + dz;
-        }
-        const double qs = mono ? 0.0 : 1.0;      // monopole: no quadrupole moments
-        const double q0 = qs*m[4], q2 = qs*m[6];
-        if (MIXED) {
-          s4a[lane] = make_float4((float) (cx - gc.x), (float) (cy - gc.y),
-                                  (float) (cz - gc.z), (float) m[3]);
-          s4b[lane] = make_float4((float) q0, (float) (qs*m[5]), (float) q2, (float) (qs*m[7]));
-          s2[lane] = make_float2((float) (qs*m[8]), -((float) q0 + (float) q2));
-        } else {
-          sd[0][lane] = make_double2(cx, cy); sd[1][lane] = make_double2(cz, m[3]);
-          sd[2][lane] = make_double2(q0, qs*m[5]); sd[3][lane] = make_double2(q2, qs*m[7]);
-          sd[4][lane] = make_double2(qs*m[8], -(q0 + q2));
-        }
+        // the cell relative to the expansion point, with the node test's replica
+        double dx = cx - gc.x, dy = cy - gc.y, dz = cz - gc.z;
+        nearest_image<double>(a.p, dx, dy, dz);
+        fast_add(fc, dx - rcx, dy - rcy, dz - rcz, mc, m + 4,
+                 a.p.multipole == GDF_MULTIPOLE_FAST_QUADRUPOLE);
+      }
+      if (a.p.periodic) {
+        // nearest periodic replica of the cell relative to the group centre
+        double dx = cx - gc.x, dy = cy - gc.y, dz = cz - gc.z;
+        nearest_image<double>(a.p, dx, dy, dz);
+        cx = gc.x + dx; cy = gc.y + dy; cz = gc.z + dz;
+      }
+      const double qs = mono || fill ? 0.0 : 1.0;      // monopole: no quadrupole moments
+      const double q0 = qs*m[4], q2 = qs*m[6];
+      if (MIXED) {
+        s4a[lane] = make_float4((float) (cx - gc.x), (float) (cy - gc.y),
+                                (float) (cz - gc.z), (float) mc);
+        s4b[lane] = make_float4((float) q0, (float) (qs*m[5]), (float) q2, (float) (qs*m[7]));
+        s2[lane] = make_float2((float) (qs*m[8]), -((float) q0 + (float) q2));
+      } else {
+        sd[0][lane] = make_double2(cx, cy); sd[1][lane] = make_double2(cz, mc);
+        sd[2][lane] = make_double2(q0, qs*m[5]); sd[3][lane] = make_double2(q2, qs*m[7]);
+        sd[4][lane] = make_double2(qs*m[8], -(q0 + q2));
       }
       wave_lds_order();
       // fast multipoles leave only the periodic corrections to the per-target sweep

@@ -760,6 +760,7 @@ int block_check_timesteps(gdf_ctx* c, int* activecount) {
   BlkArgs b = blk_args(c);
   k_check_timesteps<<<count_grid(c->N), BS, 0, c->stream>>>(b);
   GDF_HIP(c, hipGetLastError());
+  sph_active_changed(c);
   return read_counter(c, activecount);
 }
 

@@ -169,9 +169,9 @@ struct gdf_ctx {
   gdf::CandSet cs_g, cs_s;
   bool sg_valid = false;
   bool sg_masks = false;        // the scatter-gather candidate set holds its masks
-  // mixed path: the last density pass's candidate lists (cs_g) also hold every scatter-gather
-  // pair of the final smoothing lengths (walked with the search radii as bounds); the force
-  // pass then reads them instead of walking the tree again (sg_from_union)
+  // the last density pass's candidate lists (cs_g) also hold every scatter-gather pair of the
+  // final smoothing lengths (walked with the search radii as bounds), for the particles active in
+  // that pass; the force pass then reads them instead of walking the tree again (sg_from_union)
   bool sg_union = false;
   bool sg_from_union = false;
   // the last mixed block-step force pass's targets (its active flags, kept for decoding the
@@ -330,6 +330,9 @@ int sph_density(gdf_ctx* c, int nopbc);
 // hydro kernel tests its candidates itself)
 int sph_build_sg(gdf_ctx* c, bool masks = false);
 int sph_hydro(gdf_ctx* c, int variant);
+// block timesteps: particles may have become active since the density pass, whose lists were made
+// for those active in it
+inline void sph_active_changed(gdf_ctx* c) { c->sg_union = false; }
 
 // gravity (gdf_gravity.hip)
 int gravity_walk(gdf_ctx* c);

@@ -74,6 +74,7 @@ __global__ __launch_bounds__(BS) void k_bounds_final(int nb, const double* __res
 // ---- serving batches: per-segment bounds and segment-prefixed keys ----
 // partial-reduction blocks per segment: kMaxSeg x 16 x 6 partials fit the reduction buffer
 constexpr int kSegBlocks = 16;
+constexpr int kSegShift = 57;       // the segment id's place in a key
 constexpr int kSelBlock = 256;      // workgroup of the group selection
 
 // grid (kSegBlocks, nseg): block (b, s) folds a strided share of segment s
@@ -190,7 +191,7 @@ __device__ __forceinline__ int delta(const uint64_t* __restrict__ key, int N, in
   return 64 + __clz((int) (i ^ (int) j));
 }
 
-// segment-prefixed key: segment id in bits 57-63, 19 bits per axis below
+// segment-prefixed key: segment id from bit kSegShift (57) on, 19 bits per axis below
 __global__ void k_morton_seg(int N, const double* __restrict__ x, const double* __restrict__ y,
                              const double* __restrict__ z, const int* __restrict__ seg,
                              const double* __restrict__ bnd, uint64_t* __restrict__ keys,
@@ -206,7 +207,7 @@ __global__ void k_morton_seg(int N, const double* __restrict__ x, const double* 
     const double f = __dmul_rn(__dadd_rn(v[k], -bnd[4*sg + k]), scale);
     q[k] = f >= 524287.0 ? 524287ULL : (uint64_t) f;
   }
-  keys[i] = ((uint64_t) sg << 57) | (spread3(q[0]) << 2) | (spread3(q[1]) << 1) | spread3(q[2]);
+  keys[i] = ((uint64_t) sg << kSegShift) | (spread3(q[0]) << 2) | (spread3(q[1]) << 1) | spread3(q[2]);
   vals[i] = i;
 }
 
@@ -275,9 +276,10 @@ __global__ void k_grp_roots(int ngroups, const int* __restrict__ grp_first,
 }
 
 // Karras 2012, "Maximizing parallelism in the construction of BVHs, octrees, and k-d trees".  The
-// walk groups are the maximal nodes of at most gmax particles: a node of more marks those of its
+// walk groups are the maximal nodes of at most gmax particles, in a serving batch (segs) of one
+// request alone (a group walks from its request's subtree): a node that is more marks those of its
 // children that are groups, with their sizes, at their first particles.
-__global__ void k_lbvh(int N, int gmax, int* __restrict__ gstart, int* __restrict__ gsize, const uint64_t* __restrict__ key, int* __restrict__ left,
+__global__ void k_lbvh(int N, int gmax, bool segs, int* __restrict__ gstart, int* __restrict__ gsize, const uint64_t* __restrict__ key, int* __restrict__ left,
                        int* __restrict__ right, int* __restrict__ first, int* __restrict__ last,
                        int* __restrict__ parent, int4* __restrict__ lnk) {
   const int i = blockIdx.x*BS + threadIdx.x;
@@ -306,9 +308,12 @@ __global__ void k_lbvh(int N, int gmax, int* __restrict__ gstart, int* __restric
   lnk[i] = make_int4(f, la, L, R);
   parent[L] = i; parent[R] = i;
   if (i == 0) parent[0] = -1;
-  if (la - f + 1 > gmax) {
-    if (gamma - f + 1 <= gmax) { gstart[f] = L; gsize[f] = gamma - f + 1; }
-    if (la - gamma <= gmax) { gstart[gamma + 1] = R; gsize[gamma + 1] = la - gamma; }
+  auto group = [&](int a, int b) {
+    return b - a + 1 <= gmax && !(segs && key[a] >> kSegShift != key[b] >> kSegShift);
+  };
+  if (!group(f, la)) {
+    if (group(f, gamma)) { gstart[f] = L; gsize[f] = gamma - f + 1; }
+    if (group(gamma + 1, la)) { gstart[gamma + 1] = R; gsize[gamma + 1] = la - gamma; }
   } else if (i == 0) {
     gstart[0] = 0;
     gsize[0] = N;
@@ -1025,7 +1030,7 @@ int build_body(gdf_ctx* c, hipStream_t s, bool launch) {
   if (!launch) return GDF_OK;
   // 4. topology
   if (N > 1)
-    k_lbvh<<<nblocks(N - 1, BS), BS, 0, s>>>(N, c->cfg.group_max, c->gstart, c->visit, c->keys, c->left, c->right, c->first, c->last,
+    k_lbvh<<<nblocks(N - 1, BS), BS, 0, s>>>(N, c->cfg.group_max, c->nseg > 0, c->gstart, c->visit, c->keys, c->left, c->right, c->first, c->last,
                                              c->parent, c->lnk);
   // 5. moments, bottom-up
   NodeArgs na = node_args(c);

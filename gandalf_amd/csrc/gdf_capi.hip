@@ -429,7 +429,7 @@ void gdf_destroy(gdf_ctx* c) {
   if (c->ktabf) hipFree(c->ktabf);
   if (c->ewald_tab) hipFree(c->ewald_tab);
   if (c->ewald_tabf) hipFree(c->ewald_tabf);
-  void* segp[] = {c->d_seg_off, c->seg_root, c->seg_dt, c->seg_bnd};
+  void* segp[] = {c->d_seg_off, c->seg_root, c->seg_dt, c->seg_bnd, c->seg_bad};
   for (void* q : segp) if (q) hipFree(q);
   if (c->h_counters) hipHostFree(c->h_counters);
   if (c->h_red) hipHostFree(c->h_red);
@@ -480,7 +480,7 @@ int gdf_set_particles(gdf_ctx* c, int N, const double* r, const double* v, const
   if (h) GDF_TRY(xfer_in(c, h, n, col(F_H, nullptr)));
   k_iota<<<nblocks(N, BS), BS, 0, c->stream>>>(N, c->iorig);
   GDF_HIP(c, hipStreamSynchronize(c->stream));
-  c->tree_valid = false; c->topo_valid = false; c->sg_valid = false; c->sg_union = false; c->setup_done = false;
+  c->tree_valid = false; c->topo_valid = false; sph_drop_lists(c); c->setup_done = false;
   c->t = c->timestep = c->tlast = 0.0; c->nsteps = 0;
   return GDF_OK;
 }
@@ -522,7 +522,7 @@ int gdf_set_field(gdf_ctx* c, const char* name, const double* in) {
   GDF_HIP(c, hipGetLastError());
   GDF_HIP(c, hipStreamSynchronize(c->stream));
   if (!strcmp(name, "r") || !strcmp(name, "m") || !strcmp(name, "h")) c->tree_valid = false;
-  c->sg_valid = false; c->sg_union = false;
+  sph_drop_lists(c);
   return GDF_OK;
 }
 

@@ -174,6 +174,10 @@ struct gdf_ctx {
   // that pass; the force pass then reads them instead of walking the tree again (sg_from_union)
   bool sg_union = false;
   bool sg_from_union = false;
+  // serving batch: that holds for the requests (segments) that seg_bad does not mark; the force
+  // pass walks again for the marked ones alone (into cs_s), so that no request's lists, and with
+  // them the order of its sums, depend on what the others need
+  bool sg_part = false;
   // the last mixed block-step force pass's targets (its active flags, kept for decoding the
   // sets it evaluated); sg_tgt_all: every particle was a target (global timesteps)
   int* sg_tgt = nullptr;
@@ -224,6 +228,7 @@ struct gdf_ctx {
   double* grp_gmac = nullptr;
   double* seg_dt = nullptr;      // [kMaxSeg]: drift / kick length of the segment's step
   double* seg_bnd = nullptr;     // [4 kMaxSeg]: lower corner and scale of its Morton grid
+  int* seg_bad = nullptr;        // [kMaxSeg]: a search radius of it grew or was outgrown
 
   // timing
   bool timing = false;
@@ -333,6 +338,8 @@ int sph_hydro(gdf_ctx* c, int variant);
 // block timesteps: particles may have become active since the density pass, whose lists were made
 // for those active in it
 inline void sph_active_changed(gdf_ctx* c) { c->sg_union = false; }
+// no candidate lists any more: the particles or their tree have changed
+inline void sph_drop_lists(gdf_ctx* c) { c->sg_valid = c->sg_union = c->sg_part = false; }
 
 // gravity (gdf_gravity.hip)
 int gravity_walk(gdf_ctx* c);

@@ -309,6 +309,9 @@ struct DensArgs {
   // stars of a gas + star run for their zeta terms (nstar = 0: none, or the terms are off)
   int nstar, star_soft;
   int ordered;             // tabulated FP32 kernels: see k_density
+  // serving batches: a particle's request, and the requests whose lists do not bound their
+  // scatter-gather sets (NULL otherwise)
+  const int* seg; int* seg_bad;
   const double* sx; const double* sy; const double* sz; const double* sm; const double* sh;
   PhysParams p;
 };
@@ -581,6 +584,7 @@ __global__ void k_hrho_finish(DensArgs a) {
     for (int k = 0; k < kMaxRounds && hs < h && !a.ordered; k++) hs *= 1.05;
     a.hsearch[i] = hs;
     a.status[i] = 1;
+    if (a.seg_bad) a.seg_bad[a.seg[i]] = 1;
     // past the last radius that a round each would try
     if (hs > kMaxGrowth*a.h[i]) atomicOr(&a.flags[3], 4);
     return;
@@ -589,16 +593,29 @@ __global__ void k_hrho_finish(DensArgs a) {
   a.status[i] = 0;
   // a final h past the search radius (h from rho after the convergence test can exceed it by
   // up to h_converge): the walk's union lists no longer bound the scatter-gather set
-  if (a.h[i] > a.hsearch[i]) atomicOr(&a.flags[3], 2);
+  if (a.h[i] > a.hsearch[i]) {
+    atomicOr(&a.flags[3], 2);
+    if (a.seg_bad) a.seg_bad[a.seg[i]] = 1;
+  }
 }
 
-// act (block timesteps): only the active particles iterate; NULL = all
+// act (block timesteps): only the active particles iterate; NULL = all.  seg_bad[0, nseg) is cleared
+// (a batch's requests have two particles or more each)
 __global__ void k_init_density(int N, const double* __restrict__ h, double* __restrict__ hs,
-                               int* __restrict__ status, const int* __restrict__ act) {
+                               int* __restrict__ status, const int* __restrict__ act, int nseg,
+                               int* __restrict__ seg_bad) {
   const int i = blockIdx.x*BS + threadIdx.x;
   if (i >= N) return;
+  if (i < nseg) seg_bad[i] = 0;
   hs[i] = 1.05*h[i];      // the search radius and bisection bracket, as GradhSphTree.cpp:154
   status[i] = act ? act[i] : 1;
+}
+
+// status 1 for the particles of the requests that seg_bad marks (or, bad = 0, does not), 0 for the rest
+__global__ void k_seg_status(int N, const int* __restrict__ seg, const int* __restrict__ seg_bad,
+                             int bad, int* __restrict__ status) {
+  const int i = blockIdx.x*BS + threadIdx.x;
+  if (i < N) status[i] = seg_bad[seg[i]] == bad;
 }
 
 __global__ void k_zero_ints(int n, int* __restrict__ p) {
@@ -625,6 +642,8 @@ struct HydroArgs {
   const int* grp_node; const int* grp_first; const int* grp_count;
   const double4* geo_c; const double4* geo_h;
   const int* idx; const int* ncand;
+  // serving batches: the lists of the groups that walked again (ncand2 > 0), in place of idx's
+  int capb2; const int* idx2; const int* ncand2;
   const double4* posm; const double4* A; const double4* B;
   const double* h;
   const double* invomega; const double* pressure; const double* zeta;
@@ -689,7 +708,8 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
   __shared__ HydroStage<T, VAR, BLK> stage[W];
   const int g = xcd_block(blockIdx.x, gridDim.x);
   const int lane = threadIdx.x & (kWave - 1), wv = W == 1 ? 0 : (int) threadIdx.x/kWave;
-  const int nc = a.ncand[g];
+  const int n2 = a.ncand2 ? a.ncand2[g] : 0;
+  const int nc = n2 > 0 ? n2 : a.ncand[g];
   if (nc <= 0) return;                        // no target in this group
   const int gfirst = a.grp_first[g], gcnt = a.grp_count[g];
   HydroStage<T, VAR, BLK>& st = stage[wv];
@@ -732,7 +752,7 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
   HydroSums<double> sum;
   KahanF kx, ky, kz, ku, kv;
   const PairBatches pb((nc - wv + W - 1)/W);
-  const int* idx = a.idx + (size_t) g*a.capb*kWave + wv;
+  const int* idx = (n2 > 0 ? a.idx2 + (size_t) g*a.capb2*kWave : a.idx + (size_t) g*a.capb*kWave) + wv;
   const double w1f = HydroKern<T, KT>::w1_factor(p.kern);
   HitQueue hq;
   int rec = 0;
@@ -1081,7 +1101,8 @@ int sph_density(gdf_ctx* c, int nopbc) {
   if (!c->tree_valid) return fail(c, GDF_ERR_INVALID, "density pass before tree build");
   GDF_TRY(ensure_cand(c, c->cs_g, c->ngroups, false));
   const int* act = c->nlevels > 1 ? c->pi[I_ACT] : nullptr;
-  k_init_density<<<nblocks(N, BS), BS, 0, s>>>(N, c->pf[F_H], c->df[D_HSEARCH], c->status, act);
+  k_init_density<<<nblocks(N, BS), BS, 0, s>>>(N, c->pf[F_H], c->df[D_HSEARCH], c->status, act,
+                                               c->nseg, c->seg_bad);
   DensArgs d;
   d.N = N; d.ngroups = c->ngroups; d.nopbc = nopbc;
   d.grp_node = c->grp_node; d.grp_first = c->grp_first; d.grp_count = c->grp_count;
@@ -1095,19 +1116,22 @@ int sph_density(gdf_ctx* c, int nopbc) {
   d.star_soft = c->cfg.nbody_softening;
   d.sx = c->sv[S_X]; d.sy = c->sv[S_Y]; d.sz = c->sv[S_Z]; d.sm = c->sv[S_M]; d.sh = c->sv[S_H];
   d.p = c->phys;
-  c->sg_union = false;
+  d.seg = c->pi[I_SEG]; d.seg_bad = c->nseg > 0 ? c->seg_bad : nullptr;
+  c->sg_union = c->sg_part = false;
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
   d.ordered = ordered_sums(c);
   const int waves = density_waves(c);
   // with periodic images the walk makes the union lists, which the force pass reads if they
-  // still bound its set: no search radius may have grown (a retry) or been outgrown
+  // still bound its set: no search radius may have grown (a retry) or been outgrown, in a batch of
+  // several requests none of the request's own
   const bool uni = !nopbc;
+  const bool several = c->nseg > 1;
   const WalkKind kind = uni ? WALK_UNION : WALK_GATHER;
   bool grown = false, retried = false, outgrown = false;
   for (int round = 0; round < kMaxRounds; round++) {
-    // also clears the round's flags
-    GDF_TRY(group_list(c, c->status, c->glist, c->cs_g.ncand, nullptr, nullptr, c->counters,
-                       4));
+    // also clears the round's flags (and, where they are not read any more, the settled groups' lists)
+    GDF_TRY(group_list(c, c->status, c->glist, round > 0 && several ? nullptr : c->cs_g.ncand,
+                       nullptr, nullptr, c->counters, 4));
     GDF_TRY(launch_walk(c, kind, nopbc, c->cs_g, c->status, c->glist));
     d.capb = c->cs_g.capb; d.idx = c->cs_g.idx; d.ncand = c->cs_g.ncand;
     if (mixed) launch_density<float>(d, waves, s);
@@ -1130,17 +1154,23 @@ int sph_density(gdf_ctx* c, int nopbc) {
     if (f[0] != 0) continue;
     c->sg_valid = false;
     c->sg_union = uni && !retried && !outgrown;
-    if (c->sg_union && grown) {
-      // growing dropped the lists of the groups settled before: every group's again, as the
-      // first round would have made them with room enough (the radii and the nodes' bounds are
-      // still those of its start)
-      if (act) GDF_TRY(group_list(c, act, c->glist, c->cs_g.ncand, nullptr, nullptr,
-                                  c->counters, 4));
+    c->sg_part = uni && !c->sg_union && several;
+    if ((c->sg_union || c->sg_part) && grown) {
+      // growing dropped the lists of the groups settled before: every group's again (of the
+      // requests whose lists are read), as the first round would have made them with room enough
+      // (the radii and the nodes' bounds are still those of its start)
+      const int* on = act;
+      if (c->sg_part) {
+        k_seg_status<<<nblocks(N, BS), BS, 0, s>>>(N, c->pi[I_SEG], c->seg_bad, 0, c->status);
+        on = c->status;
+      }
+      if (on) GDF_TRY(group_list(c, on, c->glist, c->cs_g.ncand, nullptr, nullptr,
+                                 c->counters, 4));
       else k_zero_ints<<<1, BS, 0, s>>>(4, c->counters);
-      GDF_TRY(launch_walk(c, kind, nopbc, c->cs_g, act, act ? c->glist : nullptr));
+      GDF_TRY(launch_walk(c, kind, nopbc, c->cs_g, on, on ? c->glist : nullptr));
       GDF_TRY(read_flags(c));
       if (c->h_counters[2]) return fail(c, GDF_ERR_CAPACITY, "tree walk stack overflow in gather pass");
-      if (c->h_counters[1] > 0) c->sg_union = false;
+      if (c->h_counters[1] > 0) c->sg_union = c->sg_part = false;
     }
     return tree_refit_h(c);
   }
@@ -1157,8 +1187,12 @@ int sph_build_sg(gdf_ctx* c, bool masks) {
   }
   const int ng = c->ngroups;
   GDF_TRY(ensure_cand(c, c->cs_s, ng, masks));
+  const int* act = c->nlevels > 1 ? c->pi[I_ACT] : nullptr;
+  if (!masks && c->sg_part) {       // the marked requests' groups alone
+    k_seg_status<<<nblocks(c->N, BS), BS, 0, c->stream>>>(c->N, c->pi[I_SEG], c->seg_bad, 1, c->status);
+    act = c->status;
+  }
   for (int round = 0; round < 8; round++) {
-    const int* act = c->nlevels > 1 ? c->pi[I_ACT] : nullptr;
     int* sl = c->glist + (c->Ncap + 1);
     if (act) GDF_TRY(group_list(c, act, sl, c->cs_s.ncand, nullptr, nullptr, c->counters, 4));
     else k_zero_ints<<<1, BS, 0, c->stream>>>(4, c->counters);
@@ -1169,6 +1203,7 @@ int sph_build_sg(gdf_ctx* c, bool masks) {
       GDF_TRY(grow_cand(c, c->cs_s, ng, c->h_counters[1], masks));
       continue;
     }
+    c->sg_from_union = !masks && c->sg_part;
     c->sg_valid = true;
     c->sg_masks = masks;
     return GDF_OK;
@@ -1190,6 +1225,8 @@ int sph_hydro(gdf_ctx* c, int variant) {
   h.grp_node = c->grp_node; h.grp_first = c->grp_first; h.grp_count = c->grp_count;
   h.geo_c = c->geo_c; h.geo_h = c->geo_h;
   h.idx = cs.idx; h.ncand = cs.ncand;
+  const bool part = c->sg_from_union && c->sg_part;
+  h.capb2 = c->cs_s.capb; h.idx2 = c->cs_s.idx; h.ncand2 = part ? c->cs_s.ncand : nullptr;
   h.posm = c->posm; h.A = c->hrecA; h.B = c->hrecB; h.h = c->pf[F_H];
   h.invomega = c->df[D_INVOMEGA]; h.pressure = c->df[D_PRESSURE]; h.zeta = c->df[D_ZETA];
   h.ax = c->df[D_AX]; h.ay = c->df[D_AY]; h.az = c->df[D_AZ];

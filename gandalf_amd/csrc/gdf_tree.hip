@@ -807,6 +807,7 @@ int seg_alloc(gdf_ctx* c) {
   GDF_HIP(c, hipMalloc(&c->seg_root, sizeof(int)*kMaxSeg));
   GDF_HIP(c, hipMalloc(&c->seg_dt, sizeof(double)*kMaxSeg));
   GDF_HIP(c, hipMalloc(&c->seg_bnd, sizeof(double)*4*kMaxSeg));
+  GDF_HIP(c, hipMalloc(&c->seg_bad, sizeof(int)*kMaxSeg));
   return GDF_OK;
 }
 
@@ -1206,7 +1207,7 @@ int tree_build(gdf_ctx* c) {
   GDF_TRY(group_mac(c, c->df_alt[0] ? nullptr : c->vals));
   c->tree_valid = true;
   c->topo_valid = true;
-  c->sg_valid = false; c->sg_union = false;
+  sph_drop_lists(c);
   GDF_HIP(c, hipGetLastError());
   return integ_pack_posm(c);
 }
@@ -1230,7 +1231,7 @@ int tree_restock(gdf_ctx* c) {
   GDF_TRY(integ_pack_posm(c));
   GDF_HIP(c, hipStreamSynchronize(s));
   c->tree_valid = true;
-  c->sg_valid = false; c->sg_union = false;
+  sph_drop_lists(c);
   return GDF_OK;
 }
 

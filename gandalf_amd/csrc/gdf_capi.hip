@@ -513,7 +513,7 @@ int gdf_set_field(gdf_ctx* c, const char* name, const double* in) {
     k_gather_in_int<<<nblocks(c->N, BS), BS, 0, c->stream>>>(c->N, c->pi[fi], c->iorig, c->tmpd);
     GDF_HIP(c, hipGetLastError());
     GDF_HIP(c, hipStreamSynchronize(c->stream));
-    if (fi == I_ACT && c->nlevels > 1) sph_active_changed(c);
+    if (fi == I_ACT && c->nlevels > 1) sph_active_set(c);
     return GDF_OK;
   }
   if (!field_ptrs(c, name, p, &w)) return fail(c, GDF_ERR_INVALID, std::string("unknown field ") + name);

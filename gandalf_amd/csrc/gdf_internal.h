@@ -178,11 +178,13 @@ struct gdf_ctx {
   // pass walks again for the marked ones alone (into cs_s), so that no request's lists, and with
   // them the order of its sums, depend on what the others need
   bool sg_part = false;
-  // the last mixed block-step force pass's targets (its active flags, kept for decoding the
-  // sets it evaluated); sg_tgt_all: every particle was a target (global timesteps)
+  // the last block-step force pass's targets (its active flags, kept for the parity tap's sets of
+  // that pass); sg_tgt_all: every particle was a target (global timesteps); sg_tgt_now: the flags
+  // have not been set since (the end of a step clears them)
   int* sg_tgt = nullptr;
   int sg_tgt_cap = 0;
   bool sg_tgt_all = true;
+  bool sg_tgt_now = false;
 
   // walk scratch
   int* stacks = nullptr;
@@ -338,6 +340,12 @@ int sph_hydro(gdf_ctx* c, int variant);
 // block timesteps: particles may have become active since the density pass, whose lists were made
 // for those active in it
 inline void sph_active_changed(gdf_ctx* c) { c->sg_union = false; }
+// ... by the caller: the parity tap's sets are those of the new flags
+inline void sph_active_set(gdf_ctx* c) {
+  sph_active_changed(c);
+  c->sg_tgt_now = false;
+  if (c->sg_masks) c->sg_valid = false;
+}
 // no candidate lists any more: the particles or their tree have changed
 inline void sph_drop_lists(gdf_ctx* c) { c->sg_valid = c->sg_union = c->sg_part = false; }
 

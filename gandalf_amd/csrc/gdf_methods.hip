@@ -97,7 +97,7 @@ int gdf_set_active_particles(gdf_ctx* c, int n) {
     k_set_active<<<nblocks(c->N, BS), BS, 0, c->stream>>>(c->N, n, c->pi[I_NLAST],
                                                           c->pi[I_NSTEP], c->pi[I_END],
                                                           c->pi[I_ACT]);
-    sph_active_changed(c);
+    sph_active_set(c);
   }
   GDF_HIP(c, hipGetLastError());
   GDF_HIP(c, hipStreamSynchronize(c->stream));

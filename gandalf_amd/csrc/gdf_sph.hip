@@ -623,15 +623,18 @@ __global__ void k_zero_ints(int n, int* __restrict__ p) {
   if (i < n) p[i] = 0;
 }
 
-// hydro neighbour records: A = (v, 1/h), B = (1/rho, P invomega/rho^2, sound, hfactor)
+// hydro neighbour records: A = (v, 1/h), B = (1/rho, P invomega/rho^2, sound, hfactor); tgt (block
+// steps): the pass's targets, kept for the parity tap
 __global__ void k_pack_hydro(int N, const double* __restrict__ vx, const double* __restrict__ vy,
                              const double* __restrict__ vz, const double* __restrict__ h,
                              const double* __restrict__ rho, const double* __restrict__ pres,
                              const double* __restrict__ iom, const double* __restrict__ snd,
                              const double* __restrict__ hf, double4* __restrict__ A,
-                             double4* __restrict__ B) {
+                             double4* __restrict__ B, const int* __restrict__ act,
+                             int* __restrict__ tgt) {
   const int i = blockIdx.x*BS + threadIdx.x;
   if (i >= N) return;
+  if (tgt) tgt[i] = act[i];
   A[i] = make_double4(vx[i], vy[i], vz[i], 1/h[i]);
   const double r = rho[i];
   B[i] = make_double4(1/r, (pres[i]*iom[i])/(r*r), snd[i], hf[i]);
@@ -1093,6 +1096,7 @@ void sph_free_lists(gdf_ctx* c) {
   c->sg_tgt = nullptr;
   c->sg_tgt_cap = 0;
   c->sg_tgt_all = true;
+  c->sg_tgt_now = false;
 }
 
 int sph_density(gdf_ctx* c, int nopbc) {
@@ -1188,6 +1192,8 @@ int sph_build_sg(gdf_ctx* c, bool masks) {
   const int ng = c->ngroups;
   GDF_TRY(ensure_cand(c, c->cs_s, ng, masks));
   const int* act = c->nlevels > 1 ? c->pi[I_ACT] : nullptr;
+  // the FP64 path's tap after a force pass: that pass's targets, whose flags the step's end clears
+  if (masks && act && c->cfg.precision != GDF_PREC_MIXED && c->sg_valid && c->sg_tgt_now) act = c->sg_tgt;
   if (!masks && c->sg_part) {       // the marked requests' groups alone
     k_seg_status<<<nblocks(c->N, BS), BS, 0, c->stream>>>(c->N, c->pi[I_SEG], c->seg_bad, 1, c->status);
     act = c->status;
@@ -1215,10 +1221,22 @@ int sph_hydro(gdf_ctx* c, int variant) {
   const int N = c->N;
   hipStream_t s = c->stream;
   if (!c->sg_valid || c->sg_masks) GDF_TRY(sph_build_sg(c));
+  const bool blk = c->nlevels > 1;
+  // the pass's targets, for the sets it evaluates (its lists cover those alone)
+  c->sg_tgt_all = !blk;
+  c->sg_tgt_now = blk;
+  if (blk && c->sg_tgt_cap < N) {
+    if (c->sg_tgt) (void) hipFree(c->sg_tgt);
+    c->sg_tgt = nullptr;
+    c->sg_tgt_cap = 0;
+    GDF_HIP(c, hipMalloc(&c->sg_tgt, sizeof(int)*(size_t) c->Ncap));
+    c->sg_tgt_cap = c->Ncap;
+  }
   k_pack_hydro<<<nblocks(N, BS), BS, 0, s>>>(N, c->pf[F_VX], c->pf[F_VY], c->pf[F_VZ],
                                              c->pf[F_H], c->df[D_RHO], c->df[D_PRESSURE],
                                              c->df[D_INVOMEGA], c->df[D_SOUND],
-                                             c->df[D_HFACTOR], c->hrecA, c->hrecB);
+                                             c->df[D_HFACTOR], c->hrecA, c->hrecB,
+                                             c->pi[I_ACT], blk ? c->sg_tgt : nullptr);
   HydroArgs h;
   const CandSet& cs = c->sg_from_union ? c->cs_g : c->cs_s;
   h.N = N; h.ngroups = c->ngroups; h.capb = cs.capb;
@@ -1235,22 +1253,6 @@ int sph_hydro(gdf_ctx* c, int variant) {
   h.icount = c->icount;
   h.act = c->pi[I_ACT]; h.level = c->pi[I_LEVEL]; h.levelneib = c->pi[I_LEVELNEIB];
   const bool mixed = c->cfg.precision == GDF_PREC_MIXED;
-  const bool blk = c->nlevels > 1;
-  if (mixed) {
-    // the pass's targets, for decoding the sets it evaluates (its lists cover those alone)
-    c->sg_tgt_all = !blk;
-    if (blk) {
-      if (c->sg_tgt_cap < N) {
-        if (c->sg_tgt) (void) hipFree(c->sg_tgt);
-        c->sg_tgt = nullptr;
-        c->sg_tgt_cap = 0;
-        GDF_HIP(c, hipMalloc(&c->sg_tgt, sizeof(int)*(size_t) c->Ncap));
-        c->sg_tgt_cap = c->Ncap;
-      }
-      GDF_HIP(c, hipMemcpyAsync(c->sg_tgt, c->pi[I_ACT], sizeof(int)*(size_t) N,
-                                hipMemcpyDeviceToDevice, s));
-    }
-  }
   const int kt = ktime_begin(c, s, 6);
   if (mixed) launch_hydro<float>(h, variant, blk, hydro_waves(c), s);
   else launch_hydro<double>(h, variant, blk, hydro_waves(c), s);
@@ -1261,7 +1263,7 @@ int sph_hydro(gdf_ctx* c, int variant) {
 
 int sph_copy_sg(gdf_ctx* c, std::vector<int>& idx, std::vector<unsigned long long>& mask,
                 std::vector<int>& ncand, int& capb) {
-  // the mixed force pass leaves no masks: the set is walked again with them (same tests)
+  // the force passes leave no masks: the set is walked again with them (same tests)
   if (!c->sg_valid || !c->sg_masks) GDF_TRY(sph_build_sg(c, true));
   GDF_HIP(c, hipStreamSynchronize(c->stream));
   const CandSet& cs = c->cs_s;

@@ -28,11 +28,13 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr float kFilterSlack = 8.0e-6f;
 constexpr float kFilterFar = 1.0e30f;     // |c|^2 of an empty slot (and, negated, of a sure hit)
 
-// power of two that brings the length `ext` (> 0) below one
-__device__ __forceinline__ float filter_scale(double ext) {
+// power of two that brings the length `ext` (> 0) below one; T: the precision of the frame, so that
+// FP64 lengths outside the range of single precision are scaled before they are rounded to it
+template <typename T> __device__ __forceinline__ T filter_scale(double ext) {
+  constexpr int most = sizeof(T) == 8 ? 1000 : 120;
   int e;
   (void) frexp(ext, &e);
-  return (float) ldexp(1.0, max(-120, min(120, -e)));
+  return (T) ldexp(1.0, max(-most, min(most, -e)));
 }
 
 // One candidate's features: scaled position and the square of its own scaled range (widened;

@@ -416,13 +416,15 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
   const double rsq = p.kern.rangesqd;
   // the filter's frame: the group's half-diagonal plus the targets' largest search range below one
   const double rG = p.kern.range*wave_max_d(has ? hmax : 0.0);
-  const float fs = filter_scale(sqrt(gh.x*gh.x + gh.y*gh.y + gh.z*gh.z) + rG);
+  const T fs = filter_scale<T>(sqrt(gh.x*gh.x + gh.y*gh.y + gh.z*gh.z) + rG);
+  const float fx = (float) ((T) (me.x - gc.x)*fs), fy = (float) ((T) (me.y - gc.y)*fs),
+              fz = (float) ((T) (me.z - gc.z)*fs);
   // FP64 separations take the nearest image target by target: where a candidate's image about
   // the group's centre need not be its image about every target, all candidates are taken
   const bool all = F64 && p.periodic && (gh.x + rG >= p.boxhalf[0] || gh.y + rG >= p.boxhalf[1] ||
                                          gh.z + rG >= p.boxhalf[2]);
   FiltTargets ft;
-  ft.position(rxi*fs, ryi*fs, rzi*fs);
+  ft.position(fx, fy, fz);
   const PairBatches pb((nc - wv + W - 1)/W);
   const int* idx = a.idx + (size_t) g*a.capb*kWave + wv;
   while (__ballot(state == 2)) {
@@ -430,8 +432,8 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
     if (run) iteration++;
     const double invh = 1.0/h;
     const double invhsqd = invh*invh;
-    const float invhsqdf = (float) invhsqd, hs = (float) h*fs;
-    ft.range(rxi*fs, ryi*fs, rzi*fs, run ? (float) rsq*hs*hs : -1.f);
+    const float invhsqdf = (float) invhsqd, hs = (float) ((T) h*fs);
+    ft.range(fx, fy, fz, run ? (float) rsq*hs*hs : -1.f);
     int inside = 0;
     DensSums<double, KT> sum;
     KahanF kr, kom, kz;
@@ -460,11 +462,11 @@ __global__ __launch_bounds__(64*W, 3) void k_density(DensArgs a) {
         if (F64) {
           double dx = r.x - gc.x, dy = r.y - gc.y, dz = r.z - gc.z;
           nearest_image<double>(p, dx, dy, dz);
-          f.x = (float) dx; f.y = (float) dy; f.z = (float) dz;
+          f.x = (float) (dx*fs); f.y = (float) (dy*fs); f.z = (float) (dz*fs);
         } else {
-          f.x = (float) r.x; f.y = (float) r.y; f.z = (float) r.z;
+          f.x = (float) (r.x*fs); f.y = (float) (r.y*fs); f.z = (float) (r.z*fs);
         }
-        f.x *= fs; f.y *= fs; f.z *= fs; f.thr = 0.f;
+        f.thr = 0.f;
         f.state = !pb.filled(b, l) ? 1 : all ? -1 : 0;
         return f;
       });
@@ -738,8 +740,8 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
     h_i = a.h[i];
     r2i = (T) range2_rn(krsqd, h_i);
   }
-  const float rxf = (float) (me.x - gc.x), ryf = (float) (me.y - gc.y), rzf = (float) (me.z - gc.z);
-  const T rxi = F64 ? (T) me.x : (T) rxf, ryi = F64 ? (T) me.y : (T) ryf, rzi = F64 ? (T) me.z : (T) rzf;
+  const T rxi = (T) (F64 ? me.x : me.x - gc.x), ryi = (T) (F64 ? me.y : me.y - gc.y),
+          rzi = (T) (F64 ? me.z : me.z - gc.z);
   const T vxi = F64 ? (T) mA.x : (T) (mA.x - vref.x), vyi = F64 ? (T) mA.y : (T) (mA.y - vref.y),
           vzi = F64 ? (T) mA.z : (T) (mA.z - vref.z);
   const T invh_i = (T) mA.w, invrho_i = (T) mB.x, pterm_i = (T) mB.y, snd_i = (T) mB.z;
@@ -748,10 +750,12 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
   // the filter's frame: the group's half-diagonal plus the targets' largest range below one
   const double rG = p.kern.range*wave_max_d(h_i);
   const double diag = sqrt(gh.x*gh.x + gh.y*gh.y + gh.z*gh.z);
-  const float fs = filter_scale(diag + rG);
+  const T fs = filter_scale<T>(diag + rG);
+  const float fx = (float) ((T) (me.x - gc.x)*fs), fy = (float) ((T) (me.y - gc.y)*fs),
+              fz = (float) ((T) (me.z - gc.z)*fs);
   FiltTargets ft;
-  ft.position(rxf*fs, ryf*fs, rzf*fs);
-  ft.range(rxf*fs, ryf*fs, rzf*fs, has ? (float) ((double) r2i*fs*fs) : -1.f);
+  ft.position(fx, fy, fz);
+  ft.range(fx, fy, fz, has ? (float) ((double) r2i*fs*fs) : -1.f);
   HydroSums<double> sum;
   KahanF kx, ky, kz, ku, kv;
   const PairBatches pb((nc - wv + W - 1)/W);
@@ -790,7 +794,7 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
       if (F64) {
         double dx = r.x - gc.x, dy = r.y - gc.y, dz = r.z - gc.z;
         nearest_image<double>(p, dx, dy, dz);
-        f.x = (float) dx; f.y = (float) dy; f.z = (float) dz;
+        f.x = (float) (dx*fs); f.y = (float) (dy*fs); f.z = (float) (dz*fs);
         if (p.periodic) {
           // taken unless its image about the centre is its image about every target in range
           const double R = fmax(rG, sqrt((double) r2));
@@ -798,9 +802,8 @@ __global__ __launch_bounds__(64*W, sizeof(T) == 8 ? 2 : 3) void k_hydro(HydroArg
             f.state = -1;
         }
       } else {
-        f.x = (float) r.x; f.y = (float) r.y; f.z = (float) r.z;
+        f.x = (float) (r.x*fs); f.y = (float) (r.y*fs); f.z = (float) (r.z*fs);
       }
-      f.x *= fs; f.y *= fs; f.z *= fs;
       f.thr = filter_thr((float) ((double) r2*fs*fs));
       return f;
     });

@@ -154,7 +154,7 @@ struct gdf_ctx {
   int* left = nullptr; int* right = nullptr; int* first = nullptr; int* last = nullptr;
   int* parent = nullptr; int* visit = nullptr;   // visit: scratch of the group selections
   int4* lnk = nullptr;          // internal node: (first, last, left, right) in one 16-byte record
-  int* front = nullptr;                                // refit frontier [N] + count
+  int* front = nullptr;                                // refit frontiers, 2 x [N], and their counts
   double4* geo_c = nullptr; double4* geo_h = nullptr;
   double* mp = nullptr;                                // kMom per node
   int* gstart = nullptr;                               // per-slot group-start marker

@@ -318,8 +318,9 @@ struct DensArgs {
 
 // One step of the grad-h iteration after the sums at h (GradhSph.cpp:219-256): the fixed point
 // h <- h_fac (m/rho)^(1/3), bisection on [h_lower, h_upper] after hrho_itmax (30) iterations,
-// failure after five times as many.  Returns 2 to iterate again, 1 done (converged, or the bracket closed), 0 retry with a
-// larger search radius, -1 no convergence.
+// failure after five times as many; cbrt differs from the reference's pow(., 1/3), which the final h
+// takes, in the last bit.  Returns 2 to iterate again, 1 done (converged, or the bracket closed), 0
+// retry with a larger search radius, -1 no convergence.
 __device__ __forceinline__ int hrho_step(const PhysParams& p, double m, double hmax, int iteration,
                                          double rho, double& h, double& h_lower,
                                          double& h_upper) {

@@ -847,7 +847,7 @@ int tree_alloc(gdf_ctx* c) {
   GDF_HIP(c, hipMalloc(&c->parent, sizeof(int)*nn));
   GDF_HIP(c, hipMalloc(&c->lnk, sizeof(int4)*N));
   GDF_HIP(c, hipMalloc(&c->visit, sizeof(int)*(N + 16)));   // 16-byte-padded byte flags
-  // refit frontiers: phase 1 (one RB slot per chunk), chunk counts, phase 2 (N + count)
+  // refit frontiers: two buffers of N nodes that the phases use in turn, and a count a run for each
   GDF_HIP(c, hipMalloc(&c->front, sizeof(int)*(2*N + 2*(N/1024 + 16))));
   GDF_HIP(c, hipMalloc(&c->geo_c, sizeof(double4)*nn));
   GDF_HIP(c, hipMalloc(&c->geo_h, sizeof(double4)*nn));

@@ -552,8 +552,7 @@ int gdf_update_all_sph_forces(gdf_ctx* c) {
   GDF_TRY(integ_zero_accelerations(c));
   if (c->phys.hydro_forces) {
     GDF_TRY(gravity_launch(c));        // beside the hydro pass, on the second stream
-    GDF_TRY(sph_build_sg(c));
-    GDF_TRY(sph_hydro(c, 1));
+    GDF_TRY(gravity_beside_hydro(c));
     GDF_TRY(gravity_join(c));
     return stars_on_gas(c);
   }

@@ -34,6 +34,8 @@
 // 2.65, FP32), from counters a line apart (on one line: 560 us at 262144 particles instead of 455).
 #include <hip/hip_runtime.h>
 
+#include <cstdlib>
+
 #include "gdf_internal.h"
 #include "gdf_device.h"
 #include "gdf_filter.h"
@@ -956,6 +958,21 @@ int gravity_launch(gdf_ctx* c) {
                             hipMemcpyDeviceToHost, s2));
   GDF_HIP(c, hipEventRecord(c->ev_grav, s2));
   return GDF_OK;
+}
+
+// Fault injection for the failure-path tests: with GDF_FAULT_HYDRO=1 in the environment the hydro
+// pass beside the gravity walk reports a failure.
+static bool hydro_fault_injected() {
+  const char* e = std::getenv("GDF_FAULT_HYDRO");
+  return e && e[0] == '1';
+}
+
+int gravity_beside_hydro(gdf_ctx* c) {
+  int rc = hydro_fault_injected() ? fail(c, GDF_ERR_NOMEM, "injected failure of the hydro pass")
+                                  : sph_build_sg(c);
+  if (rc == GDF_OK) rc = sph_hydro(c, 1);
+  if (rc != GDF_OK) (void) hipStreamSynchronize(c->stream2);
+  return rc;
 }
 
 int gravity_join(gdf_ctx* c) {

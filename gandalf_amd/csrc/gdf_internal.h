@@ -355,6 +355,9 @@ int gravity_walk(gdf_ctx* c);
 // atree += walk, gpot = (self + gpot) + walk, a += atree
 int gravity_launch(gdf_ctx* c);
 int gravity_join(gdf_ctx* c);
+// the scatter-gather lists and the hydro pass between the two; a failure waits for the walk, whose
+// inputs the caller may write next
+int gravity_beside_hydro(gdf_ctx* c);
 
 // integration (gdf_integrate.hip)
 int zero_icount(gdf_ctx* c);    // clears the eight interaction counters of a step

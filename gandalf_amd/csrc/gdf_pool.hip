@@ -187,8 +187,7 @@ int batch_forces(gdf_ctx* c) {
   if (c->phys.self_gravity) {
     if (c->phys.hydro_forces) {
       GDF_TRY(gravity_launch(c));          // beside the hydro pass, on the second stream
-      GDF_TRY(sph_build_sg(c));
-      GDF_TRY(sph_hydro(c, 1));
+      GDF_TRY(gravity_beside_hydro(c));
       return gravity_join(c);
     }
     GDF_TRY(gravity_walk(c));

@@ -61,8 +61,7 @@ int GradhSphTreeGpu<ndim>::UpdateAllSphForces() {
     // the gravity walk needs only h and zeta of the density pass: it runs on the second stream
     // while the scatter-gather walk and the hydro pass run on the first
     GDF_TRY(gdf::gravity_launch(ctx));
-    GDF_TRY(gdf::sph_build_sg(ctx));
-    GDF_TRY(gdf::sph_hydro(ctx, 1));
+    GDF_TRY(gdf::gravity_beside_hydro(ctx));
     record(ctx, 3);
     GDF_TRY(gdf::gravity_join(ctx));
     return gdf::stars_on_gas(ctx);      // GradhSphTree.cpp:600-607
